@@ -249,6 +249,16 @@ int sytrd_lower_f32(hipStream_t s, float* a, long lda, int n, float* d, float* e
 int ormtr_lower_f32(hipStream_t s, const float* a, long lda, int n, const float* tau, float* z,
                     long ldz, int ncols, void* work, size_t workBytes);
 size_t sytrd_work_bytes(int n, int elemSize);
+// The columns from c0 on of sytrd_lower_batched when the trailing matrices fit on the chip
+// (sytrd_resident.hip). sytrd_resident_from: the first such column, a multiple of the panel width
+// (n: none). sytrd_resident: *done = false and nothing launched under stream capture or when the
+// device refuses the launch. ring: kResidentWords (n - c0) words per problem, sRing apart; flag:
+// one int for all problems.
+constexpr int kResidentWords = 12;
+int sytrd_resident_from(int n, int K, int* c0);
+template <typename T>
+int sytrd_resident(hipStream_t s, T* a, long lda, long sA, int n, int c0, T* d, T* e, T* tau,
+                   long sV, unsigned long long* ring, long sRing, int* flag, int K, bool* done);
 int set_symv_tiles(int tiles);   // row tiles per SYMV workgroup: 2, 4, 8, 16 or 0 (by size)
 // capture the tridiagonalisation's launch sequence in a HIP graph and replay it for repeated
 // calls on the same buffers (off by default); release_sytrd_graphs frees the kept graphs

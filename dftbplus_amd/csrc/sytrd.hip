@@ -549,12 +549,14 @@ __global__ void panel_restore_kernel(T* a, long lda, int n, int j0, int pw, T* d
 // K problems of size n at once: problem k's matrix at a + k sA, d, e, tau at + k sV and its
 // workspace block at work + k wsStride bytes (wsStride >= sytrd_layout(n)). The column kernels
 // run all problems in one launch each; the panel products and trailing updates run per problem.
+// Panels from .. to - 1 (multiples of kNB, or to = n); the panels before `from` have been run.
 template <typename T>
 static int sytrd_launches(hipStream_t s, T* a, long lda, long sA, int n, T* d, T* e, T* tau,
-                          long sV, void* work, size_t wsStride, int K) {
+                          long sV, void* work, size_t wsStride, int K, int from, int to) {
   std::vector<SytrdWs<T>> wk(K);
   for (int k = 0; k < K; ++k) {
     sytrd_layout<T>(n, &wk[k], static_cast<char*>(work) + (size_t)k * wsStride);
+    if (from > 0) continue;
     DH_TRY(fill<double>(s, wk[k].nrm2, n, 0.0));
     DH_TRY(fill<double>(s, wk[k].dot, n, 0.0));
     DH_TRY(fill<double>(s, wk[k].t12, (size_t)kT12Size, 0.0));
@@ -564,7 +566,7 @@ static int sytrd_launches(hipStream_t s, T* a, long lda, long sA, int n, T* d, T
   const SytrdWs<T>& ws = wk[0];
   const ProblemStrides ps{K > 1 ? sA : 0, K > 1 ? (long)wsStride : 0, K > 1 ? sV : 0};
   const long ldw = n;
-  for (int j0 = 0; j0 < n; j0 += kNB) {
+  for (int j0 = from; j0 < to; j0 += kNB) {
     const int pw = std::min(kNB, n - j0);
     for (int i = 0; i < pw; ++i) {
       const int c = j0 + i;
@@ -633,10 +635,10 @@ static int sytrd_launches(hipStream_t s, T* a, long lda, long sA, int n, T* d, T
   return 0;
 }
 
-// The launch sequence of one tridiagonalisation (3 launches per column and the panel updates:
-// about 47 000 launches at n = 15769) depends only on the sizes, the buffers and the tile
-// choice, and holds no host synchronisation: it is captured once into a HIP graph and replayed
-// for every later call with the same arguments (an SCC cycle calls it once per iteration on
+// The launch sequence of one tridiagonalisation (3 launches per column and the panel updates, up
+// to the size from which the resident kernels take over) depends only on the sizes, the buffers
+// and the tile choice, and holds no host synchronisation: it is captured once into a HIP graph
+// and replayed for every later call with the same arguments (an SCC cycle calls it once per iteration on
 // the same buffers), which removes the host launch cost between the short column kernels
 // (when switched on: set_sytrd_graphs).
 // Cleared memory inside the sequence is written by fill kernels (no memset nodes). A few
@@ -679,18 +681,12 @@ void release_sytrd_graphs() {
   g_sytrdGraphs.clear();
 }
 
+// the panels up to column `to`: launched one by one, or replayed
 template <typename T>
-int sytrd_lower_batched_t(hipStream_t s, T* a, long lda, long sA, int n, T* d, T* e, T* tau,
-                          long sV, void* work, size_t wsStride, int K) {
-  DH_CHECK(K >= 1, "sytrd: no problems");
-  DH_CHECK(wsStride >= sytrd_layout<T>(n, nullptr, nullptr), "sytrd: workspace too small");
-  DH_CHECK(K == 1 || (sA >= lda * (long)n && sV >= n && wsStride % 256 == 0),
-           "sytrd: problems overlap or are misaligned");
-  if (!g_sytrdGraphOn || g_symvProf.on || n < 2) {
-    DH_TRY(sytrd_launches<T>(s, a, lda, sA, n, d, e, tau, sV, work, wsStride, K));
-    DH_TRY(symv_prof_collect(s));
-    return 0;
-  }
+static int sytrd_panels(hipStream_t s, T* a, long lda, long sA, int n, T* d, T* e, T* tau,
+                        long sV, void* work, size_t wsStride, int K, int to) {
+  if (!g_sytrdGraphOn || g_symvProf.on || n < 2)
+    return sytrd_launches<T>(s, a, lda, sA, n, d, e, tau, sV, work, wsStride, K, 0, to);
   std::lock_guard<std::mutex> lock(g_sytrdGraphMutex);
   const SytrdGraphKey key{a, lda, sA, sV, n, K, (int)sizeof(T), d, e, tau, work, wsStride,
                           g_tileGen};
@@ -701,7 +697,7 @@ int sytrd_lower_batched_t(hipStream_t s, T* a, long lda, long sA, int n, T* d, T
       return 0;
     }
   DH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-  const int rc = sytrd_launches<T>(s, a, lda, sA, n, d, e, tau, sV, work, wsStride, K);
+  const int rc = sytrd_launches<T>(s, a, lda, sA, n, d, e, tau, sV, work, wsStride, K, 0, to);
   hipGraph_t graph = nullptr;
   const hipError_t ec = hipStreamEndCapture(s, &graph);
   if (rc != 0) {
@@ -726,6 +722,35 @@ int sytrd_lower_batched_t(hipStream_t s, T* a, long lda, long sA, int n, T* d, T
   }
   g_sytrdGraphs.push_back(SytrdGraph{key, exec, ++g_sytrdGraphUse});
   DH_HIP(hipGraphLaunch(exec, s));
+  return 0;
+}
+
+// allColumns: the blocked form to the end (the autotuner times its launches at every size)
+template <typename T>
+int sytrd_lower_batched_t(hipStream_t s, T* a, long lda, long sA, int n, T* d, T* e, T* tau,
+                          long sV, void* work, size_t wsStride, int K, bool allColumns = false) {
+  DH_CHECK(K >= 1, "sytrd: no problems");
+  DH_CHECK(wsStride >= sytrd_layout<T>(n, nullptr, nullptr), "sytrd: workspace too small");
+  DH_CHECK(K == 1 || (sA >= lda * (long)n && sV >= n && wsStride % 256 == 0),
+           "sytrd: problems overlap or are misaligned");
+  int handOver = n;
+  if (!allColumns && n > 1) DH_TRY(sytrd_resident_from(n, K, &handOver));
+  if (handOver > 0)
+    DH_TRY(sytrd_panels<T>(s, a, lda, sA, n, d, e, tau, sV, work, wsStride, K, handOver));
+  if (handOver < n) {
+    // the exchange ring lies in P, the flag in Q: both are written at panel ends only
+    static_assert(sizeof(T) * 2 * kNB >= 8 * kResidentWords, "ring larger than the panel copy");
+    SytrdWs<T> ws;
+    sytrd_layout<T>(n, &ws, static_cast<char*>(work));
+    bool done = false;
+    DH_TRY(sytrd_resident<T>(s, a, lda, K > 1 ? sA : 0, n, handOver, d, e, tau, K > 1 ? sV : 0,
+                             reinterpret_cast<unsigned long long*>(ws.P),
+                             K > 1 ? (long)(wsStride / 8) : 0, reinterpret_cast<int*>(ws.Q), K,
+                             &done));
+    if (!done)
+      DH_TRY(sytrd_launches<T>(s, a, lda, sA, n, d, e, tau, sV, work, wsStride, K, handOver, n));
+  }
+  DH_TRY(symv_prof_collect(s));
   return 0;
 }
 
@@ -957,7 +982,7 @@ static int symv_autotune_t(hipStream_t s, int n, std::vector<std::pair<int, int>
       pf.on = nn == n;
       pf.sink = nn == n ? &rec : nullptr;
       rec.clear();
-      rc = sytrd_lower_t<T>(s, a.p, nn, nn, d.p, e.p, tau.p, work.p, wb);
+      rc = sytrd_lower_batched_t<T>(s, a.p, nn, 0, nn, d.p, e.p, tau.p, 0, work.p, wb, 1, true);
       pf.sink = nullptr;
       if (rc) break;
     }
