@@ -4,12 +4,17 @@
 //
 //   C = alpha * op(A) * diag(w) * op(B) + beta * C        (column-major, LAPACK convention)
 //
-// Workgroup tile 128x128, 256 threads = 4 wave64s in a 2x2 arrangement, each wave owns a 64x64
-// sub-tile = 4x4 MFMA blocks of 16x16. K is staged through LDS in steps of 16 with a register
-// prefetch of the next step. Options used by the eigensolver and density-matrix builds:
+// Workgroup tile BT x BT (128, 64 or 32), 256 threads = 4 wave64s in a 2x2 arrangement, each wave
+// owns a (BT/2)^2 sub-tile = 4x4, 2x2 or 1 MFMA blocks of 16x16. K is staged through LDS in steps
+// of 16 with a register prefetch of the next step. The 128 tile is the efficient one; a small
+// output has too few of them for the chip (573 x 573: 25 tiles on 256 compute units, 45 us), and
+// one of the smaller tiles is taken (see pick_tile). Options used by the eigensolver and
+// density-matrix builds:
 //  * lowerOut: only tiles on/below the diagonal are computed (SYRK/SYR2K-like outputs);
 //  * klim: skip the zero part of a triangular operand;
 //  * w: per-k weights folded into op(A) (C = X diag(f) X^T for the density matrices).
+#include <utility>
+
 #include "common.h"
 #include "mfma.h"
 
@@ -26,27 +31,30 @@ int set_gemm_order(int order) {
   return 0;
 }
 
-template <typename T, bool TA, bool TB>
+template <typename T, bool TA, bool TB, int BT = kBM>
 __device__ __forceinline__ void gemm_tile(int tm, int tn, int M, int N, int K, T alpha,
                                           const T* __restrict__ A, long lda,
                                           const T* __restrict__ B, long ldb, T beta,
                                           T* __restrict__ C, long ldc, int klim,
                                           const T* __restrict__ w, int kz = 0, int nkz = 1) {
   using acc_t = typename Mfma<T>::acc_t;
+  constexpr int WB = BT / 32;          // MFMA blocks per wave and direction
+  constexpr int WR = 16 * WB;          // rows (columns) of a wave's sub-tile
+  constexpr int LQ = BT * kBK / kNT;   // elements of each operand per thread and K step
   // LDS: A and B staging during the K loop, reused for the output staging afterwards
-  constexpr int kStage = 2 * kBK * (kBM + kPad);
-  constexpr int kOut = 4 * 16 * (64 + 1);
+  constexpr int kStage = 2 * kBK * (BT + kPad);
+  constexpr int kOut = 4 * 16 * (WR + 1);
   __shared__ T smem[kStage > kOut ? kStage : kOut];
-  T (*As)[kBM + kPad] = reinterpret_cast<T (*)[kBM + kPad]>(smem);
-  T (*Bs)[kBN + kPad] = reinterpret_cast<T (*)[kBN + kPad]>(smem + kBK * (kBM + kPad));
+  T (*As)[BT + kPad] = reinterpret_cast<T (*)[BT + kPad]>(smem);
+  T (*Bs)[BT + kPad] = reinterpret_cast<T (*)[BT + kPad]>(smem + kBK * (BT + kPad));
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const int i0 = tm * kBM, j0 = tn * kBN;
+  const int i0 = tm * BT, j0 = tn * BT;
   int kbeg = 0, kend = K;
-  if (klim == kKALower) kend = min(K, i0 + kBM);
+  if (klim == kKALower) kend = min(K, i0 + BT);
   else if (klim == kKAUpper) kbeg = min(K, i0);
-  else if (klim == kKBUpper) kend = min(K, j0 + kBN);
+  else if (klim == kKBUpper) kend = min(K, j0 + BT);
   else if (klim == kKBLower) kbeg = min(K, j0);
   // split-K: slice kz of nkz (slices are multiples of the K step); partial sums added atomically
   if (nkz > 1) {
@@ -57,19 +65,19 @@ __device__ __forceinline__ void gemm_tile(int tm, int tn, int M, int N, int K, T
     kbeg = b;
   }
 
-  acc_t acc[4][4];
+  acc_t acc[WB][WB];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < WB; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
+    for (int b = 0; b < WB; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
 
-  T ra[8], rb[8];
+  T ra[LQ], rb[LQ];
   auto gload = [&](int k0) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < LQ; ++q) {
       const int e = tid + q * kNT;
       int r, c;
-      if (!TA) { r = e % kBM; c = e / kBM; } else { c = e % kBK; r = e / kBK; }
+      if (!TA) { r = e % BT; c = e / BT; } else { c = e % kBK; r = e / kBK; }
       const int gi = i0 + r, gk = k0 + c;
       T v = T(0);
       if (gi < M && gk < kend) {
@@ -79,10 +87,10 @@ __device__ __forceinline__ void gemm_tile(int tm, int tn, int M, int N, int K, T
       ra[q] = v;
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < LQ; ++q) {
       const int e = tid + q * kNT;
       int r, c;
-      if (!TB) { c = e % kBK; r = e / kBK; } else { r = e % kBN; c = e / kBN; }
+      if (!TB) { c = e % kBK; r = e / kBK; } else { r = e % BT; c = e / BT; }
       const int gj = j0 + r, gk = k0 + c;
       T v = T(0);
       if (gj < N && gk < kend) v = TB ? B[gj + (long)gk * ldb] : B[gk + (long)gj * ldb];
@@ -91,17 +99,17 @@ __device__ __forceinline__ void gemm_tile(int tm, int tn, int M, int N, int K, T
   };
   auto sstore = [&]() {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < LQ; ++q) {
       const int e = tid + q * kNT;
       int r, c;
-      if (!TA) { r = e % kBM; c = e / kBM; } else { c = e % kBK; r = e / kBK; }
+      if (!TA) { r = e % BT; c = e / BT; } else { c = e % kBK; r = e / kBK; }
       As[c][r] = ra[q];
     }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
+    for (int q = 0; q < LQ; ++q) {
       const int e = tid + q * kNT;
       int r, c;
-      if (!TB) { c = e % kBK; r = e / kBK; } else { r = e % kBN; c = e / kBN; }
+      if (!TB) { c = e % kBK; r = e / kBK; } else { r = e % BT; c = e / BT; }
       Bs[c][r] = rb[q];
     }
   };
@@ -115,57 +123,59 @@ __device__ __forceinline__ void gemm_tile(int tm, int tn, int M, int N, int K, T
       if (k0 + kBK < kend) gload(k0 + kBK);
 #pragma unroll
       for (int kk = 0; kk < kBK / 4; ++kk) {
-        T fa[4], fb[4];
+        T fa[WB], fb[WB];
         const int kr = kk * 4 + (lane >> 4);
 #pragma unroll
-        for (int m = 0; m < 4; ++m) fa[m] = As[kr][wm * 64 + m * 16 + (lane & 15)];
+        for (int m = 0; m < WB; ++m) fa[m] = As[kr][wm * WR + m * 16 + (lane & 15)];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) fb[n] = Bs[kr][wn * 64 + n * 16 + (lane & 15)];
+        for (int n = 0; n < WB; ++n) fb[n] = Bs[kr][wn * WR + n * 16 + (lane & 15)];
 #pragma unroll
-        for (int m = 0; m < 4; ++m)
+        for (int m = 0; m < WB; ++m)
 #pragma unroll
-          for (int n = 0; n < 4; ++n) acc[m][n] = Mfma<T>::op(fa[m], fb[n], acc[m][n]);
+          for (int n = 0; n < WB; ++n) acc[m][n] = Mfma<T>::op(fa[m], fb[n], acc[m][n]);
       }
     }
   }
   // Output layout of the 16x16 accumulator, column l%16 for lane l; element r sits in row
   // l/16 + 4r for FP64 and in row 4(l/16) + r for FP32 (pinned by the layout probes below).
-  // Each wave stages 16 columns x 64 rows of its sub-tile in its own LDS area and writes them
-  // back one column per store instruction (64 consecutive rows). The area is private to the
-  // wave, so only the first staging waits for the other waves (their K loop reads the same
-  // LDS); within the wave an LDS-count wait orders the staging before the reads. The 16 C
-  // values a lane updates are loaded before any of its stores.
+  // Each wave stages 16 columns x WR rows of its sub-tile in its own LDS area and writes them
+  // back, 64 / WR columns per store instruction. The area is private to the wave, so only the
+  // first staging waits for the other waves (their K loop reads the same LDS); within the wave an
+  // LDS-count wait orders the staging before the reads. The C values a lane updates are loaded
+  // before any of its stores.
   __syncthreads();
-  T* Cs = smem + wave * 16 * 65;
+  constexpr int CPS = 64 / WR, NST = 16 / CPS;   // columns per store, stores per 16 columns
+  T* Cs = smem + wave * 16 * (WR + 1);
   auto wave_lds_sync = [&]() {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0); vmcnt, expcnt untouched (gfx9 encoding)
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
   };
-  const int gi = i0 + wm * 64 + lane;
+  const int lrow = lane % WR, lcol = lane / WR;
+  const int gi = i0 + wm * WR + lrow;
 #pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int gj0 = j0 + wn * 64 + n * 16;
-    T cold[16];
+  for (int n = 0; n < WB; ++n) {
+    const int gj0 = j0 + wn * WR + n * 16 + lcol;
+    T cold[NST];
     if (beta != T(0) && nkz == 1) {
 #pragma unroll
-      for (int cc = 0; cc < 16; ++cc)
-        cold[cc] = (gi < M && gj0 + cc < N) ? C[gi + (long)(gj0 + cc) * ldc] : T(0);
+      for (int cc = 0; cc < NST; ++cc)
+        cold[cc] = (gi < M && gj0 + cc * CPS < N) ? C[gi + (long)(gj0 + cc * CPS) * ldc] : T(0);
     }
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < WB; ++m)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int rr = Mfma<T>::kRowMajorQuad ? (lane >> 4) * 4 + r : (lane >> 4) + 4 * r;
-        Cs[(lane & 15) * 65 + m * 16 + rr] = acc[m][n][r];
+        Cs[(lane & 15) * (WR + 1) + m * 16 + rr] = acc[m][n][r];
       }
     wave_lds_sync();
     if (gi < M) {
 #pragma unroll
-      for (int cc = 0; cc < 16; ++cc) {
-        const int gj = gj0 + cc;
+      for (int cc = 0; cc < NST; ++cc) {
+        const int gj = gj0 + cc * CPS;
         if (gj < N) {
-          T v = alpha * Cs[cc * 65 + lane];
+          T v = alpha * Cs[(cc * CPS + lcol) * (WR + 1) + lrow];
           T* dst = C + gi + (long)gj * ldc;
           if (nkz > 1) {
             atomicAdd(dst, v);
@@ -237,14 +247,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void g
                        (int)blockIdx.z, (int)gridDim.z);
 }
 
-template <typename T, bool TA, bool TB>
+template <typename T, bool TA, bool TB, int BT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void gemm_batched_kernel(const GemmDesc<T>* desc, T alpha,
                                                            T beta) {
   const GemmDesc<T> d = desc[blockIdx.z];
   const int tm = blockIdx.x, tn = blockIdx.y;
-  if (tm * kBM >= d.M || tn * kBN >= d.N) return;
-  gemm_tile<T, TA, TB>(tm, tn, d.M, d.N, d.K, alpha, d.A, d.lda, d.B, d.ldb, beta, d.C, d.ldc,
+  if (tm * BT >= d.M || tn * BT >= d.N) return;
+  gemm_tile<T, TA, TB, BT>(tm, tn, d.M, d.N, d.K, alpha, d.A, d.lda, d.B, d.ldb, beta, d.C, d.ldc,
                        kKFull, nullptr);
+}
+
+// The smaller tiles: plain and lower outputs only
+template <typename T, bool TA, bool TB, int BT>
+__global__ __launch_bounds__(256) void gemm_small_kernel(int M, int N, int K, T alpha, const T* A,
+                                                         long lda, const T* B, long ldb, T beta,
+                                                         T* C, long ldc, int lowerOut, int klim,
+                                                         const T* w) {
+  int tm = blockIdx.x, tn = blockIdx.y;
+  if (lowerOut) lower_tile_index(blockIdx.x, tm, tn);
+  gemm_tile<T, TA, TB, BT>(tm, tn, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, klim, w,
+                           (int)blockIdx.z, (int)gridDim.z);
+}
+
+// Tile of an output of M x N (times `batch` slices or problems): a compute unit works through its
+// share of the tiles one after the other, at a rate that falls with the tile (LDS reads per MFMA:
+// measured 0.7, 0.6 and 0.4 of the peak for 128, 64 and 32), so the time goes as
+// ceil(tiles / units) BT^2 / rate. 573 x 573: 25, 81 or 324 tiles, times 1 : 0.29 : 0.22.
+static int pick_tile(long M, long N, bool lower, long batch) {
+  constexpr long kUnits = 256;
+  int best = 128;
+  double bestCost = 0.0;
+  for (const auto& o : {std::pair<int, double>{128, 0.7}, {64, 0.6}, {32, 0.4}}) {
+    const long tm = (M + o.first - 1) / o.first, tn = (N + o.first - 1) / o.first;
+    const long tiles = (lower ? tm * (tm + 1) / 2 : tm * tn) * batch;
+    const double cost =
+        (double)((tiles + kUnits - 1) / kUnits) * o.first * o.first / o.second;
+    if (o.first == 128 || cost < 0.9 * bestCost) {
+      best = o.first;
+      bestCost = cost;
+    }
+  }
+  return best;
 }
 
 template <typename T>
@@ -259,6 +302,30 @@ int gemm(hipStream_t s, bool ta, bool tb, int M, int N, int K, T alpha, const T*
     DH_TRY(fill2d<T>(s, C, ldc, M, N, T(0)));
   }
   splitK = std::max(splitK, 1);
+  // an in-place product (C one of the operands) is only right while one tile spans its columns
+  // (rows), so that a workgroup has read what it overwrites: it keeps the large tile
+  const bool inPlace = C == A || C == B;
+  const int bt = inPlace ? kBM : pick_tile(M, N, lowerOut, splitK);
+  if (bt != kBM) {
+    const long tm = cdiv(M, bt);
+    const dim3 sg = lowerOut ? dim3((unsigned)(tm * (tm + 1) / 2)) : dim3((unsigned)tm, cdiv(N, bt), splitK);
+#define DH_GEMM_SMALL(TA_, TB_)                                                                \
+  do {                                                                                         \
+    if (bt == 64)                                                                              \
+      hipLaunchKernelGGL((gemm_small_kernel<T, TA_, TB_, 64>), sg, dim3(kNT), 0, s, M, N, K,   \
+                         alpha, A, lda, B, ldb, beta, C, ldc, (int)lowerOut, (int)klim, w);    \
+    else                                                                                       \
+      hipLaunchKernelGGL((gemm_small_kernel<T, TA_, TB_, 32>), sg, dim3(kNT), 0, s, M, N, K,   \
+                         alpha, A, lda, B, ldb, beta, C, ldc, (int)lowerOut, (int)klim, w);    \
+  } while (0)
+    if (!ta && !tb) DH_GEMM_SMALL(false, false);
+    else if (!ta && tb) DH_GEMM_SMALL(false, true);
+    else if (ta && !tb) DH_GEMM_SMALL(true, false);
+    else DH_GEMM_SMALL(true, true);
+#undef DH_GEMM_SMALL
+    DH_LAUNCH_CHECK();
+    return 0;
+  }
   dim3 grid;
   // grouped only for full-K products: with a triangular k-limit the work of a tile row grows
   // or shrinks along the rows, and XCDs given contiguous bands of rows would be unbalanced
@@ -338,10 +405,20 @@ template <typename T>
 int gemm_batched(hipStream_t s, bool ta, bool tb, const GemmDesc<T>* dDesc, int nBatch, int maxM,
                  int maxN, T alpha, T beta) {
   if (nBatch <= 0 || maxM <= 0 || maxN <= 0) return 0;
-  dim3 grid(cdiv(maxM, kBM), cdiv(maxN, kBN), nBatch);
+  const int bt = pick_tile(maxM, maxN, false, nBatch);
+  dim3 grid(cdiv(maxM, bt), cdiv(maxN, bt), nBatch);
 #define DH_GEMMB_CASE(TA_, TB_)                                                            \
-  hipLaunchKernelGGL((gemm_batched_kernel<T, TA_, TB_>), grid, dim3(kNT), 0, s, dDesc, alpha, \
-                     beta)
+  do {                                                                                      \
+    if (bt == 128)                                                                          \
+      hipLaunchKernelGGL((gemm_batched_kernel<T, TA_, TB_, 128>), grid, dim3(kNT), 0, s,    \
+                         dDesc, alpha, beta);                                               \
+    else if (bt == 64)                                                                      \
+      hipLaunchKernelGGL((gemm_batched_kernel<T, TA_, TB_, 64>), grid, dim3(kNT), 0, s,     \
+                         dDesc, alpha, beta);                                               \
+    else                                                                                    \
+      hipLaunchKernelGGL((gemm_batched_kernel<T, TA_, TB_, 32>), grid, dim3(kNT), 0, s,     \
+                         dDesc, alpha, beta);                                               \
+  } while (0)
   if (!ta && !tb) DH_GEMMB_CASE(false, false);
   else if (!ta && tb) DH_GEMMB_CASE(false, true);
   else if (ta && !tb) DH_GEMMB_CASE(true, false);
