@@ -59,7 +59,7 @@ struct EigenSolver {
   DevBuf<float> Linv32, d32, e32, tau32;
   DevBuf<double> band;          // two-stage tridiagonalisation workspace (reflectors of stage 2)
   size_t workSize = 0, bandBytes = 0;
-  bool twoStage = true;         // two-stage (band) tridiagonalisation, else one-stage
+  bool twoStage = false;        // two-stage (band) tridiagonalisation, else one-stage
   std::shared_ptr<StedcWs> sws;   // divide-and-conquer device buffers, kept between solves
   StedcWs* dc_ws() {
     if (!sws) sws.reset(stedc_ws_new(), stedc_ws_delete);
