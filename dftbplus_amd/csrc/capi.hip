@@ -26,6 +26,7 @@
 #include "neigh.h"
 #include "eigen.h"
 #include "sparse.h"
+#include "stedc.h"
 #include "zhegv.h"
 
 namespace dftbhip {
@@ -2138,19 +2139,11 @@ static int ctx_scc_step(Context& c) {
       auto dcPointBody = [&](int k) -> int {
         Context::KPointDc& r = *c.kdc[k];
         DH_HIP(hipSetDevice(dev));
-        std::vector<double> dh(n), eh(std::max(n - 1, 1));
-        DH_HIP(hipMemcpyAsync(dh.data(), c.kD.p + (size_t)k * n, n * sizeof(double),
-                              hipMemcpyDeviceToHost, r.st));
-        if (n > 1)
-          DH_HIP(hipMemcpyAsync(eh.data(), c.kE.p + (size_t)k * n, (n - 1) * sizeof(double),
-                                hipMemcpyDeviceToHost, r.st));
-        DH_HIP(hipStreamSynchronize(r.st));
-        DH_TRY(stedc(r.st, n, dh.data(), eh.data(), r.w.p, c.XK[k].p, n, r.work.p, dcWork,
-                     &infoK[k], r.ws.get()));
-        if (infoK[k] != 0) return 0;
+        DH_TRY(stedc_device(r.st, n, c.kD.p + (size_t)k * n, c.kE.p + (size_t)k * n, r.w.p,
+                            c.XK[k].p, n, r.work.p, dcWork, r.ws.get()));
         c.eigK[k].resize(n);
-        DH_HIP(hipMemcpyAsync(c.eigK[k].data(), r.w.p, n * sizeof(double), hipMemcpyDeviceToHost,
-                              r.st));
+        DH_TRY(stedc_fetch(r.st, n, r.w.p, c.eigK[k].data(), r.ws.get(), &infoK[k]));
+        if (infoK[k] != 0) return 0;
         // back-transformation on the same stream, the D&C workspace (free now) holding the
         // product L^-T (Q Z) and the reflector workspace: Q Z in place, product, copy back
         double* prod = r.work.p;

@@ -7,6 +7,7 @@
 // The contract is that of LAPACK dsygvd with itype = 1, uplo = 'L' (the routine DFTB+ calls
 // through hegvd / magmaHegvd, src/dftbp/math/eigensolver.F90:561-660, 1143-1245).
 #include "eigen.h"
+#include "stedc.h"
 
 namespace dftbhip {
 
@@ -61,17 +62,9 @@ int EigenSolver::reduce(hipStream_t s, const double* Li, const double* H, long l
 int EigenSolver::tridiag_eigen(hipStream_t s, const double* dDev, const double* eDev,
                                std::vector<double>& wHost, int* info) {
   *info = 0;
-  std::vector<double> dh(n), eh(std::max(n - 1, 1));
-  DH_HIP(hipMemcpyAsync(dh.data(), dDev, n * sizeof(double), hipMemcpyDeviceToHost, s));
-  if (n > 1)
-    DH_HIP(hipMemcpyAsync(eh.data(), eDev, (n - 1) * sizeof(double), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipStreamSynchronize(s));
-  DH_TRY(stedc(s, n, dh.data(), eh.data(), w.p, Zd.p, n, work.p, workSize, info, dc_ws()));
-  if (*info != 0) return 0;
+  DH_TRY(stedc_device(s, n, dDev, eDev, w.p, Zd.p, n, work.p, workSize, dc_ws()));
   wHost.resize(n);
-  DH_HIP(hipMemcpyAsync(wHost.data(), w.p, n * sizeof(double), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipStreamSynchronize(s));
-  return 0;
+  return stedc_fetch(s, n, w.p, wHost.data(), dc_ws(), info);
 }
 
 int EigenSolver::vectors_from(hipStream_t s, const double* Li, const double* A,
@@ -517,17 +510,13 @@ int EigenSolver::solve_mixed(hipStream_t s, const float* H, long ldh, std::vecto
     DH_TRY(sytrd_lower_f32(s, A32, n, n, d32.p, e32.p, tau32.p, work.p, workSize * sizeof(double)));
   }
   DH_HIP(hipEventRecord(ev[2], s));
-  std::vector<float> df(n), ef(std::max(n - 1, 1));
-  DH_HIP(hipMemcpyAsync(df.data(), d32.p, n * sizeof(float), hipMemcpyDeviceToHost, s));
-  if (n > 1)
-    DH_HIP(hipMemcpyAsync(ef.data(), e32.p, (n - 1) * sizeof(float), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipStreamSynchronize(s));
-  std::vector<double> dh(df.begin(), df.end()), eh(ef.begin(), ef.end());
-  DH_TRY(stedc(s, n, dh.data(), eh.data(), w.p, Zd.p, n, work.p, workSize, info, dc_ws()));
+  // the tridiagonal in FP64
+  DH_TRY((convert2d<float, double>(s, d32.p, n, d.p, n, n, 1)));
+  if (n > 1) DH_TRY((convert2d<float, double>(s, e32.p, n, e.p, n, n - 1, 1)));
+  DH_TRY(stedc_device(s, n, d.p, e.p, w.p, Zd.p, n, work.p, workSize, dc_ws()));
   DH_HIP(hipEventRecord(ev[3], s));
   wHost.resize(n);
-  DH_HIP(hipMemcpyAsync(wHost.data(), w.p, n * sizeof(double), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipStreamSynchronize(s));
+  DH_TRY(stedc_fetch(s, n, w.p, wHost.data(), dc_ws(), info));
   if (times) {
     float ms;
     for (int k = 0; k < 3; ++k) {

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "common.h"
+#include "stedc.h"
 #include "zhegv.h"
 
 namespace dftbhip {
@@ -372,21 +373,15 @@ int ZhegvSolver::solve(hipStream_t s, const double* aDev, long lda, const double
                      Hi.p, ld, n, E2.p, (long)n2);
   DH_LAUNCH_CHECK();
   DH_TRY(sytrd_lower(s, E2.p, n2, n2, d2.p, e2.p, tau2.p, work.p, workSize));
-  std::vector<double> dh(n2), eh(n2);
-  DH_HIP(hipMemcpyAsync(dh.data(), d2.p, n2 * sizeof(double), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipMemcpyAsync(eh.data(), e2.p, (n2 - 1) * sizeof(double), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipStreamSynchronize(s));
   if (!sws) sws.reset(stedc_ws_new(), stedc_ws_delete);
   int dcInfo = 0;
-  DH_TRY(stedc(s, n2, dh.data(), eh.data(), w2.p, Z2.p, n2, work.p, workSize, &dcInfo,
-               sws.get()));
+  std::vector<double> w2h(n2);
+  DH_TRY(stedc_device(s, n2, d2.p, e2.p, w2.p, Z2.p, n2, work.p, workSize, sws.get()));
+  DH_TRY(stedc_fetch(s, n2, w2.p, w2h.data(), sws.get(), &dcInfo));
   if (dcInfo != 0) {
     *info = dcInfo;
     return 0;
   }
-  std::vector<double> w2h(n2);
-  DH_HIP(hipMemcpyAsync(w2h.data(), w2.p, n2 * sizeof(double), hipMemcpyDeviceToHost, s));
-  DH_HIP(hipStreamSynchronize(s));
   wHost.resize(n);
   for (int j = 0; j < n; ++j) wHost[j] = w2h[2 * j];
   if (!vectors) return 0;
