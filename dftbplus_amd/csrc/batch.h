@@ -1,21 +1,25 @@
 // Per-molecule layout of a molecule batch and the batched kernels (batch.hip).
 #pragma once
 
+#include <memory>
+#include <vector>
+
 #include "sparse.h"
+#include "stedc.h"
 
 namespace dftbhip {
 
 constexpr int kBatchMaxOrb = 512;   // orbitals per molecule in a batch
-// size classes of the batched eigensolver, by orbital count: up to kBatchLdsSmall and
-// kBatchLdsC the reduced matrix A and the eigenvectors C stay in LDS (49 / 153 KB per
-// workgroup), up to kBatchLdsMid A alone (148 KB, C in HBM), larger molecules keep both in HBM
-constexpr int kBatchLdsSmall = 64;
-constexpr int kBatchLdsC = 112;
-constexpr int kBatchLdsMid = 190;
-constexpr int kBatchClasses = 4;
-// info of a molecule whose Jacobi sweeps did not converge within their limit (distinct from the
-// leading minor of a non-positive-definite overlap and from the negative size-class error)
-constexpr int kBatchJacobiNoConv = 1 << 24;
+// size classes of the batched eigensolver, by orbital count (largest first): above kWgBatchMax
+// Jacobi with both matrices in HBM, up to it the direct solve, whose reduction has shapes for
+// 224, 192, 128, 64 and 32 orbitals
+constexpr int kBatchClasses = 6;
+inline int batch_class(long n) {
+  return n > kWgBatchMax ? 0 : n > 192 ? 1 : n > 128 ? 2 : n > 64 ? 3 : n > 32 ? 4 : 5;
+}
+// info of a molecule whose eigensolver did not converge within its limit (distinct from the
+// leading minor of a non-positive-definite overlap)
+constexpr int kBatchEigenNoConv = 1 << 24;
 
 struct BatchLayout {
   int nmol;
@@ -33,17 +37,35 @@ int launch_batch_unpack(hipStream_t s, const PairsDev& pr, const int* norb,
                         double* dense, long denseSize);
 int launch_batch_pack(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
                       const BatchLayout& L, const double* dense, double* x);
+// Buffers and tables of the batched eigensolver for one set of geometries
+struct BatchDescs {
+  GemmDesc<double>*hc, *chc, *back;
+  int* solve;   // per molecule: solved in this call
+};
+struct BatchEigen {
+  int first[kBatchClasses + 1] = {}, maxn[kBatchClasses] = {}, direct = 0;
+  std::shared_ptr<StedcWs> dc;
+  DevBuf<double> work, d, e, tau;
+  DevBuf<GemmDesc<double>> desc;
+  DevBuf<int> solve;
+  int prepare(hipStream_t s, const BatchLayout& L, const std::vector<int>& order,
+              const std::vector<long>& orb0, const std::vector<long>& dOff);
+};
 // eigenvalues w (ascending per molecule, at orb0), eigenvectors C (packed), info per molecule
 // (0, or j+1 when the leading minor j+1 of S is not positive definite); work 3 x packed size,
 // kept between calls. Molecules with active[m] == 0 are skipped (active may be null: all).
-// warm: S is the one of the previous call on the same work array and the Jacobi sweeps start
-// from that call's eigenvectors (a cold call factors S).
-// st[0 .. kBatchClasses-1]: the streams of the size classes (largest first; may coincide)
-int launch_batch_sygv(const hipStream_t* st, const BatchLayout& L, const double* S,
+// warm: S is the one of the previous call on the same work array (a cold call factors S; the
+// Jacobi sweeps of large molecules then start from that call's eigenvectors).
+// st[0]: the stream of the call, st[1 .. kBatchClasses-1]: streams forked from it by the caller
+// and joined afterwards; done[0 .. kBatchClasses-1]: events for the forks in between. Launches
+// only, so a call can be captured.
+int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L, const double* S,
                       const double* H, double* work, double* w, double* C, int* info,
-                      const int* active, bool warm);
-int launch_batch_density(hipStream_t s, const BatchLayout& L, const double* C, const double* f,
-                         const int* nocc, double* P, const int* active);
+                      const int* active, bool warm, hipEvent_t* done);
+// P = C diag(f) C^T over the first nocc columns; work as above (B1 is overwritten)
+int launch_batch_density(hipStream_t s, BatchEigen& E, const BatchLayout& L, const double* C,
+                         const double* f, const int* nocc, double* P, const int* active,
+                         double* work);
 int launch_batch_gamma(hipStream_t s, const BatchLayout& L, const double* coords,
                        const int* species, const double* hubbu, const double* gcut, int nsp,
                        double* g);

@@ -4,12 +4,13 @@
 // consecutively and the neighbour list holds only intra-molecule pairs, so the sparse kernels
 // (H0/S assembly, shift, pack, Mulliken, pair forces, repulsive) run unchanged over the union.
 // What is per molecule lives here: the dense matrices (packed one after the other, n_m x n_m
-// column-major), the generalized eigensolver (one workgroup per molecule: Cholesky and L^-T once
-// per geometry, then per call a congruence with workgroup GEMMs and parallel cyclic Jacobi), the
-// density matrices and the cluster gamma matrix with its products and gradient. The eigensolver
-// and density kernels visit the molecules largest first (BatchLayout::order).
+// column-major), the generalized eigensolver (Cholesky and L^-T once per geometry, then per call
+// a direct solve, or for molecules above kWgBatchMax orbitals parallel cyclic Jacobi by one
+// workgroup), the density matrices and the cluster gamma matrix with its products and gradient.
+// The eigensolver and density kernels visit the molecules largest first (BatchLayout::order).
 #include "batch.h"
 #include "gamma_dev.h"
+#include "lanes.h"
 
 namespace dftbhip {
 
@@ -62,7 +63,7 @@ __global__ void batch_pack_kernel(PairsDev pr, const int* norbAtom, const long* 
 }
 
 // ------------------------------------------------------------------------------------------
-// Generalized eigensolver H C = S C E per molecule, one 1024-thread workgroup each.
+// Generalized eigensolver H C = S C E of a large molecule, one 1024-thread workgroup each.
 //
 // S is fixed for a geometry, so the reduction to standard form is done once: a cold call
 // factors S = L L^T and starts from C = L^-T. Every call forms A = C^T H C with two workgroup
@@ -213,6 +214,61 @@ __device__ void wg_gemm(int n, int kd, const double* __restrict__ X, const doubl
   __syncthreads();
 }
 
+// Cholesky S = L L^T of one molecule (B0 overwritten) and Cw = L^-T: column i of Cw is row i of
+// L^-1. False (and info) when a leading minor is not positive definite.
+__device__ bool wg_factor(int n, const double* Sm, double* B0, double* Cw, int* info) {
+  constexpr int NT = kSygvThreads;
+  const long nn = (long)n * n;
+  const int tid = threadIdx.x;
+  __shared__ int flag;
+  if (tid == 0) flag = 0;
+  for (long e = tid; e < nn; e += NT) B0[e] = Sm[e];
+  __syncthreads();
+  // Cholesky S = L L^T (lower, right-looking)
+  for (int j = 0; j < n; ++j) {
+    if (tid == 0) {
+      const double d = B0[j + (long)j * n];
+      if (!(d > 0.0)) {
+        flag = j + 1;
+      } else {
+        B0[j + (long)j * n] = sqrt(d);
+      }
+    }
+    __syncthreads();
+    if (flag != 0) {
+      if (tid == 0) *info = flag;
+      return false;
+    }
+    const double djj = B0[j + (long)j * n];
+    for (int i = j + 1 + tid; i < n; i += NT) B0[i + (long)j * n] /= djj;
+    __syncthreads();
+    const int len = n - j - 1;
+    for (long e = tid; e < (long)len * len; e += NT) {
+      const int i = j + 1 + (int)(e % len), k = j + 1 + (int)(e / len);
+      if (i >= k) B0[i + (long)k * n] -= B0[i + (long)j * n] * B0[k + (long)j * n];
+    }
+    __syncthreads();
+  }
+  // L^T into the upper triangle: row i of L is then contiguous (column i of the upper part)
+  for (long e = tid; e < nn; e += NT) {
+    const int i = (int)(e % n), k = (int)(e / n);
+    if (i > k) B0[k + (long)i * n] = B0[i + (long)k * n];
+  }
+  __syncthreads();
+  // Cw = L^-T: thread c forms column c of L^-1 by forward substitution and stores it as row c
+  // of Cw, so that the lanes of a wave read and write consecutive addresses
+  for (int c = tid; c < n; c += NT)
+    for (int i = 0; i < n; ++i) {
+      double v = 0.0;
+      if (i >= c)
+        v = ((i == c ? 1.0 : 0.0) - dot4(B0 + (long)i * n, 1, Cw + c, n, i)) /
+            B0[i + (long)i * n];
+      Cw[c + (long)i * n] = v;
+    }
+  __syncthreads();
+  return true;
+}
+
 __global__ __launch_bounds__(kSygvThreads) void batch_sygv_kernel(BatchLayout L, const int* list,
                                                                   const double* S,
                                                                   const double* H, double* work,
@@ -226,7 +282,7 @@ __global__ __launch_bounds__(kSygvThreads) void batch_sygv_kernel(BatchLayout L,
   __shared__ double rc[kBatchMaxOrb / 2], rs[kBatchMaxOrb / 2];
   __shared__ int rp[kBatchMaxOrb / 2], rq[kBatchMaxOrb / 2];
   __shared__ int perm[kBatchMaxOrb];
-  __shared__ int flag, nrot, need;
+  __shared__ int nrot, need;
   __shared__ unsigned long long dmaxBits;
   const int tid = threadIdx.x;
   const long base = L.dOff[m];
@@ -239,52 +295,7 @@ __global__ __launch_bounds__(kSygvThreads) void batch_sygv_kernel(BatchLayout L,
   double* Cm = C + base;
   double* wm = w + L.orb0[m];
   if (!warm) {
-    const double* Sm = S + base;
-    if (tid == 0) flag = 0;
-    for (long e = tid; e < nn; e += NT) B0[e] = Sm[e];
-    __syncthreads();
-    // Cholesky S = L L^T (lower, right-looking)
-    for (int j = 0; j < n; ++j) {
-      if (tid == 0) {
-        const double d = B0[j + (long)j * n];
-        if (!(d > 0.0)) {
-          flag = j + 1;
-        } else {
-          B0[j + (long)j * n] = sqrt(d);
-        }
-      }
-      __syncthreads();
-      if (flag != 0) {
-        if (tid == 0) info[m] = flag;
-        return;
-      }
-      const double djj = B0[j + (long)j * n];
-      for (int i = j + 1 + tid; i < n; i += NT) B0[i + (long)j * n] /= djj;
-      __syncthreads();
-      const int len = n - j - 1;
-      for (long e = tid; e < (long)len * len; e += NT) {
-        const int i = j + 1 + (int)(e % len), k = j + 1 + (int)(e / len);
-        if (i >= k) B0[i + (long)k * n] -= B0[i + (long)j * n] * B0[k + (long)j * n];
-      }
-      __syncthreads();
-    }
-    // L^T into the upper triangle: row i of L is then contiguous (column i of the upper part)
-    for (long e = tid; e < nn; e += NT) {
-      const int i = (int)(e % n), k = (int)(e / n);
-      if (i > k) B0[k + (long)i * n] = B0[i + (long)k * n];
-    }
-    __syncthreads();
-    // Cw = L^-T: thread c forms column c of L^-1 by forward substitution and stores it as row c
-    // of Cw, so that the lanes of a wave read and write consecutive addresses
-    for (int c = tid; c < n; c += NT)
-      for (int i = 0; i < n; ++i) {
-        double v = 0.0;
-        if (i >= c)
-          v = ((i == c ? 1.0 : 0.0) - dot4(B0 + (long)i * n, 1, Cw + c, n, i)) /
-              B0[i + (long)i * n];
-        Cw[c + (long)i * n] = v;
-      }
-    __syncthreads();
+    if (!wg_factor(n, S + base, B0, Cw, info + m)) return;
   }
   // A = Cw^T H Cw (symmetrized)
   wg_gemm<false, false>(n, n, Hm, Cw, nullptr, B1, Xs, Ys);
@@ -433,255 +444,142 @@ __global__ __launch_bounds__(kSygvThreads) void batch_sygv_kernel(BatchLayout L,
   }
   // a molecule whose last allowed sweep still rotated is reported (info > 0), not taken as
   // converged
-  if (tid == 0) info[m] = done ? 0 : kBatchJacobiNoConv;
+  if (tid == 0) info[m] = done ? 0 : kBatchEigenNoConv;
 }
 
-// The same eigensolver for molecules of at most kMaxN orbitals with A resident in LDS (upper
-// triangle packed by columns: (i, j), i <= j, at i + j(j+1)/2) and, for kCLds, C as well: a
-// Jacobi round then waits on LDS alone. Otherwise C stays in HBM and each round ends with a
-// full barrier. The LDS block of A doubles as the GEMM staging before the sweeps.
-__device__ __forceinline__ int sym_idx(int i, int j) {
-  return i <= j ? i + j * (j + 1) / 2 : j + i * (i + 1) / 2;
-}
-
-// The smallest class (49 KB of LDS per workgroup) is held to 64 VGPRs so that two 1024-thread
-// workgroups share a CU; the larger classes fill a CU's LDS with one.
-template <int kMaxN, bool kCLds>
-__global__ __launch_bounds__(kSygvThreads)
-__attribute__((amdgpu_waves_per_eu(kMaxN <= 64 ? 8 : 1))) void batch_sygv_lds_kernel(
-    BatchLayout L, const int* list, const double* S, const double* H, double* work, double* w,
-    double* C, int* info, const int* active, int warm) {
-  constexpr int NT = kSygvThreads;
-  constexpr int kPacked = kMaxN * (kMaxN + 1) / 2;
-  constexpr int kStage = 2 * kGK * (kGT + 1);
-  __shared__ double As[kPacked > kStage ? kPacked : kStage];
-  __shared__ double Cs[kCLds ? kMaxN * kMaxN : 1];
-  __shared__ double rc[kMaxN / 2 + 1], rs[kMaxN / 2 + 1];
-  __shared__ int rp[kMaxN / 2 + 1], rq[kMaxN / 2 + 1];
-  __shared__ int perm[kMaxN];
-  __shared__ int flag, nrot, need;
-  __shared__ unsigned long long dmaxBits;
+// ------------------------------------------------------------------------------------------
+// Direct eigensolver for molecules of up to kWgBatchMax orbitals: Cw = L^-T once per geometry,
+// then per call A = Cw^T H Cw (batched MFMA GEMMs), tridiagonalisation with the matrix in the
+// registers of one workgroup (sytrd_resident.hip), divide and conquer of all molecules together
+// (stedc.hip), the reflectors applied to strips of eigenvectors, and C = Cw (Q Z). A parallel
+// cyclic Jacobi with A and C in LDS ran here before, n dependent rounds per sweep and 7 to 10
+// sweeps. One SCC cycle of 32 molecules of 13 to 190 orbitals: 135 ms before, 16.7 ms now; of
+// 1000 molecules: 250 ms before, 51 ms now. Bound by the column chain of the reduction (0.38 ms
+// per iteration for 190 orbitals, 0.12 for 112), then by the solve's own latencies.
+// ------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(kSygvThreads) void batch_factor_kernel(BatchLayout L, const int* list,
+                                                                    const double* S, double* work,
+                                                                    int* info) {
   const int m = list[blockIdx.x];
-  if (active && !active[m]) return;   // converged: eigenpairs stay from the last pass
-  const int tid = threadIdx.x;
-  const long base = L.dOff[m];
   const int n = (int)(L.orb0[m + 1] - L.orb0[m]);
-  if (n > kMaxN) {   // a molecule in the wrong size class: reported, nothing touched
-    if (tid == 0) info[m] = -n;
-    return;
-  }
-  const long nn = (long)n * n;
-  double* B0 = work + 3 * base;
-  double* B1 = B0 + nn;
-  double* Cw = B1 + nn;
-  if (!warm) {
-    if (tid == 0) flag = 0;
-    for (long e = tid; e < nn; e += NT) B0[e] = S[base + e];
-    __syncthreads();
-    for (int j = 0; j < n; ++j) {
-      if (tid == 0) {
-        const double d = B0[j + (long)j * n];
-        if (!(d > 0.0)) {
-          flag = j + 1;
-        } else {
-          B0[j + (long)j * n] = sqrt(d);
-        }
-      }
-      __syncthreads();
-      if (flag != 0) {
-        if (tid == 0) info[m] = flag;
-        return;
-      }
-      const double djj = B0[j + (long)j * n];
-      for (int i = j + 1 + tid; i < n; i += NT) B0[i + (long)j * n] /= djj;
-      __syncthreads();
-      const int len = n - j - 1;
-      for (long e = tid; e < (long)len * len; e += NT) {
-        const int i = j + 1 + (int)(e % len), k = j + 1 + (int)(e / len);
-        if (i >= k) B0[i + (long)k * n] -= B0[i + (long)j * n] * B0[k + (long)j * n];
-      }
-      __syncthreads();
-    }
-    for (long e = tid; e < nn; e += NT) {
-      const int i = (int)(e % n), k = (int)(e / n);
-      if (i > k) B0[k + (long)i * n] = B0[i + (long)k * n];
-    }
-    __syncthreads();
-    for (int c = tid; c < n; c += NT)
-      for (int i = 0; i < n; ++i) {
-        double v = 0.0;
-        if (i >= c)
-          v = ((i == c ? 1.0 : 0.0) - dot4(B0 + (long)i * n, 1, Cw + c, n, i)) /
-              B0[i + (long)i * n];
-        Cw[c + (long)i * n] = v;
-      }
-    __syncthreads();
-  }
-  double (*Xs)[kGT + 1] = reinterpret_cast<double (*)[kGT + 1]>(As);
-  double (*Ys)[kGT + 1] = reinterpret_cast<double (*)[kGT + 1]>(As + kGK * (kGT + 1));
-  wg_gemm<false, false>(n, n, H + base, Cw, nullptr, B1, Xs, Ys);
-  wg_gemm<true, false>(n, n, Cw, B1, nullptr, B0, Xs, Ys);
-  // A (symmetrized) into LDS
-  for (long e = tid; e < nn; e += NT) {
-    const int i = (int)(e % n), j = (int)(e / n);
-    if (i <= j) As[i + j * (j + 1) / 2] = 0.5 * (B0[i + (long)j * n] + B0[j + (long)i * n]);
-    if (kCLds) Cs[e] = Cw[e];
-  }
-  __syncthreads();
-  double* Cr = kCLds ? Cs : Cw;   // the C the sweeps rotate
-  auto lds_barrier = [&]() {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0); vmcnt, expcnt untouched (gfx9 encoding)
-    __builtin_amdgcn_s_barrier();
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  };
-  const int N2 = n + (n & 1);
-  const int np = N2 / 2;
-  const int nunit = np * (np + 1) / 2;
-  const int npair = n * (n - 1) / 2;
-  // rounding level of the matrix: 4 eps max |a_ii| (bits of non-negative doubles order as
-  // unsigned integers, so the maximum is an integer atomic)
-  if (tid == 0) dmaxBits = 0ull;
-  __syncthreads();
-  {
-    double dm = 0.0;
-    for (int i = tid; i < n; i += NT) dm = fmax(dm, fabs(As[sym_idx(i, i)]));
-    atomicMax(&dmaxBits, (unsigned long long)__double_as_longlong(dm));
-  }
-  __syncthreads();
-  const double rotFloor = 4.0 * 2.220446049250313e-16 * __longlong_as_double((long long)dmaxBits);
-  bool done = n <= 1;
-  for (int sweep = 0; sweep < kJacobiMaxSweeps && n > 1; ++sweep) {
-    // a sweep in which no pair passes the rotation test changes nothing: test all pairs first
-    if (tid == 0) {
-      nrot = 0;
-      need = 0;
-    }
-    lds_barrier();
-    for (int u = tid; u < npair; u += NT) {
-      int k1, k2;
-      unit_pairs(u, k1, k2);
-      const int p = k1, q = k2 + 1;
-      const double apq = As[sym_idx(p, q)];
-      const double app = As[sym_idx(p, p)], aqq = As[sym_idx(q, q)];
-      if (jacobi_rotates(apq, app, aqq, rotFloor)) need = 1;
-    }
-    lds_barrier();
-    if (need == 0) {
-      done = true;
-      break;
-    }
-    for (int r = 0; r < N2 - 1; ++r) {
-      for (int k = tid; k < np; k += NT) {
-        int p, q;
-        jacobi_pair(N2, r, k, p, q);
-        double c = 1.0, s = 0.0;
-        if (p < n && q < n) {
-          const double apq = As[sym_idx(p, q)];
-          const double app = As[sym_idx(p, p)], aqq = As[sym_idx(q, q)];
-          if (jacobi_rotates(apq, app, aqq, rotFloor)) {
-            const double th = (aqq - app) / (2.0 * apq);
-            const double t = copysign(1.0, th) / (fabs(th) + sqrt(th * th + 1.0));
-            c = 1.0 / sqrt(t * t + 1.0);
-            s = t * c;
-            atomicAdd(&nrot, 1);
-          }
-        }
-        rp[k] = p;
-        rq[k] = q;
-        rc[k] = c;
-        rs[k] = s;
-      }
-      lds_barrier();
-      // A <- J^T A J over the unordered 2 x 2 blocks (pairs k1 <= k2)
-      for (int u = tid; u < nunit; u += NT) {
-        int k1, k2;
-        unit_pairs(u, k1, k2);
-        const double s1 = rs[k1], s2 = rs[k2];
-        if (s1 == 0.0 && s2 == 0.0) continue;
-        const double c1 = rc[k1], c2 = rc[k2];
-        const int row[2] = {rp[k1], rq[k1]}, col[2] = {rp[k2], rq[k2]};
-        double x[4];
-        int o[4];
-        bool v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int ri = row[e & 1], ci = col[e >> 1];
-          v[e] = ri < n && ci < n;
-          o[e] = v[e] ? sym_idx(ri, ci) : 0;
-          x[e] = v[e] ? As[o[e]] : 0.0;
-        }
-        // e = 0 (p1, p2), 1 (q1, p2), 2 (p1, q2), 3 (q1, q2); columns first
-        const double y0 = c2 * x[0] - s2 * x[2];
-        const double y1 = c2 * x[1] - s2 * x[3];
-        const double y2 = s2 * x[0] + c2 * x[2];
-        const double y3 = s2 * x[1] + c2 * x[3];
-        const double z[4] = {c1 * y0 - s1 * y1, s1 * y0 + c1 * y1, c1 * y2 - s1 * y3,
-                             s1 * y2 + c1 * y3};
-        if (k1 == k2) {
-          // (p, p), (q, q) and the shared off-diagonal element
-          if (v[0]) As[o[0]] = z[0];
-          if (v[3]) As[o[3]] = z[3];
-          if (v[2]) As[o[2]] = z[2];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (v[e]) As[o[e]] = z[e];
-        }
-      }
-      // columns of C: LDS-resident C needs only the LDS barrier below; C in HBM is shared
-      // between the threads of a row across rounds, so its stores complete first
-      if (kCLds) {
-        rotate_columns<8>(Cr, n, np, rp, rq, rc, rs);
-      } else {
-        rotate_columns<10>(Cr, n, np, rp, rq, rc, rs);
-        __syncthreads();
-      }
-      lds_barrier();
-    }
-    const int nr = nrot;
-    lds_barrier();   // every thread has read nrot before the next sweep clears it
-    if (nr == 0) {
-      done = true;
-      break;
-    }
-  }
-  __syncthreads();   // every column of C written before other threads read it
-  double* wm = w + L.orb0[m];
-  for (int i = tid; i < n; i += NT) {
-    const double di = As[sym_idx(i, i)];
-    int rank = 0;
-    for (int j = 0; j < n; ++j) {
-      const double dj = As[sym_idx(j, j)];
-      rank += (dj < di || (dj == di && j < i)) ? 1 : 0;
-    }
-    perm[rank] = i;
-    wm[rank] = di;
-  }
-  __syncthreads();
-  double* Cm = C + base;
-  for (long e = tid; e < nn; e += NT) {
-    const int i = (int)(e % n), c = (int)(e / n);
-    Cm[e] = Cr[i + (long)perm[c] * n];
-    if (kCLds) Cw[e] = Cs[e];   // the next warm call starts from the rotated C
-  }
-  // a molecule whose last allowed sweep still rotated is reported (info > 0), not taken as
-  // converged
-  if (tid == 0) info[m] = done ? 0 : kBatchJacobiNoConv;
+  double* B0 = work + 3 * L.dOff[m];
+  if (wg_factor(n, S + L.dOff[m], B0, B0 + 2 * (long)n * n, info + m) && threadIdx.x == 0)
+    info[m] = 0;
 }
 
-// P_m = C_m diag(f) C_m^T over the first nocc[m] columns (lower and upper)
-__global__ __launch_bounds__(kSygvThreads) void batch_density_kernel(BatchLayout L,
-                                                                     const double* C,
-                                                                     const double* f,
-                                                                     const int* nocc, double* P,
-                                                                     const int* active) {
-  const int m = L.order[blockIdx.x];
-  if (active && !active[m]) return;
-  __shared__ double Xs[kGK][kGT + 1], Ys[kGK][kGT + 1];
+// The products of a call, empty for molecules that are not active (or whose overlap failed)
+__global__ void batch_desc_kernel(BatchLayout L, const int* list, int count, const double* H,
+                                  double* work, double* C, const int* info, const int* active,
+                                  BatchDescs g) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= count) return;
+  const int m = list[t];
+  const bool on = (!active || active[m]) && info[m] == 0;
+  const int n = on ? (int)(L.orb0[m + 1] - L.orb0[m]) : 0;
+  const long nn = L.dOff[m + 1] - L.dOff[m], ld = L.orb0[m + 1] - L.orb0[m];
+  double* B0 = work + 3 * L.dOff[m];
+  double* B1 = B0 + nn;
+  const double* Cw = B1 + nn;
+  g.hc[t] = {n, n, n, H + L.dOff[m], ld, Cw, ld, B1, ld};
+  g.chc[t] = {n, n, n, Cw, ld, B1, ld, B0, ld};
+  g.back[t] = {n, n, n, Cw, ld, B1, ld, C + L.dOff[m], ld};
+  g.solve[m] = on;
+}
+
+// Z <- Q Z for the reflectors in A (below the subdiagonal of its columns): eight lanes per column
+// of Z, lane g rows g + 8 r, all rows in registers, a wave eight columns; the reflectors are
+// applied one after the other without any barrier, the next one's rows loaded meanwhile (without
+// conditions: the rows above it are set to zero at their use). Bound by the chain of a reflector
+// (dot product, sum over eight lanes, update): 103 us for 190 orbitals; 273 us with one
+// accumulator and the row ranges tested per load.
+// reflectors c1 down to c0, which leave the rows below 8 R0 as they are
+template <int RQ, int R0>
+__device__ __forceinline__ void apply_reflectors(int n, const double* A, const double* tm, int g,
+                                                 int c1, int c0, double (&z)[RQ]) {
+  if (c1 < c0) return;
+  constexpr int K = RQ - R0;
+  double v[K];
+  auto load = [&](int c) {
+#pragma unroll
+    for (int r = 0; r < K; ++r) v[r] = A[min(g + 8 * (R0 + r), n - 1) + c * n];
+  };
+  load(c1);
+  double t = tm[c1];
+  for (int c = c1; c >= c0; --c) {
+    double u[K];
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      const int i = g + 8 * (R0 + r);
+      u[r] = i > c + 1 && i < n ? v[r] : (i == c + 1 ? 1.0 : 0.0);
+    }
+    const double tc = t;
+    const int cn = max(c - 1, 0);
+    load(cn);
+    t = tm[cn];
+    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+      double& p = (r & 3) == 0 ? p0 : (r & 3) == 1 ? p1 : (r & 3) == 2 ? p2 : p3;
+      p = fma(u[r], z[R0 + r], p);
+    }
+    const double dot = -tc * octet_sum((p0 + p1) + (p2 + p3));
+#pragma unroll
+    for (int r = 0; r < K; ++r) z[R0 + r] = fma(dot, u[r], z[R0 + r]);
+  }
+}
+
+template <int RQ>
+__global__ __launch_bounds__(256) void batch_apply_q_kernel(BatchLayout L, const int* list,
+                                                            const int* solve, double* work,
+                                                            const double* tau) {
+  const int m = list[blockIdx.y];
+  if (!solve[m]) return;
+  const int n = (int)(L.orb0[m + 1] - L.orb0[m]);
+  const int lane = threadIdx.x & 63, g = lane & 7;
+  const int col = blockIdx.x * 32 + (threadIdx.x >> 6) * 8 + (lane >> 3);
+  if (blockIdx.x * 32 + (threadIdx.x >> 6) * 8 >= n || n > 8 * RQ) return;   // whole waves
+  const double* A = work + 3 * L.dOff[m];
+  double* Z = work + 3 * L.dOff[m] + (long)n * n + (long)min(col, n - 1) * n;
+  const double* tm = tau + L.orb0[m];
+  double z[RQ];
+#pragma unroll
+  for (int r = 0; r < RQ; ++r) z[r] = g + 8 * r < n ? Z[g + 8 * r] : 0.0;
+  // reflector c has rows from c + 1 on: four ranges of c, each with the rows it can reach
+  constexpr int S1 = RQ / 4, S2 = RQ / 2, S3 = 3 * RQ / 4;
+  apply_reflectors<RQ, S3>(n, A, tm, g, n - 2, 8 * S3 - 1, z);
+  apply_reflectors<RQ, S2>(n, A, tm, g, min(n - 2, 8 * S3 - 2), 8 * S2 - 1, z);
+  apply_reflectors<RQ, S1>(n, A, tm, g, min(n - 2, 8 * S2 - 2), 8 * S1 - 1, z);
+  apply_reflectors<RQ, 0>(n, A, tm, g, min(n - 2, 8 * S1 - 2), 0, z);
+  if (col < n)
+#pragma unroll
+    for (int r = 0; r < RQ; ++r)
+      if (g + 8 * r < n) Z[g + 8 * r] = z[r];
+}
+
+// info of a molecule from its divide and conquer
+__global__ void batch_info_kernel(const int* list, int count, const int* dc, int* info) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < count && dc[t] > 0) info[list[t]] = kBatchEigenNoConv;
+}
+
+// B1 = C diag(f) over the first nocc columns and the product P = B1 C^T
+__global__ void batch_scale_kernel(BatchLayout L, const int* list, const double* C, const double* f,
+                                   const int* nocc, double* P, const int* active, double* work,
+                                   GemmDesc<double>* desc) {
+  const int t = blockIdx.y, m = list[t];
   const long base = L.dOff[m];
   const int n = (int)(L.orb0[m + 1] - L.orb0[m]);
-  wg_gemm<false, true>(n, nocc[m], C + base, C + base, f + L.orb0[m], P + base, Xs, Ys);
+  const bool on = !active || active[m];
+  double* B1 = work + 3 * base + (long)n * n;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const int nd = on ? n : 0;
+    desc[t] = {nd, nd, nocc[m], B1, (long)n, C + base, (long)n, P + base, (long)n};
+  }
+  if (!on) return;
+  const long len = (long)n * nocc[m];
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < len;
+       e += (long)gridDim.x * blockDim.x)
+    B1[e] = C[base + e] * f[L.orb0[m] + e / n];
 }
 
 // gamma_m: 1/r off the diagonal minus the short-range expGamma part within its cutoff (on the
@@ -768,38 +666,124 @@ int launch_batch_pack(hipStream_t s, const PairsDev& pr, const int* norb, const 
   return 0;
 }
 
-int launch_batch_sygv(const hipStream_t* st, const BatchLayout& L, const double* S,
-                      const double* H, double* work, double* w, double* C, int* info,
-                      const int* active, bool warm) {
-  DH_CHECK(L.ncls[0] + L.ncls[1] + L.ncls[2] + L.ncls[3] == L.nmol,
-           "batch_sygv: size classes do not cover the batch");
-  const int wm = warm ? 1 : 0;
-  const int* list = L.order;   // molecules by decreasing size: the classes in turn
-  if (L.ncls[0] > 0)
-    hipLaunchKernelGGL(batch_sygv_kernel, dim3(L.ncls[0]), dim3(kSygvThreads), 0, st[0], L, list,
-                       S, H, work, w, C, info, active, wm);
-  list += L.ncls[0];
-  if (L.ncls[1] > 0)
-    hipLaunchKernelGGL((batch_sygv_lds_kernel<kBatchLdsMid, false>), dim3(L.ncls[1]),
-                       dim3(kSygvThreads), 0, st[1], L, list, S, H, work, w, C, info, active, wm);
-  list += L.ncls[1];
-  if (L.ncls[2] > 0)
-    hipLaunchKernelGGL((batch_sygv_lds_kernel<kBatchLdsC, true>), dim3(L.ncls[2]),
-                       dim3(kSygvThreads), 0, st[2], L, list, S, H, work, w, C, info, active, wm);
-  list += L.ncls[2];
-  if (L.ncls[3] > 0)
-    hipLaunchKernelGGL((batch_sygv_lds_kernel<kBatchLdsSmall, true>), dim3(L.ncls[3]),
-                       dim3(kSygvThreads), 0, st[3], L, list, S, H, work, w, C, info, active, wm);
-  DH_LAUNCH_CHECK();
+int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<int>& order,
+                        const std::vector<long>& orb0, const std::vector<long>& dOff) {
+  int nDirect = 0;
+  first[0] = 0;
+  for (int c = 0; c < kBatchClasses; ++c) {
+    first[c + 1] = first[c] + L.ncls[c];
+    maxn[c] = L.ncls[c] > 0
+                  ? (int)(orb0[order[first[c]] + 1] - orb0[order[first[c]]])   // largest first
+                  : 0;
+    if (c > 0) nDirect += L.ncls[c];
+  }
+  DH_CHECK(first[kBatchClasses] == L.nmol, "batch_sygv: size classes do not cover the batch");
+  std::vector<DcBlock> blocks;
+  for (int t = first[1]; t < L.nmol; ++t) {
+    const int m = order[t];
+    const int n = (int)(orb0[m + 1] - orb0[m]);
+    // z goes to B1 of the molecule's work area
+    blocks.push_back({n, orb0[m], dOff[m], 3 * dOff[m] + (long)n * n, n, m});
+  }
+  if (!dc) dc.reset(stedc_ws_new(), stedc_ws_delete);
+  size_t dcWork = 0;
+  if (!blocks.empty()) DH_TRY(stedc_many_prepare(s, blocks, dc.get(), &dcWork));
+  DH_TRY(work.alloc(dcWork));
+  DH_TRY(desc.alloc(4 * (size_t)std::max(L.nmol, 1)));
+  DH_TRY(solve.alloc(std::max(L.nmol, 1)));
+  const size_t norb = orb0.back();
+  DH_TRY(d.alloc(norb));
+  DH_TRY(e.alloc(norb));
+  DH_TRY(tau.alloc(norb));
+  direct = nDirect;
   return 0;
 }
 
-int launch_batch_density(hipStream_t s, const BatchLayout& L, const double* C, const double* f,
-                         const int* nocc, double* P, const int* active) {
-  if (L.nmol == 0) return 0;
-  hipLaunchKernelGGL(batch_density_kernel, dim3(L.nmol), dim3(kSygvThreads), 0, s, L, C, f, nocc,
-                     P, active);
+int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L, const double* S,
+                      const double* H, double* work, double* w, double* C, int* info,
+                      const int* active, bool warm, hipEvent_t* done) {
+  hipStream_t s = st[0];
+  if (L.ncls[0] > 0) {
+    hipLaunchKernelGGL(batch_sygv_kernel, dim3(L.ncls[0]), dim3(kSygvThreads), 0, st[1], L,
+                       L.order, S, H, work, w, C, info, active, warm ? 1 : 0);
+    DH_LAUNCH_CHECK();
+  }
+  if (E.direct == 0) return 0;
+  const int* list = L.order + E.first[1];
+  const int nd = E.direct;
+  GemmDesc<double>* g = E.desc.p;
+  const BatchDescs ds{g, g + L.nmol, g + 2 * (size_t)L.nmol, E.solve.p};
+  if (!warm) {
+    hipLaunchKernelGGL(batch_factor_kernel, dim3(nd), dim3(kSygvThreads), 0, s, L, list, S, work,
+                       info);
+    DH_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(batch_desc_kernel, dim3(cdiv(nd, 256)), dim3(256), 0, s, L, list, nd, H, work,
+                     C, info, active, ds);
   DH_LAUNCH_CHECK();
+  auto each = [&](auto&& f) -> int {
+    for (int c = 1; c < kBatchClasses; ++c)
+      if (L.ncls[c] > 0) DH_TRY(f(c, E.first[c] - E.first[1], L.ncls[c], E.maxn[c]));
+    return 0;
+  };
+  // the classes' reductions side by side: a large molecule's chain of columns is long, and its
+  // class has few workgroups
+  DH_HIP(hipEventRecord(done[0], s));
+  DH_TRY(each([&](int c, int o, int cnt, int mx) -> int {
+    hipStream_t sc = st[c];
+    if (c > 1) DH_HIP(hipStreamWaitEvent(sc, done[0], 0));
+    else sc = s;
+    DH_TRY(gemm_batched<double>(sc, false, false, ds.hc + o, cnt, mx, mx, 1.0, 0.0));
+    DH_TRY(gemm_batched<double>(sc, true, false, ds.chc + o, cnt, mx, mx, 1.0, 0.0));
+    WgBatch bt;
+    bt.list = list + o;
+    bt.active = E.solve.p;
+    bt.aOff = L.dOff;
+    bt.aMul = 3;
+    bt.vOff = L.orb0;
+    DH_TRY(sytrd_wg_batch(sc, work, cnt, mx, bt, E.d.p, E.e.p, E.tau.p));
+    if (c > 1) {
+      DH_HIP(hipEventRecord(done[c], sc));
+      DH_HIP(hipStreamWaitEvent(s, done[c], 0));
+    }
+    return 0;
+  }));
+  DH_TRY(stedc_many(s, E.d.p, E.e.p, w, work, E.work.p, E.solve.p, E.dc.get()));
+  hipLaunchKernelGGL(batch_info_kernel, dim3(cdiv(nd, 256)), dim3(256), 0, s, list, nd,
+                     stedc_info(E.dc.get()), info);
+  DH_LAUNCH_CHECK();
+  return each([&](int c, int o, int cnt, int mx) -> int {
+    for (int p = 0; p < cnt; p += 32768) {
+      const dim3 grid(cdiv(mx, 32), std::min(32768, cnt - p));
+#define DH_APPLY(RQ_)                                                                           \
+  hipLaunchKernelGGL((batch_apply_q_kernel<RQ_>), grid, dim3(256), 0, s, L, list + o + p, E.solve.p, \
+                     work, E.tau.p)
+      if (mx <= 32) DH_APPLY(4);
+      else if (mx <= 64) DH_APPLY(8);
+      else if (mx <= 128) DH_APPLY(16);
+      else if (mx <= 192) DH_APPLY(24);
+      else DH_APPLY(28);
+#undef DH_APPLY
+      DH_LAUNCH_CHECK();
+    }
+    return gemm_batched<double>(s, false, false, ds.back + o, cnt, mx, mx, 1.0, 0.0);
+  });
+}
+
+int launch_batch_density(hipStream_t s, BatchEigen& E, const BatchLayout& L, const double* C,
+                         const double* f, const int* nocc, double* P, const int* active,
+                         double* work) {
+  GemmDesc<double>* g = E.desc.p + 3 * (size_t)L.nmol;
+  for (int c = 0; c < kBatchClasses; ++c) {
+    const int mx = E.maxn[c];
+    for (int p = 0; p < L.ncls[c]; p += 32768) {
+      const int cnt = std::min(32768, L.ncls[c] - p), o = E.first[c] + p;
+      hipLaunchKernelGGL(batch_scale_kernel, dim3(cdiv((long)mx * mx, 2048), cnt), dim3(256), 0, s,
+                         L, L.order + o, C, f, nocc, P, active, work, g + o);
+      DH_LAUNCH_CHECK();
+      DH_TRY(gemm_batched<double>(s, false, true, g + o, cnt, mx, mx, 1.0, 0.0));
+    }
+  }
   return 0;
 }
 

@@ -2609,7 +2609,8 @@ struct BatchContext {
   // fork them from s and join them back
   static constexpr int kSx = kBatchClasses - 1;
   hipStream_t sx[kSx] = {};
-  hipEvent_t fork = nullptr, join[kSx] = {};
+  hipEvent_t fork = nullptr, join[kSx] = {}, stage[kBatchClasses] = {};
+  BatchEigen be;
   // SCC iteration with the Fermi levels, energies, convergence and Broyden mixing on the device
   // (sccMode 1: launched one by one; 2: the warm iterations replay one captured HIP graph) or
   // on host threads (sccMode 0)
@@ -2632,6 +2633,8 @@ struct BatchContext {
     for (hipStream_t x : sx)
       if (x) (void)hipStreamDestroy(x);
     for (hipEvent_t e : join)
+      if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : stage)
       if (e) (void)hipEventDestroy(e);
     if (fork) (void)hipEventDestroy(fork);
   }
@@ -2736,7 +2739,7 @@ static int batch_geometry(BatchContext& b, int nmol, const int* natMol, const do
   for (int& c : b.L.ncls) c = 0;
   for (int m : order) {
     const long nm = b.orb0[m + 1] - b.orb0[m];
-    ++b.L.ncls[nm > kBatchLdsMid ? 0 : nm > kBatchLdsC ? 1 : nm > kBatchLdsSmall ? 2 : 3];
+    ++b.L.ncls[batch_class(nm)];
   }
   b.L.atom0 = b.atom0D.p;
   b.L.orb0 = b.orb0D.p;
@@ -2751,6 +2754,7 @@ static int batch_geometry(BatchContext& b, int nmol, const int* natMol, const do
   for (DevBuf<double>* x : {&b.Sd, &b.Hd, &b.Cv, &b.P}) DH_TRY(x->alloc(b.denseSize));
   DH_TRY(b.work.alloc(3 * b.denseSize));
   DH_TRY(b.gamma.alloc(b.gammaSize));
+  DH_TRY(b.be.prepare(s, b.L, order, b.orb0, b.dOff));
   DH_TRY(b.infoD.alloc(nmol));
   DH_TRY(b.noccD.alloc(nmol));
   DH_TRY(b.activeD.alloc(nmol));
@@ -2882,8 +2886,8 @@ static int batch_scc_step(BatchContext& b) {
   for (int q = 0; q < BatchContext::kSx; ++q) DH_HIP(hipStreamWaitEvent(b.sx[q], b.fork, 0));
   hipStream_t st[kBatchClasses] = {s};
   for (int q = 0; q < BatchContext::kSx; ++q) st[q + 1] = b.sx[q];
-  DH_TRY(launch_batch_sygv(st, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p, b.infoD.p,
-                           b.activeD.p, it > 1));
+  DH_TRY(launch_batch_sygv(st, b.be, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p, b.infoD.p,
+                           b.activeD.p, it > 1, b.stage));
   for (int q = 0; q < BatchContext::kSx; ++q) {
     DH_HIP(hipEventRecord(b.join[q], b.sx[q]));
     DH_HIP(hipStreamWaitEvent(s, b.join[q], 0));
@@ -2895,12 +2899,10 @@ static int batch_scc_step(BatchContext& b) {
   std::copy(b.pEig.p, b.pEig.p + n, b.eigv.begin());
   for (int m = 0; m < nmol; ++m)
     if (info[m] != 0) {
-      set_error(info[m] == kBatchJacobiNoConv
-                    ? "batch: Jacobi eigensolver of molecule " + std::to_string(m) +
-                          " did not converge within its sweep limit"
-                : info[m] < 0 ? "batch: molecule " + std::to_string(m) + " of " +
-                                    std::to_string(-info[m]) + " orbitals in a smaller size class"
-                              : "batch: overlap of molecule " + std::to_string(m) +
+      set_error(info[m] == kBatchEigenNoConv
+                    ? "batch: eigensolver of molecule " + std::to_string(m) +
+                          " did not converge within its iteration limit"
+                    : "batch: overlap of molecule " + std::to_string(m) +
                                     " not positive definite (minor " + std::to_string(info[m]) +
                                     ")");
       return kErrState;
@@ -2918,7 +2920,8 @@ static int batch_scc_step(BatchContext& b) {
   std::copy(b.fill.begin(), b.fill.end(), b.pFill.p);
   DH_HIP(hipMemcpyAsync(b.f.p, b.pFill.p, n * sizeof(double), hipMemcpyHostToDevice, s));
   DH_HIP(hipMemcpyAsync(b.noccD.p, b.nocc.data(), nmol * sizeof(int), hipMemcpyHostToDevice, s));
-  DH_TRY(launch_batch_density(s, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, b.activeD.p));
+  DH_TRY(launch_batch_density(s, b.be, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, b.activeD.p,
+                              b.work.p));
   DH_TRY(launch_batch_pack(s, b.dblk.pr, b.dblk.norb.p, b.dblk.atomStart.p, b.L, b.P.p,
                            b.rho.p));
   DH_TRY(launch_mulliken_rows(s, b.dblk.rows, b.dblk.norb.p, b.dblk.atomStart.p, b.dblk.start.p,
@@ -3056,15 +3059,16 @@ static int batch_dev_enqueue(BatchContext& b, bool warm) {
   for (int q = 0; q < BatchContext::kSx; ++q) DH_HIP(hipStreamWaitEvent(b.sx[q], b.fork, 0));
   hipStream_t st[kBatchClasses] = {s};
   for (int q = 0; q < BatchContext::kSx; ++q) st[q + 1] = b.sx[q];
-  DH_TRY(launch_batch_sygv(st, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p, b.infoD.p,
-                           b.activeD.p, warm));
+  DH_TRY(launch_batch_sygv(st, b.be, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p, b.infoD.p,
+                           b.activeD.p, warm, b.stage));
   for (int q = 0; q < BatchContext::kSx; ++q) {
     DH_HIP(hipEventRecord(b.join[q], b.sx[q]));
     DH_HIP(hipStreamWaitEvent(s, b.join[q], 0));
   }
   DH_TRY(launch_bscc_info(s, d, b.infoD.p));
   DH_TRY(launch_bscc_fermi(s, d, b.w.p, b.f.p));
-  DH_TRY(launch_batch_density(s, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, b.activeD.p));
+  DH_TRY(launch_batch_density(s, b.be, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, b.activeD.p,
+                              b.work.p));
   DH_TRY(launch_batch_pack(s, b.dblk.pr, b.dblk.norb.p, b.dblk.atomStart.p, b.L, b.P.p,
                            b.rho.p));
   DH_TRY(launch_mulliken_rows(s, b.dblk.rows, b.dblk.norb.p, b.dblk.atomStart.p, b.dblk.start.p,
@@ -3108,12 +3112,10 @@ static int batch_dev_step(BatchContext& b) {
       std::vector<int> info(b.nmol);
       DH_HIP(hipMemcpy(info.data(), b.infoD.p, b.nmol * sizeof(int), hipMemcpyDeviceToHost));
       const int im = (m >= 0 && m < b.nmol) ? info[m] : 0;
-      set_error(im == kBatchJacobiNoConv
-                    ? "batch: Jacobi eigensolver of molecule " + std::to_string(m) +
-                          " did not converge within its sweep limit"
-                : im < 0 ? "batch: molecule " + std::to_string(m) + " of " +
-                               std::to_string(-im) + " orbitals in a smaller size class"
-                         : "batch: overlap of molecule " + std::to_string(m) +
+      set_error(im == kBatchEigenNoConv
+                    ? "batch: eigensolver of molecule " + std::to_string(m) +
+                          " did not converge within its iteration limit"
+                    : "batch: overlap of molecule " + std::to_string(m) +
                                " not positive definite (minor " + std::to_string(im) + ")");
     } else if (c[1] == 2) {
       set_error("batch: Fermi level search did not converge for molecule " + std::to_string(m));
@@ -3215,7 +3217,7 @@ static int batch_gradients(BatchContext& b, double* grad) {
   for (int m = 0; m < b.nmol; ++m)
     for (long k = 0; k < b.nocc[m]; ++k) fe[b.orb0[m] + k] = b.fill[b.orb0[m] + k] * b.eigv[b.orb0[m] + k];
   DH_HIP(hipMemcpyAsync(b.f.p, fe.data(), n * sizeof(double), hipMemcpyHostToDevice, s));
-  DH_TRY(launch_batch_density(s, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, nullptr));
+  DH_TRY(launch_batch_density(s, b.be, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, nullptr, b.work.p));
   DH_TRY(launch_batch_pack(s, b.dblk.pr, b.dblk.norb.p, b.dblk.atomStart.p, b.L, b.P.p, b.erho.p));
   DH_TRY(batch_potential(b, b.dqout, nullptr));
   DH_TRY(fill<double>(s, b.eatom.p, nat, 0.0));
@@ -3255,7 +3257,9 @@ extern "C" int dftbhip_batch_create(dftbhip_batch** bp, const dftbhip_params* p,
       return dftbhip::kErrDevice;
     }
   }
-  if (hipEventCreate(&h->b.fork) != hipSuccess) {
+  bool events = hipEventCreate(&h->b.fork) == hipSuccess;
+  for (hipEvent_t& e : h->b.stage) events = events && hipEventCreate(&e) == hipSuccess;
+  if (!events) {
     delete h;
     dftbhip::set_error("batch_create: event creation failed");
     return dftbhip::kErrDevice;

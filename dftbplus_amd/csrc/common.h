@@ -259,6 +259,19 @@ int sytrd_resident_from(int n, int K, int* c0);
 template <typename T>
 int sytrd_resident(hipStream_t s, T* a, long lda, long sA, int n, int c0, T* d, T* e, T* tau,
                    long sV, unsigned long long* ring, long sRing, int* flag, int K, bool* done);
+// Many small matrices, one workgroup each: matrix of molecule m = list[block] at aMul aOff[m]
+// (n x n, n = vOff[m + 1] - vOff[m], full symmetric or lower), its d, e, tau at vOff[m];
+// molecules with active[m] == 0 (active may be null) and those above the bound are left alone.
+constexpr int kWgBatchMax = 224;
+struct WgBatch {
+  const int* list = nullptr;
+  const int* active = nullptr;
+  const long* aOff = nullptr;
+  long aMul = 1;
+  const long* vOff = nullptr;
+};
+int sytrd_wg_batch(hipStream_t s, double* a, int count, int maxN, const WgBatch& bt, double* d,
+                   double* e, double* tau);
 int set_symv_tiles(int tiles);   // row tiles per SYMV workgroup: 2, 4, 8, 16 or 0 (by size)
 // capture the tridiagonalisation's launch sequence in a HIP graph and replay it for repeated
 // calls on the same buffers (off by default); release_sytrd_graphs frees the kept graphs

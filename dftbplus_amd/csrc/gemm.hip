@@ -405,6 +405,11 @@ template <typename T>
 int gemm_batched(hipStream_t s, bool ta, bool tb, const GemmDesc<T>* dDesc, int nBatch, int maxM,
                  int maxN, T alpha, T beta) {
   if (nBatch <= 0 || maxM <= 0 || maxN <= 0) return 0;
+  constexpr int kDepth = 32768;   // descriptors in the z dimension of a launch
+  if (nBatch > kDepth) {
+    DH_TRY(gemm_batched<T>(s, ta, tb, dDesc, kDepth, maxM, maxN, alpha, beta));
+    return gemm_batched<T>(s, ta, tb, dDesc + kDepth, nBatch - kDepth, maxM, maxN, alpha, beta);
+  }
   const int bt = pick_tile(maxM, maxN, false, nBatch);
   dim3 grid(cdiv(maxM, bt), cdiv(maxN, bt), nBatch);
 #define DH_GEMMB_CASE(TA_, TB_)                                                            \

@@ -16,11 +16,23 @@ using u64 = unsigned long long;
 int stedc_device(hipStream_t s, int n, const double* d, const double* e, double* w, double* z,
                  long ldz, double* work, size_t workSize, StedcWs* ws);
 int stedc_fetch(hipStream_t s, int n, const double* w, double* wHost, StedcWs* ws, int* info);
-// Many tridiagonals at once: problem p's d, e, w at the sum of the sizes before it, its z (n x n,
-// leading dimension n) at the sum of their squares. work: 4 sum n^2 doubles. stedc_info: a failure
-// word per problem (device).
-int stedc_many(hipStream_t s, const std::vector<int>& sizes, const double* d, const double* e,
-               double* w, double* z, double* work, StedcWs* ws);
+// Many tridiagonals at once: block p has n rows, its d, e, w at off, its matrices within the
+// work buffers at q and its z (n x n, leading dimension ldz) at z. prepare makes the tables
+// (copies to the device, not under stream capture) and says how many doubles of work a solve
+// needs; a solve is launches only and leaves the blocks with active[id] == 0 alone (active may be
+// null). stedc_info: a failure word per block (device; 0 solved, -1 left alone).
+struct DcBlock {
+  int n;
+  long off, q, z, ldz;
+  int id;
+  bool operator==(const DcBlock& o) const {
+    return n == o.n && off == o.off && q == o.q && z == o.z && ldz == o.ldz && id == o.id;
+  }
+};
+int stedc_many_prepare(hipStream_t s, const std::vector<DcBlock>& blocks, StedcWs* ws,
+                       size_t* workSize);
+int stedc_many(hipStream_t s, const double* d, const double* e, double* w, double* z,
+               double* work, const int* active, StedcWs* ws);
 const int* stedc_info(const StedcWs* ws);
 
 }  // namespace dftbhip

@@ -57,15 +57,14 @@ struct MergeDev {
 
 struct ProblemDev {
   int s, n, parity;   // parity: which of the two Q buffers holds the eigenvectors
-  int pad;
+  int id;
   long q, z, ldz;     // offsets in Q and in the output
 };
 
 // Device buffers and the size-dependent tables of a solve, kept by the caller between calls:
 // they only grow, so repeated solves of one size allocate and copy nothing.
 struct StedcWs {
-  std::vector<int> sizes;                 // the sizes the tables are for
-  std::vector<long> zoff, ldz;
+  std::vector<DcBlock> blocks;            // what the tables are for
   std::vector<LeafDev> leaves;
   std::vector<MergeDev> merges;           // by height
   std::vector<ProblemDev> problems;
@@ -125,6 +124,7 @@ __global__ __launch_bounds__(64) void leaf_kernel(const double* dIn, const doubl
   __shared__ double d[kLeaf + 1], e[kLeaf + 1];
   const LeafDev L = leaves[blockIdx.x];
   const int m = L.m, t = threadIdx.x;
+  if (A.info[L.prob] < 0) return;
   if (t < m) {
     double v = dIn[L.s + t];
     // the tears on both sides of the leaf
@@ -682,10 +682,13 @@ __global__ void collect_kernel(const ProblemDev* pr, const double* Qa, const dou
   for (int r = lane; r < p.n; r += 64) dst[r] = src[r];
 }
 
-__global__ void stedc_zero_kernel(double* q, size_t n, int* info, int ninfo) {
+// zeros, and the state of each problem: to be solved, or (-1) left as it is
+__global__ void stedc_zero_kernel(double* q, size_t n, const ProblemDev* pr, const int* active,
+                                  int* info, int ninfo) {
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (size_t k = i; k < (size_t)ninfo; k += stride) info[k] = 0;
+  for (size_t k = i; k < (size_t)ninfo; k += stride)
+    info[k] = active && !active[pr[k].id] ? -1 : 0;
   for (; i < n; i += stride) q[i] = 0.0;
 }
 
@@ -708,43 +711,44 @@ void build_tree(int s, int n, int height, std::vector<Node>& merges,
 }
 }  // namespace
 
-static int dc_tables(hipStream_t s, StedcWs& W, const std::vector<int>& sizes,
-                     const std::vector<long>& zoff, const std::vector<long>& ldz) {
-  if (W.sizes == sizes && W.zoff == zoff && W.ldz == ldz) return 0;
-  W.sizes.clear();
+static int dc_tables(hipStream_t s, StedcWs& W, const std::vector<DcBlock>& blocks) {
+  if (W.blocks == blocks) return 0;
+  W.blocks.clear();
   W.leaves.clear();
   W.merges.clear();
   W.problems.clear();
   W.maxProblem = 0;
-  long off = 0, q = 0;
+  long off = 0, q = 0;   // ends of the arrays and of Q
   std::vector<std::vector<MergeDev>> byHeight;
-  for (size_t p = 0; p < sizes.size(); ++p) {
-    const int n = sizes[p];
+  for (size_t p = 0; p < blocks.size(); ++p) {
+    const DcBlock& bl = blocks[p];
+    const int n = bl.n;
+    DH_CHECK(n > 0 && n < (1 << 21), "stedc: problem size");   // packed counts of the deflation
     int h = 0;
     while (((n + (1 << h) - 1) >> h) > kLeaf) ++h;
     std::vector<Node> nodes;
     std::vector<std::pair<int, int>> lv;
     build_tree(0, n, h, nodes, lv);
     for (const auto& l : lv)
-      W.leaves.push_back({(int)off + l.first, l.second, l.first, n, (int)p, 0,
-                          q + l.first + (long)l.first * n, n});
+      W.leaves.push_back({(int)bl.off + l.first, l.second, l.first, n, (int)p, 0,
+                          bl.q + l.first + (long)l.first * n, n});
     if ((int)byHeight.size() < h + 1) byHeight.resize(h + 1);
     for (const Node& x : nodes) {
       MergeDev m{};
-      m.s = (int)off + x.s;
+      m.s = (int)bl.off + x.s;
       m.n1 = x.n1;
       m.n2 = x.n2;
       m.prob = (int)p;
-      m.q = q + x.s + (long)x.s * n;
+      m.q = bl.q + x.s + (long)x.s * n;
       m.ld = n;
       byHeight[x.height].push_back(m);
     }
-    W.problems.push_back({(int)off, n, h & 1, 0, q, zoff[p], ldz[p]});
+    W.problems.push_back({(int)bl.off, n, h & 1, bl.id, bl.q, bl.z, bl.ldz});
     W.maxProblem = std::max(W.maxProblem, n);
-    off += n;
-    q += (long)n * n;
+    off = std::max(off, bl.off + n);
+    q = std::max(q, bl.q + (long)n * n);
   }
-  DH_CHECK(off < (1L << 21), "stedc: too many rows");   // packed counts of the deflation
+  DH_CHECK(off < (1L << 31), "stedc: too many rows");
   W.total = off;
   W.totalSq = q;
   W.first.assign(1, 0);
@@ -769,17 +773,16 @@ static int dc_tables(hipStream_t s, StedcWs& W, const std::vector<int>& sizes,
   DH_TRY(W.dproblem.upload(W.problems.data(), W.problems.size(), s));
   DH_TRY(W.ddesc.alloc(std::max<size_t>(2 * W.merges.size(), 1)));
   DH_TRY(W.darr.alloc((size_t)kDcDoubles * W.total));
-  DH_TRY(W.iarr.alloc((size_t)kDcInts * W.total + sizes.size()));
+  DH_TRY(W.iarr.alloc((size_t)kDcInts * W.total + blocks.size()));
   W.info = W.iarr.p + (size_t)kDcInts * W.total;
-  W.sizes = sizes;
-  W.zoff = zoff;
-  W.ldz = ldz;
+  W.blocks = blocks;
   return 0;
 }
 
 // The launches of a solve on the tables in W. work: 4 totalSq doubles.
 static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e, double* w,
-                     double* z, double* work) {
+                     double* z, double* work, const int* active) {
+  constexpr int kRows = 32768;   // merges or problems in the y dimension of a launch
   DcArrays A;
   {
     double** dp[kDcDoubles] = {&A.D, &A.z, &A.DL, &A.W, &A.tau, &A.lam, &A.zhat, &A.dval,
@@ -797,37 +800,43 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
   // zeros outside the blocks of the leaves; the second buffer's blocks are written whole, its
   // zeros outside them are read by the next height
   hipLaunchKernelGGL(stedc_zero_kernel, dim3((unsigned)std::min<size_t>(cdiv(2 * sq, 1024), 2048)),
-                     dim3(256), 0, s, work, 2 * sq, W.info, (int)W.problems.size());
+                     dim3(256), 0, s, work, 2 * sq, W.dproblem.p, active, W.info, (int)W.problems.size());
   DH_LAUNCH_CHECK();
   hipLaunchKernelGGL(leaf_kernel, dim3((unsigned)W.leaves.size()), dim3(64), 0, s, d, e, W.dleaf.p,
                      Q[0], A);
   DH_LAUNCH_CHECK();
   for (size_t h = 1; h + 1 < W.first.size(); ++h) {
-    const int f = W.first[h], nm = W.first[h + 1] - f;
-    if (nm == 0) continue;
     const int mx = W.maxn[h];
-    MergeDev* md = W.dmerge.p + f;
-    GemmDesc<double>* gd = W.ddesc.p + 2 * (size_t)f;
     double* Qo = Q[(h - 1) & 1];
     double* Qn = Q[h & 1];
-    hipLaunchKernelGGL(deflate_kernel, dim3(nm), dim3(kDefT), 0, s, md, e, Qo, Qn, Qg, U, gd, A);
-    DH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(rotate_kernel, dim3(cdiv(mx, 64), nm), dim3(64), 0, s, md, Qo, A);
-    DH_LAUNCH_CHECK();
-    const dim3 gg(cdiv((long)mx * kSecG, 64), nm), gw(cdiv((long)mx * 64, 256), nm);
-    hipLaunchKernelGGL(secular_kernel, gg, dim3(64), 0, s, md, A);
-    DH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(zhat_kernel, gg, dim3(64), 0, s, md, A);
-    DH_LAUNCH_CHECK();
-    hipLaunchKernelGGL(buildu_kernel, gw, dim3(256), 0, s, md, Qo, U, Qg, A);
-    DH_LAUNCH_CHECK();
-    DH_TRY(gemm_batched<double>(s, false, false, gd, 2 * nm, (mx + 1) / 2, mx, 1.0, 0.0));
-    hipLaunchKernelGGL(finish_kernel, gw, dim3(256), 0, s, md, Qo, Qn, A);
+    for (int f = W.first[h]; f < W.first[h + 1]; f += kRows) {
+      const int nm = std::min(kRows, W.first[h + 1] - f);
+      MergeDev* md = W.dmerge.p + f;
+      GemmDesc<double>* gd = W.ddesc.p + 2 * (size_t)f;
+      hipLaunchKernelGGL(deflate_kernel, dim3(nm), dim3(kDefT), 0, s, md, e, Qo, Qn, Qg, U, gd, A);
+      DH_LAUNCH_CHECK();
+      hipLaunchKernelGGL(rotate_kernel, dim3(cdiv(mx, 64), nm), dim3(64), 0, s, md, Qo, A);
+      DH_LAUNCH_CHECK();
+      const dim3 gg(cdiv((long)mx * kSecG, 64), nm), gw(cdiv((long)mx * 64, 256), nm);
+      hipLaunchKernelGGL(secular_kernel, gg, dim3(64), 0, s, md, A);
+      DH_LAUNCH_CHECK();
+      hipLaunchKernelGGL(zhat_kernel, gg, dim3(64), 0, s, md, A);
+      DH_LAUNCH_CHECK();
+      hipLaunchKernelGGL(buildu_kernel, gw, dim3(256), 0, s, md, Qo, U, Qg, A);
+      DH_LAUNCH_CHECK();
+      DH_TRY(gemm_batched<double>(s, false, false, gd, 2 * nm, (mx + 1) / 2, mx, 1.0, 0.0));
+      hipLaunchKernelGGL(finish_kernel, gw, dim3(256), 0, s, md, Qo, Qn, A);
+      DH_LAUNCH_CHECK();
+    }
+  }
+  for (size_t p = 0; p < W.problems.size(); p += kRows) {
+    DcArrays Ap = A;
+    Ap.info += p;
+    hipLaunchKernelGGL(collect_kernel, dim3(cdiv((long)W.maxProblem * 64, 256),
+                                            (unsigned)std::min<size_t>(kRows, W.problems.size() - p)),
+                       dim3(256), 0, s, W.dproblem.p + p, Q[0], Q[1], w, z, Ap);
     DH_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(collect_kernel, dim3(cdiv((long)W.maxProblem * 64, 256), (unsigned)W.problems.size()),
-                     dim3(256), 0, s, W.dproblem.p, Q[0], Q[1], w, z, A);
-  DH_LAUNCH_CHECK();
   return 0;
 }
 
@@ -840,21 +849,20 @@ int stedc_device(hipStream_t s, int n, const double* d, const double* e, double*
                  long ldz, double* work, size_t workSize, StedcWs* ws) {
   DH_CHECK(n > 0 && ws, "stedc: bad arguments");
   DH_CHECK(workSize >= stedc_work_size(n), "stedc: workspace too small");
-  DH_TRY(dc_tables(s, *ws, {n}, {0}, {ldz}));
-  return dc_launch(s, *ws, d, e, w, z, work);
+  DH_TRY(dc_tables(s, *ws, {DcBlock{n, 0, 0, 0, ldz, 0}}));
+  return dc_launch(s, *ws, d, e, w, z, work, nullptr);
 }
 
-int stedc_many(hipStream_t s, const std::vector<int>& sizes, const double* d, const double* e,
-               double* w, double* z, double* work, StedcWs* ws) {
-  std::vector<long> zoff, ldz;
-  long q = 0;
-  for (int n : sizes) {
-    zoff.push_back(q);
-    ldz.push_back(n);
-    q += (long)n * n;
-  }
-  DH_TRY(dc_tables(s, *ws, sizes, zoff, ldz));
-  return dc_launch(s, *ws, d, e, w, z, work);
+int stedc_many_prepare(hipStream_t s, const std::vector<DcBlock>& blocks, StedcWs* ws,
+                       size_t* workSize) {
+  DH_TRY(dc_tables(s, *ws, blocks));
+  *workSize = 4 * (size_t)ws->totalSq;
+  return 0;
+}
+
+int stedc_many(hipStream_t s, const double* d, const double* e, double* w, double* z,
+               double* work, const int* active, StedcWs* ws) {
+  return ws->blocks.empty() ? 0 : dc_launch(s, *ws, d, e, w, z, work, active);
 }
 
 const int* stedc_info(const StedcWs* ws) { return ws->info; }

@@ -20,51 +20,13 @@
 #include <cstring>
 
 #include "common.h"
+#include "lanes.h"
 
 namespace dftbhip {
 
 using u64 = unsigned long long;
 
 namespace {
-
-__device__ __forceinline__ double hilo(unsigned lo, unsigned hi) {
-  return __hiloint2double((int)hi, (int)lo);
-}
-
-// sum over the 64 lanes, the same bits in every lane (each step adds a pair both ways round)
-template <int Ctrl>
-__device__ __forceinline__ double dpp(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), Ctrl, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), Ctrl, 0xf, 0xf, false);
-  return __hiloint2double(hi, lo);
-}
-constexpr int kRor8 = 0x128, kRor4 = 0x124, kRor2 = 0x122, kRor1 = 0x121;
-constexpr int kHalfMirror = 0x141, kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;
-
-// rows (16 lanes) r of a and b: even rows a_r + a_(r+1), odd rows b_(r-1) + b_r
-__device__ __forceinline__ double swap16_add(double a, double b) {
-  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a),
-                                                  (unsigned)__double2loint(b), false, false);
-  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a),
-                                                  (unsigned)__double2hiint(b), false, false);
-  return hilo(l[0], h[0]) + hilo(l[1], h[1]);
-}
-// lanes < 32: a_l + a_(l+32); lanes >= 32: b_(l-32) + b_l
-__device__ __forceinline__ double swap32_add(double a, double b) {
-  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a),
-                                                  (unsigned)__double2loint(b), false, false);
-  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a),
-                                                  (unsigned)__double2hiint(b), false, false);
-  return hilo(l[0], h[0]) + hilo(l[1], h[1]);
-}
-__device__ __forceinline__ double wave_total(double v) {
-  v += dpp<kRor8>(v);
-  v += dpp<kRor4>(v);
-  v += dpp<kRor2>(v);
-  v += dpp<kRor1>(v);
-  v = swap16_add(v, v);
-  return swap32_add(v, v);
-}
 
 // Sums of four values per lane over the 64 lanes: lane l returns the total of acc[(l >> 2) & 3].
 // Each halving exchanges the pair of values a lane does not keep: three exchanges and four plain
@@ -94,10 +56,6 @@ __device__ __forceinline__ double part_total(double v) {
   return v + dpp<kRor1>(v);
 }
 
-__device__ __forceinline__ double lane_value(double v, int lane) {
-  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                          __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
 // element idx of the vector whose element l + 64 q is x[q] of lane l
 template <int C>
 __device__ __forceinline__ double element(const double (&x)[C], int idx) {
@@ -202,19 +160,43 @@ __device__ __forceinline__ double octet_total(const double (&acc)[S], int lc) {
   return v + dpp<kQuadXor1>(v);
 }
 
+// row sums of all S rows of a lane group into y, four at a time
+template <int S, int S0, int NW>
+__device__ __forceinline__ void octet_store(const double (&acc)[S], int lc, int row0, double* y) {
+  constexpr int N = S - S0 < 4 ? S - S0 : 4;
+  double part[N];
+#pragma unroll
+  for (int s = 0; s < N; ++s) part[s] = acc[S0 + s];
+  const double v = octet_total<N>(part, lc);
+  constexpr int sh = N > 2 ? 1 : 2;
+  if ((lc & ((1 << sh) - 1)) == 0 && (lc >> sh) < N) y[row0 + 8 * NW * (S0 + (lc >> sh))] = v;
+  if constexpr (S0 + 4 < S) octet_store<S, S0 + 4, NW>(acc, lc, row0, y);
+}
+
 template <typename T, int NW, int S, int Q>
 __global__ __launch_bounds__(64 * NW) void sytrd_wg_kernel(T* a, long lda, long sA, int n, int c0,
-                                                           T* d, T* e, T* tauOut, long sV) {
+                                                           T* d, T* e, T* tauOut, long sV,
+                                                           WgBatch bt) {
   constexpr int C = (Q + 7) / 8;        // elements per lane of a vector over the wave
   constexpr int QP = Q + 2;             // padded: the eight lanes of a read meet distinct banks
   constexpr int NV = 8 * QP, QG = 4;
-  static_assert(Q % QG == 0 && S <= 4, "sytrd_wg: shape");
+  static_assert(Q % QG == 0, "sytrd_wg: shape");
   __shared__ double sVec[NW][3][NV];    // v of even and odd columns, w
   __shared__ double sY[2][8 * NW * S], sX[2][NV];
-  a += blockIdx.x * sA + c0 + (long)c0 * lda;
-  d += blockIdx.x * sV + c0;
-  e += blockIdx.x * sV + c0;
-  tauOut += blockIdx.x * sV + c0;
+  long offA = blockIdx.x * sA, offV = blockIdx.x * sV;
+  if (bt.list) {
+    const int mol = bt.list[blockIdx.x];
+    if (bt.active && !bt.active[mol]) return;
+    offA = bt.aMul * bt.aOff[mol];
+    offV = bt.vOff[mol];
+    n = (int)(bt.vOff[mol + 1] - offV);
+    lda = n;
+    if (n > 8 * NW * S || n > 8 * Q) return;   // a size the shape does not hold: left alone
+  }
+  a += offA + c0 + (long)c0 * lda;
+  d += offV + c0;
+  e += offV + c0;
+  tauOut += offV + c0;
   const int m = n - c0;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int lr = lane >> 3, lc = lane & 7;
@@ -292,12 +274,7 @@ __global__ __launch_bounds__(64 * NW) void sytrd_wg_kernel(T* a, long lda, long 
 #pragma unroll
         for (int q = 0; q < Q; ++q) sX[par][lc * QP + q] = A[s][q];
       }
-    const double yr = octet_total<S>(acc, lc);
-    if constexpr (S > 2) {
-      if ((lc & 1) == 0 && (lc >> 1) < S) sY[par][row0 + 8 * NW * (lc >> 1)] = yr;
-    } else {
-      if ((lc & 3) == 0 && (lc >> 2) < S) sY[par][row0 + 8 * NW * (lc >> 2)] = yr;
-    }
+    octet_store<S, 0, NW>(acc, lc, row0, sY[par]);
     lds_barrier();
     double y[C], an[C];
     double dt = 0.0;
@@ -629,7 +606,7 @@ static int wg_launch(hipStream_t s, T* a, long lda, long sA, int n, int c0, T* d
   const int m = n - c0;
 #define DH_WG(NW_, S_, Q_)                                                                     \
   hipLaunchKernelGGL((sytrd_wg_kernel<T, NW_, S_, Q_>), dim3(K), dim3(64 * NW_), 0, s, a, lda, sA, \
-                     n, c0, d, e, tau, sV)
+                     n, c0, d, e, tau, sV, WgBatch{})
   if (m <= 32) DH_WG(4, 1, 4);
   else if (m <= 64) DH_WG(4, 2, 8);
   else DH_WG(4, 4, 16);
@@ -661,6 +638,25 @@ static const GridShape* grid_shape(int m, int maxP) {
   for (const GridShape& g : shapes)
     if (m <= g.nt * g.c && (m + g.r - 1) / g.r <= maxP) return &g;
   return nullptr;
+}
+
+int sytrd_wg_batch(hipStream_t s, double* a, int count, int maxN, const WgBatch& bt, double* d,
+                   double* e, double* tau) {
+  if (count <= 0) return 0;
+  DH_CHECK(bt.list && bt.aOff && bt.vOff && maxN <= kWgBatchMax, "sytrd_wg_batch: bad arguments");
+  // 192 columns fit eight waves without spills (379 us for 190); 224 columns leave too few
+  // registers either way, and four waves spill least (680 us for 190)
+#define DH_WGB(NW_, S_, Q_)                                                                    \
+  hipLaunchKernelGGL((sytrd_wg_kernel<double, NW_, S_, Q_>), dim3(count), dim3(64 * NW_), 0, s, \
+                     a, 0L, 0L, 0, 0, d, e, tau, 0L, bt)
+  if (maxN <= 32) DH_WGB(4, 1, 4);
+  else if (maxN <= 64) DH_WGB(4, 2, 8);
+  else if (maxN <= 128) DH_WGB(4, 4, 16);
+  else if (maxN <= 192) DH_WGB(8, 3, 24);
+  else DH_WGB(4, 7, 28);
+#undef DH_WGB
+  DH_LAUNCH_CHECK();
+  return 0;
 }
 
 static int cu_count(int* out) {
