@@ -28,11 +28,11 @@ struct DevNeighbourList {
   DevBuf<int> bAt1, bImg2, bAt2;     // pairs within the SK cutoff
   DevBuf<long> bStart;               // their block offsets in the sparse arrays
   // work arrays
-  DevBuf<double> px, fD2;
-  DevBuf<int> pbin, binCount, binStart, binFill, binItems, cnt, fPi, used, imgRank, flag, err;
-  DevBuf<long> fStart, size, bOff, scal;
+  DevBuf<double> px, binX, fD2;
+  DevBuf<int> pbin, binCount, binStart, prank, binItems, cnt, fPi, used, imgRank, err;
+  DevBuf<long> fStart, sums, scal;
   DevBuf<double> coordsD, trD;
-  DevBuf<int> norbD, bIdx, iscal;
+  DevBuf<int> norbD;
 };
 
 // Builds the list for nat atoms at coords (host, 3 nat) with lattice lat (host, 9 doubles, or
