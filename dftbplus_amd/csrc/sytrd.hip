@@ -7,10 +7,10 @@
 //                        w = tau * (A22 v - V (W^T v) - W (V^T v)),  w += -tau/2 (w.v) v;
 //     trailing update A22 -= [V W] [W V]^T on the MFMA GEMM (lower tiles).
 //
-// The symmetric product A22 v reads only the lower triangle: each workgroup owns a 64-row block
-// and a chunk of <= 8 column blocks; row-block partial sums and transposed-tile partial sums go
-// to workspaces that the next kernel reduces (no atomics on the vector). This product is the
-// HBM-bound part of the eigensolver (it streams the trailing matrix once per column).
+// The symmetric product A22 v reads only the lower triangle: each workgroup takes an equal run of
+// its 64 x 64 tiles; row-block partial sums and transposed-tile partial sums go to workspaces that
+// the next kernel reduces (no atomics on the vector). This product is the HBM-bound part of the
+// eigensolver (it streams the trailing matrix once per column).
 #include <algorithm>
 #include <mutex>
 #include <type_traits>
@@ -70,10 +70,11 @@ static int symv_prof_collect(hipStream_t s) {
   return 0;
 }
 constexpr int kTB = 64;      // SYMV tile
-constexpr int kSymvTiles8From = 7000;   // trailing sizes from which 8 tiles per workgroup
-constexpr int kSymvTiles4From = 2500;   // ... and from which 4
-constexpr int kCHMin = 2;    // fewest row tiles per SYMV workgroup (sizes the slot array)
-// row tiles per SYMV workgroup (2, 4, 8 or 16; 0: chosen from the trailing size), set through
+constexpr int kCHMin = 2;    // fewest tiles per SYMV workgroup (sizes the slot array)
+// SYMV workgroups that are resident together (two on each of 256 compute units): the tiles of
+// all problems are shared out to as many, so that there is one round and no last, half empty one
+constexpr int kSymvSlots = 512;
+// tiles per SYMV workgroup (2, 4, 8 or 16; 0: the tiles shared out evenly), set through
 // set_symv_tiles
 static int g_symvTiles = 0;
 // bumped whenever the tile choice changes: captured launch sequences (below) are only replayed
@@ -89,8 +90,8 @@ int set_symv_tiles(int tiles) {
 }
 
 // Tile choice by trailing size from the autotuner (symv_autotune), per arithmetic type
-// ([0] FP64, [1] FP32): rows (first trailing size, tiles) in ascending size; empty: the fixed
-// thresholds above.
+// ([0] FP64, [1] FP32): rows (first trailing size, tiles) in ascending size; empty: shared out
+// evenly.
 static std::vector<std::pair<int, int>> g_tileTable[2];
 
 int clear_symv_tables() {
@@ -100,19 +101,29 @@ int clear_symv_tables() {
   return 0;
 }
 
-// Long tile chains keep more loads in flight per workgroup on a large trailing matrix; a small
-// one has too few column blocks to fill the chip, and short chains there give more workgroups.
+// Tiles per SYMV workgroup for K problems of trailing size m
 template <typename T>
-static int symv_tiles(int m) {
+static int symv_tiles(int m, int K) {
   if (g_symvTiles != 0) return g_symvTiles;
   const auto& t = g_tileTable[std::is_same<T, float>::value ? 1 : 0];
   if (!t.empty()) {
+    const int mk = (int)std::min<long>((long)m * K, 1L << 30);
     int v = t.front().second;
     for (const auto& r : t)
-      if (m >= r.first) v = r.second;
+      if (mk >= r.first) v = r.second;
     return v;
   }
-  return m >= kSymvTiles8From ? 8 : (m >= kSymvTiles4From ? 4 : 2);
+  const long nRB = (m + kTB - 1) / kTB, all = nRB * (nRB + 1) / 2 * K;
+  return (int)std::max<long>(kCHMin, (all + kSymvSlots - 1) / kSymvSlots);
+}
+
+// The lower tiles of nRB row blocks in the order of their columns: column J's start at
+// symv_first(J); a workgroup takes q tiles in a row, so column J is worked out in
+// symv_pieces(J) pieces.
+__host__ __device__ inline int symv_first(int nRB, int J) { return J * nRB - J * (J - 1) / 2; }
+__device__ inline int symv_pieces(int nRB, int J, int q) {
+  const int t = symv_first(nRB, J);
+  return (t + nRB - J - 1) / q - t / q + 1;
 }
 
 template <typename T>
@@ -131,7 +142,7 @@ struct SytrdWs {
 
 static int sytrd_slots(int n) {
   const int nRB = (n + kTB - 1) / kTB;
-  return nRB + (nRB + kCHMin - 1) / kCHMin;
+  return nRB + nRB / kCHMin + 2;
 }
 
 // byte layout of the workspace (each array 256-byte aligned)
@@ -271,19 +282,44 @@ __global__ __launch_bounds__(256) void col_update_kernel(T* a, long lda, int n, 
   }
 }
 
+// Sum of each z[0..15] over the wave, in 17 exchanges instead of 96: every step adds the halves of
+// the array that two lanes exchange. Lane l returns the sum of z[l & 15].
+template <int H, typename T>
+__device__ __forceinline__ void fold_halves(T (&z)[16], int lane) {
+  const bool up = lane & H;
+#pragma unroll
+  for (int e = 0; e < H; ++e) {
+    const T send = up ? z[e] : z[e + H], keep = up ? z[e + H] : z[e];
+    z[e] = keep + __shfl_xor(send, H, 64);
+  }
+}
+template <typename T>
+__device__ __forceinline__ T wave_sum16(T (&z)[16], int lane) {
+  fold_halves<8>(z, lane);
+  fold_halves<4>(z, lane);
+  fold_halves<2>(z, lane);
+  fold_halves<1>(z, lane);
+  T v = z[0];
+  v += __shfl_xor(v, 16, 64);
+  return v + __shfl_xor(v, 32, 64);
+}
+
 // Partial sums of y = A22 v (A22 = a(c+1:n, c+1:n), lower triangle read once).
-// Workgroup (J, chunk) owns column block J and row blocks J + chunk*CH ... (CH of them):
-//   y partial of row block I  -> Y(row, J)            (one per tile, reduced over 4 waves)
-//   transposed sums (A^T v)_J -> Y(col, nRB + chunk)  (accumulated in registers over the tiles)
+// The first nRB workgroups take a row block each: they publish v and add up the panel products
+// t1, t2. Workgroup nRB + w takes the tiles w q .. w q + q - 1 of the lower triangle, column by
+// column, the next two tiles on the way while one is worked on; the first two are requested
+// before the reflector of the column is formed.
+//   y partial of tile (I, J)       -> Y(row, J)          (reduced over 4 waves)
+//   transposed sums (A^T v)_J      -> Y(col, nRB + piece) (in registers over the column's tiles)
 // Thread (ii = tid % 64, cg = tid / 64) holds rows ii of 16 columns cg*16 .. cg*16+15.
-// The chunk-0 workgroup of each column block publishes v and the panel products t1, t2.
-template <typename T, int CH>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void symv_kernel(const T* a, long lda, int n, int c, int j0,
-                                                   const T* W, long ldw, const double* nrm2,
-                                                   const T* tauA, const double* dotA, T* Y,
-                                                   int nSlot, T* vbuf, double* t12,
-                                                   double* scalOut, T* eOut, T* tauOut,
-                                                   ProblemStrides ps) {
+// Bound by the stream of the trailing triangle: 22 us on average over trailing sizes 2560 to 6656
+// (4.1 TB/s), 29 us with fixed chunks of a column per workgroup, whose last round was partly
+// empty, and the panel products ahead of the first tile of some of them.
+template <typename T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void symv_kernel(
+    const T* a, long lda, int n, int c, int j0, const T* W, long ldw, const double* nrm2,
+    const T* tauA, const double* dotA, T* Y, T* vbuf, double* t12, double* scalOut, T* eOut,
+    T* tauOut, int q, ProblemStrides ps) {
   __shared__ T vJs[kTB];
   __shared__ T red[4][4][kTB];
   a += (long)blockIdx.z * ps.a;
@@ -299,77 +335,84 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   scalOut = ws_of(scalOut, ps.ws);
   const int m = n - c - 1;
   const int nRB = (m + kTB - 1) / kTB;
-  const int J = blockIdx.x, ch = blockIdx.y;
-  const int Ib = J + ch * CH;
-  if (J >= nRB || Ib >= nRB) return;
-  const int Ie = min(Ib + CH, nRB);
   const int tid = threadIdx.x;
-  const int ii = tid & 63, cg = tid >> 6;
-  const double alpha = a[(c + 1) + (long)c * lda];
+  const int ii = tid & 63, cg = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const T* const col = a + (c + 1) + (long)c * lda;   // the column's elements below the diagonal
+  const double alpha = col[0], xn2 = nrm2[c];
   double beta, tau, scal;
-  reflector(alpha, nrm2[c], beta, tau, scal);
-  if (J == 0 && ch == 0 && tid == 0) {
-    scalOut[c] = scal;
-    eOut[c] = (T)beta;
-    tauOut[c] = (T)tau;
-  }
-  auto vval = [&](int k) -> T {
-    if (k >= m) return T(0);
-    return (k == 0) ? T(1) : (T)((double)a[(c + 1 + k) + (long)c * lda] * scal);
-  };
-  if (tid < kTB) vJs[tid] = vval(J * kTB + tid);
-  __syncthreads();
-  const int cols0 = c + 1 + J * kTB;
-  if (ch == 0) {
-    if (tid < kTB && J * kTB + tid < m) vbuf[cols0 + tid] = vJs[tid];
+  if ((int)blockIdx.x < nRB) {
+    reflector(alpha, xn2, beta, tau, scal);
+    if (blockIdx.x == 0 && tid == 0) {
+      scalOut[c] = scal;
+      eOut[c] = (T)beta;
+      tauOut[c] = (T)tau;
+    }
+    const int k = blockIdx.x * kTB + ii, r = c + 1 + k;
+    const bool rowOk = k < m;
+    const T v = !rowOk ? T(0) : (k == 0 ? T(1) : (T)((double)col[k] * scal));
+    if (cg == 0 && rowOk) vbuf[r] = v;
     // panel products over this block's rows: t12[p] += W(:, p)^T v, t12[i + p] += V(:, p)^T v
-    // for p < i (wave cg takes p = cg + 4q). All loads are issued before the reductions and
+    // for p < i (wave cg takes p = cg + 4 e). All loads are issued before the reductions and
     // atomics, which would otherwise order every load behind the previous atomic.
     const int i = c - j0;
-    const bool rowOk = J * kTB + ii < m;
-    const int r = cols0 + ii;
-    const double vv = (double)vJs[ii];
+    const double vv = (double)v;
     double pw[kNB / 4], pv[kNB / 4];
+    static_assert(kNB / 4 == 16, "wave_sum16");
 #pragma unroll
-    for (int q = 0; q < kNB / 4; ++q) {
-      const int p = cg + 4 * q;
-      pw[q] = 0.0;
-      pv[q] = 0.0;
+    for (int e = 0; e < kNB / 4; ++e) {
+      const int p = cg + 4 * e;
+      pw[e] = 0.0;
+      pv[e] = 0.0;
       if (p < i && rowOk) {
         const double vr = a[r + (long)(j0 + p) * lda];
-        pv[q] = vr * vv;
-        pw[q] = ((double)W[r + (long)p * ldw] + wcorr(j0 + p, tauA, dotA) * vr) * vv;
+        pv[e] = vr * vv;
+        pw[e] = ((double)W[r + (long)p * ldw] + wcorr(j0 + p, tauA, dotA) * vr) * vv;
       }
     }
-#pragma unroll
-    for (int q = 0; q < kNB / 4; ++q) {
-      const int p = cg + 4 * q;
-      if (p < i) {
-        const double sw = wave_sum(pw[q]), sv = wave_sum(pv[q]);
-        if (ii == 0 && sw != 0.0) atomicAdd(&t12[t12_at(c, p)], sw);
-        if (ii == 0 && sv != 0.0) atomicAdd(&t12[t12_at(c, i + p)], sv);
-      }
+    const double sw = wave_sum16(pw, ii), sv = wave_sum16(pv, ii);
+    const int p = cg + 4 * (ii & 15);
+    if (ii < 16 && p < i) {
+      if (sw != 0.0) atomicAdd(&t12[t12_at(c, p)], sw);
+      if (sv != 0.0) atomicAdd(&t12[t12_at(c, i + p)], sv);
     }
+    return;
   }
-  const T* vj = vJs + cg * 16;   // v of this thread's 16 columns (LDS broadcast reads)
+  const int w = blockIdx.x - nRB;
+  const int t0 = w * q, t1 = min(t0 + q, nRB * (nRB + 1) / 2);
+  if (t0 >= t1) return;
+  // column of the first tile
+  int J = (int)(0.5 * (2 * nRB + 1 - sqrt((double)(2 * nRB + 1) * (2 * nRB + 1) - 8.0 * t0)));
+  J = min(max(J, 0), nRB - 1);
+  while (symv_first(nRB, J) > t0) --J;
+  while (J + 1 < nRB && symv_first(nRB, J + 1) <= t0) ++J;
+  int I = J + t0 - symv_first(nRB, J);
+  int lI = I, lJ = J, left = t1 - t0;   // next tile to request
   T b0[16], b1[16], b2[16], zacc[16];
-  T v0 = T(0), v1 = T(0), v2 = T(0);
+  T v0 = T(0), v1 = T(0), v2 = T(0), u0 = T(0), u1 = T(0), u2 = T(0);
 #pragma unroll
   for (int e = 0; e < 16; ++e) zacc[e] = T(0);
-  // tile I rows ii of this thread's 16 columns, and v of row ii (prefetched with the tile)
-  auto load = [&](int I, T* dst, T& vdst) {
-    const int gr = I * kTB + ii;
-    const bool rowOk = gr < m;
-    const T* src = a + (c + 1 + gr) + (long)cols0 * lda;
+  // rows ii of the tile's 16 columns, v of row ii and of column ii & 15 (raw column-c elements,
+  // scaled at use so that the request is not waited on). Rows and columns past the end and the
+  // upper triangle of a diagonal tile are read at the nearest place that exists and masked at
+  // their use.
+  auto load = [&](T(&dst)[16], T& vdst, T& udst) __attribute__((always_inline)) {
+    const int gr = min(lI * kTB + ii, m - 1), gc0 = lJ * kTB + cg * 16;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int jj = cg * 16 + e;
-      const int gc = J * kTB + jj;
-      dst[e] = (rowOk && gc < m && (I > J || ii >= jj)) ? src[(long)jj * lda] : T(0);
+    for (int e = 0; e < 16; ++e) dst[e] = (col + (long)(1 + min(gc0 + e, m - 1)) * lda)[gr];
+    vdst = col[gr];
+    udst = col[min(gc0 + (ii & 15), m - 1)];
+    // past the run's last tile the requests repeat it (in the caches) instead of branching
+    if (--left > 0) {
+      const bool next = lI + 1 == nRB;
+      lJ += next;
+      lI = next ? lJ : lI + 1;
     }
-    // raw column-c element of the row; scaled at use so that the prefetch is not waited on
-    vdst = (rowOk && gr > 0) ? a[(c + 1 + gr) + (long)c * lda] : T(0);
   };
+  load(b0, v0, u0);
+  load(b1, v1, u1);
+  reflector(alpha, xn2, beta, tau, scal);
+  T* vj = vJs + cg * 16;   // v of this wave's 16 columns
+  bool fresh = true;       // the next tile is the first of its column here
   // barrier for the LDS row sums only: __syncthreads would also wait for the prefetched global
   // loads of the next tiles (its workgroup fence waits on every outstanding memory operation)
   auto lds_barrier = [&]() {
@@ -378,10 +421,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     __builtin_amdgcn_s_barrier();
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
   };
+  int k = 0, pI = 0, pJ = 0;   // tiles done; the tile before
   // one tile: row partials (reduced over the 4 waves through LDS) and transposed sums
-  auto tile = [&](int I, const T* t, T vraw) {
+  auto tile = [&](const T(&t)[16], T vraw, T uraw) __attribute__((always_inline)) {
     const int gr = I * kTB + ii;
     const T vi = (gr >= m) ? T(0) : (gr == 0 ? T(1) : (T)((double)vraw * scal));
+    if (fresh) {
+      const int gc = J * kTB + cg * 16 + (ii & 15);
+      if (ii < 16) vj[ii] = gc == 0 ? T(1) : (gc < m ? (T)((double)uraw * scal) : T(0));
+      __builtin_amdgcn_wave_barrier();
+      fresh = false;
+    }
     T yp = T(0);
     if (I > J) {
 #pragma unroll
@@ -392,42 +442,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     } else {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
-        yp += t[e] * vj[e];
-        if (ii > cg * 16 + e) zacc[e] += t[e] * vi;
+        const T x = ii >= cg * 16 + e && gr < m ? t[e] : T(0);
+        yp += x * vj[e];
+        if (ii > cg * 16 + e) zacc[e] += x * vi;
       }
     }
-    red[I & 3][cg][ii] = yp;
+    red[k & 3][cg][ii] = yp;
     // every second tile (and the last): one barrier, then the rows of the last two tiles are
     // summed over the waves (wave 0 and wave 1 take one tile each). A buffer is written again
     // four tiles later, after at least one more barrier.
-    if (((I - Ib) & 1) == 0 && I + 1 < Ie) return;
-    lds_barrier();
-    const int Ir = (cg == 0) ? I : I - 1;
-    if (cg < 2 && Ir >= Ib && (cg == 0 || ((I - Ib) & 1) == 1)) {
-      const int k = Ir * kTB + ii;
-      if (k < m)
-        Y[(long)J * n + k] = red[Ir & 3][0][ii] + red[Ir & 3][1][ii] + red[Ir & 3][2][ii] +
-                             red[Ir & 3][3][ii];
+    const bool last = t0 + k + 1 == t1;
+    if ((k & 1) || last) {
+      lds_barrier();
+      if (cg == 0 || (cg == 1 && (k & 1))) {
+        const int b = (k - cg) & 3, row = (cg == 0 ? I : pI) * kTB + ii;
+        if (row < m)
+          Y[(long)(cg == 0 ? J : pJ) * n + row] =
+              red[b][0][ii] + red[b][1][ii] + red[b][2][ii] + red[b][3][ii];
+      }
+    }
+    pI = I;
+    pJ = J;
+    ++k;
+    if (++I == nRB || last) {   // the column's end here
+      const T z = wave_sum16(zacc, ii);
+      const int kc = J * kTB + cg * 16 + ii;
+      if (ii < 16 && kc < m) Y[(long)(nRB + w - symv_first(nRB, J) / q) * n + kc] = z;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) zacc[e] = T(0);
+      I = ++J;
+      fresh = true;
     }
   };
-  // two tiles in flight ahead of the one being reduced
-  load(Ib, b0, v0);
-  if (Ib + 1 < Ie) load(Ib + 1, b1, v1);
-  for (int I = Ib; I < Ie; I += 3) {
-    if (I + 2 < Ie) load(I + 2, b2, v2);
-    tile(I, b0, v0);
-    if (I + 1 >= Ie) break;
-    if (I + 3 < Ie) load(I + 3, b0, v0);
-    tile(I + 1, b1, v1);
-    if (I + 2 >= Ie) break;
-    if (I + 4 < Ie) load(I + 4, b1, v1);
-    tile(I + 2, b2, v2);
-  }
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const T z = wave_sum(zacc[e]);
-    const int k = J * kTB + cg * 16 + e;
-    if (ii == 0 && k < m) Y[(long)(nRB + ch) * n + k] = z;
+  for (int t = t0; t < t1; t += 3) {
+    load(b2, v2, u2);
+    tile(b0, v0, u0);
+    if (t + 1 >= t1) break;
+    load(b0, v0, u0);
+    tile(b1, v1, u1);
+    if (t + 2 >= t1) break;
+    load(b1, v1, u1);
+    tile(b2, v2, u2);
   }
 }
 
@@ -460,7 +515,7 @@ __global__ __launch_bounds__(64 * kFinW) void finalize_w_kernel(T* a, long lda, 
   double acc = 0.0;
   if (k < m) {
     const int Ir = k / kTB;
-    const int nch = (nRB - Ir + tiles - 1) / tiles;
+    const int nch = symv_pieces(nRB, Ir, tiles);
     // this wave's slots (sl = wv, wv + kFinW, ...) with four independent sums
     double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
     int sl = wv;
@@ -577,9 +632,8 @@ static int sytrd_launches(hipStream_t s, T* a, long lda, long sA, int n, T* d, T
       const int m = n - c - 1;
       if (m <= 0) continue;
       const int nRB = (m + kTB - 1) / kTB;
-      // K problems in one launch fill the chip like one problem of K times the row blocks
-      const int tiles = symv_tiles<T>((int)std::min<long>((long)m * K, 1L << 30));
-      const int nCh = (nRB + tiles - 1) / tiles;
+      const int tiles = symv_tiles<T>(m, K);
+      const int nWg = (nRB * (nRB + 1) / 2 + tiles - 1) / tiles;
       SymvProfile& pf = g_symvProf;
       if (pf.on) {
         if (pf.ev.size() < 2 * (pf.used + 1)) {
@@ -591,15 +645,9 @@ static int sytrd_launches(hipStream_t s, T* a, long lda, long sA, int n, T* d, T
         }
         DH_HIP(hipEventRecord(pf.ev[2 * pf.used], s));
       }
-#define DH_SYMV(CH_)                                                                        \
-  hipLaunchKernelGGL((symv_kernel<T, CH_>), dim3(nRB, nCh, K), dim3(256), 0, s, a, lda, n, c, \
-                     j0, ws.W, ldw, ws.nrm2, tau, ws.dot, ws.Y, ws.nSlot, ws.vbuf, ws.t12,      \
-                     ws.scal, e, tau, ps)
-      if (tiles == 2) DH_SYMV(2);
-      else if (tiles == 4) DH_SYMV(4);
-      else if (tiles == 16) DH_SYMV(16);
-      else DH_SYMV(8);
-#undef DH_SYMV
+      hipLaunchKernelGGL(symv_kernel<T>, dim3(nRB + nWg, 1, K), dim3(256), 0, s, a, lda, n, c, j0,
+                         ws.W, ldw, ws.nrm2, tau, ws.dot, ws.Y, ws.vbuf, ws.t12, ws.scal, e, tau,
+                         tiles, ps);
       DH_LAUNCH_CHECK();
       if (pf.on) {
         DH_HIP(hipEventRecord(pf.ev[2 * pf.used + 1], s));

@@ -57,9 +57,9 @@ int dftbhip_dsytrd(char uplo, int n, double* a, int lda, double* d, double* e, d
  * (n up to about 17500); larger n is rejected with kErrArg. dftbhip_init must have been
  * called. Calls that overlap on one GPU share the workspace and race. */
 int dftbhip_dsytrd_noalloc(int n, double* a, int lda, double* d, double* e, double* tau);
-/* Kernel tuning. param 0: row tiles per workgroup of the tridiagonalisation's SYMV (2, 4, 8,
+/* Kernel tuning. param 0: tiles per workgroup of the tridiagonalisation's SYMV (2, 4, 8,
  * 16, or 0 = chosen from the trailing size per column, the default: the autotuned table of the
- * arithmetic type when there is one, else fixed thresholds); param 1, value 0: drop the
+ * arithmetic type when there is one, else the tiles shared out evenly); param 1, value 0: drop the
  * autotuned tables; param 2: k-points that are all real and of one size are tridiagonalised
  * together, one launch per column kernel for all points (1, the default) or one by one (0);
  * param 3: the neighbour list, pairs and SK blocks of a geometry are built on the device (1,
