@@ -1487,24 +1487,12 @@ struct Context {
   std::vector<DevBuf<double>> LinvK, XK;
   DevNeighbourList dnl;      // neighbour list built on the device
   bool nlOnDevice = false;
-  // k-points tridiagonalised together (all real, one size): reduced matrices and reflectors,
-  // d, e, tau and the workspace blocks of every point
-  DevBuf<double> kA, kD, kE, kTau;
+  // k-points of one size solved together: reduced matrices and reflectors, eigenvectors of the
+  // tridiagonals, d, e, tau, eigenvalues, workspaces and tables of a group of points
+  DevBuf<double> kA, kZ, kD, kE, kTau, kW, kDcWork;
+  DevBuf<GemmDesc<double>> kDesc;
+  std::shared_ptr<StedcWs> kDc;
   DevBuf<char> kWs;
-  // their divide and conquer side by side: per point a stream (default priority), the D&C
-  // buffers and the eigenvalues; the eigenvectors go straight to XK
-  struct KPointDc {
-    hipStream_t st = nullptr;
-    std::shared_ptr<StedcWs> ws;
-    DevBuf<double> work, w;
-    KPointDc() = default;
-    KPointDc(const KPointDc&) = delete;
-    KPointDc& operator=(const KPointDc&) = delete;
-    ~KPointDc() {
-      if (st) (void)hipStreamDestroy(st);
-    }
-  };
-  std::vector<std::unique_ptr<KPointDc>> kdc;
   std::vector<std::vector<double>> eigK, fillK;
   std::vector<int> noccK;
   EigenSolver eig;
@@ -2086,104 +2074,85 @@ static int ctx_scc_step(Context& c) {
       DH_HIP(hipEventRecord(ev[7], s));
       refineTimed = true;
     }
-    bool together = !ktail && g_kBatch && c.nk > 1 && !c.eig.twoStage && allReal;
-    if (together) {
-      // every point real and of size n: the reductions per point, one tridiagonalisation pass
-      // over all points (one launch per column kernel for all of them), then per point the
-      // divide and conquer and the back-transformation
-      const int K = c.nk;
-      const size_t nn = (size_t)n * n, wsStride = sytrd_work_bytes(n, 8);
-      DH_TRY(c.eig.ensure(n));
-      DH_TRY(c.kA.alloc(K * nn));
-      DH_TRY(c.kD.alloc((size_t)K * n));
-      DH_TRY(c.kE.alloc((size_t)K * n));
-      DH_TRY(c.kTau.alloc((size_t)K * n));
-      DH_TRY(c.kWs.alloc(K * wsStride));
+    // points of one size (the real ones, and the embeddings of the complex ones) are solved together
+    const bool together = !ktail && g_kBatch && c.nk > 1 && !c.eig.twoStage;
+    for (int nd = n; together && nd <= 2 * n; nd += n) {
+      std::vector<int> pt;
+      for (int k = 0; k < c.nk; ++k)
+        if (kpoint_dim(&c.kpts[3 * k], n) == nd) pt.push_back(k);
+      if (pt.empty()) continue;
+      const int nPt = (int)pt.size();
+      // the reductions per point, then one tridiagonalisation, divide and conquer and
+      // back-transformation for a group of points: a point of a few hundred orbitals leaves most
+      // of the chip idle and is bound by its launches. Groups bound the memory of the six
+      // matrices a point needs meanwhile. A thread and a stream per point took 4.6 ms for the
+      // divide and conquer and back-transformation of 8 points of 600 orbitals, this takes 1.5.
+      constexpr size_t kGroupBytes = 32ull << 30;
+      const size_t nn = (size_t)nd * nd, wsStride = sytrd_work_bytes(nd, 8);
+      const int most = (int)std::max<size_t>(1, kGroupBytes / (6 * nn * sizeof(double)));
+      const int nGroups = (nPt + most - 1) / most, G = (nPt + nGroups - 1) / nGroups;
+      DH_TRY(c.eig.ensure(nd));
+      DH_TRY(c.kA.alloc(G * nn));
+      DH_TRY(c.kZ.alloc(G * nn));
+      for (DevBuf<double>* x : {&c.kD, &c.kE, &c.kTau, &c.kW}) DH_TRY(x->alloc((size_t)G * nd));
+      DH_TRY(c.kWs.alloc(G * wsStride));
+      if (!c.kDc) c.kDc.reset(stedc_ws_new(), stedc_ws_delete);
       Events<3> kev;
       DH_TRY(kev.create());
-      DH_HIP(hipEventRecord(kev[0], s));
-      for (int k = 0; k < K; ++k) {
-        DH_TRY(launch_unpack_kpt(s, c.dblk.pr, c.dblk.norb.p, c.dblk.atomStart.p, c.blkT.p,
-                                 &c.kpts[3 * k], c.hs.p, c.Hd.p, n, n));
-        DH_TRY(c.eig.reduce(s, c.LinvK[k].p, c.Hd.p, n, c.kA.p + k * nn));
-      }
-      DH_HIP(hipEventRecord(kev[1], s));
-      DH_TRY(sytrd_lower_batched(s, c.kA.p, n, (long)nn, n, c.kD.p, c.kE.p, c.kTau.p, n,
-                                 c.kWs.p, wsStride, K));
-      DH_HIP(hipEventRecord(kev[2], s));
-      DH_HIP(hipEventSynchronize(kev[2]));
-      float ms;
-      DH_HIP(hipEventElapsedTime(&ms, kev[0], kev[1]));
-      evt[0] += ms * 1e-3;
-      DH_HIP(hipEventElapsedTime(&ms, kev[1], kev[2]));
-      evt[1] += ms * 1e-3;
-      // divide and conquer and back-transformation of the points side by side, one host thread
-      // and stream each: a D&C is mostly host deflation between short device phases, which the
-      // other points' device work fills
-      if ((int)c.kdc.size() < K) c.kdc.resize(K);
-      // one workspace per point: the D&C's, then the product L^-T (Q Z) and the reflector
-      // workspace of the back-transformation
-      const size_t dcWork = std::max(stedc_work_size(n), nn + ormtr_work_size(n, n));
-      for (int k = 0; k < K; ++k) {
-        if (!c.kdc[k]) c.kdc[k].reset(new Context::KPointDc());
-        Context::KPointDc& r = *c.kdc[k];
-        if (!r.st) DH_HIP(hipStreamCreate(&r.st));
-        if (!r.ws) r.ws.reset(stedc_ws_new(), stedc_ws_delete);
-        DH_TRY(r.work.alloc(dcWork));
-        DH_TRY(r.w.alloc(n));
-      }
-      int dev = 0;
-      DH_HIP(hipGetDevice(&dev));
-      std::vector<int> rcK(K, 0), infoK(K, 0);
-      std::vector<std::string> msgK(K);
-      auto dcPointBody = [&](int k) -> int {
-        Context::KPointDc& r = *c.kdc[k];
-        DH_HIP(hipSetDevice(dev));
-        DH_TRY(stedc_device(r.st, n, c.kD.p + (size_t)k * n, c.kE.p + (size_t)k * n, r.w.p,
-                            c.XK[k].p, n, r.work.p, dcWork, r.ws.get()));
-        c.eigK[k].resize(n);
-        DH_TRY(stedc_fetch(r.st, n, r.w.p, c.eigK[k].data(), r.ws.get(), &infoK[k]));
-        if (infoK[k] != 0) return 0;
-        // back-transformation on the same stream, the D&C workspace (free now) holding the
-        // product L^-T (Q Z) and the reflector workspace: Q Z in place, product, copy back
-        double* prod = r.work.p;
-        double* owork = r.work.p + nn;
-        DH_TRY(ormtr_lower(r.st, c.kA.p + k * nn, n, n, c.kTau.p + (size_t)k * n, c.XK[k].p, n,
-                           n, owork, dcWork - nn));
-        DH_TRY(gemm<double>(r.st, true, false, n, n, n, 1.0, c.LinvK[k].p, n, c.XK[k].p, n, 0.0,
-                            prod, n, false, kKAUpper));
-        DH_HIP(hipMemcpyAsync(c.XK[k].p, prod, nn * sizeof(double), hipMemcpyDeviceToDevice,
-                              r.st));
-        DH_HIP(hipStreamSynchronize(r.st));
-        return 0;
-      };
-      // an error leaves the point's thread only after the work it queued has ended, so that no
-      // kernel still writes the point's buffers when the caller reuses them
-      auto dcPoint = [&](int k) -> int {
-        const int rc = dcPointBody(k);
-        if (rc != 0) (void)hipStreamSynchronize(c.kdc[k]->st);
-        return rc;
-      };
-      const double tdc = now();
-      {
-        std::vector<std::thread> th;
-        th.reserve(K);
-        for (int k = 0; k < K; ++k)
-          th.emplace_back([&, k]() {
-            rcK[k] = dcPoint(k);
-            if (rcK[k] != 0) msgK[k] = last_error();
-          });
-        for (auto& t : th) t.join();
-      }
-      evt[2] += now() - tdc;
-      for (int k = 0; k < K; ++k) {
-        if (rcK[k] != 0) {
-          set_error(msgK[k]);
-          return rcK[k];
+      for (int g0 = 0; g0 < nPt; g0 += G) {
+        const int K = std::min(G, nPt - g0);
+        DH_HIP(hipEventRecord(kev[0], s));
+        for (int k = 0; k < K; ++k) {
+          DH_TRY(launch_unpack_kpt(s, c.dblk.pr, c.dblk.norb.p, c.dblk.atomStart.p, c.blkT.p,
+                                   &c.kpts[3 * pt[g0 + k]], c.hs.p, c.Hd.p, nd, n));
+          DH_TRY(c.eig.reduce(s, c.LinvK[pt[g0 + k]].p, c.Hd.p, nd, c.kA.p + k * nn));
         }
-        if (infoK[k] != 0) return infoK[k];
+        DH_HIP(hipEventRecord(kev[1], s));
+        DH_TRY(sytrd_lower_batched(s, c.kA.p, nd, (long)nn, nd, c.kD.p, c.kE.p, c.kTau.p, nd,
+                                   c.kWs.p, wsStride, K));
+        DH_HIP(hipEventRecord(kev[2], s));
+        DH_HIP(hipEventSynchronize(kev[2]));
+        float ms;
+        DH_HIP(hipEventElapsedTime(&ms, kev[0], kev[1]));
+        evt[0] += ms * 1e-3;
+        DH_HIP(hipEventElapsedTime(&ms, kev[1], kev[2]));
+        evt[1] += ms * 1e-3;
+        const double tdc = now();
+        std::vector<DcBlock> blocks;
+        for (int k = 0; k < K; ++k)
+          blocks.push_back({nd, (long)k * nd, (long)(k * nn), (long)(k * nn), nd, k});
+        size_t dcWork = 0;
+        DH_TRY(stedc_many_prepare(s, blocks, c.kDc.get(), &dcWork));
+        DH_TRY(c.kDcWork.alloc(std::max(dcWork, ormtr_many_work(nd, K))));
+        DH_TRY(stedc_many(s, c.kD.p, c.kE.p, c.kW.p, c.kZ.p, c.kDcWork.p, nullptr, c.kDc.get()));
+        std::vector<double> wAll((size_t)K * nd);
+        std::vector<int> infoK(K);
+        DH_HIP(hipMemcpyAsync(wAll.data(), c.kW.p, wAll.size() * sizeof(double),
+                              hipMemcpyDeviceToHost, s));
+        DH_HIP(hipMemcpyAsync(infoK.data(), stedc_info(c.kDc.get()), K * sizeof(int),
+                              hipMemcpyDeviceToHost, s));
+        DH_HIP(hipStreamSynchronize(s));
+        for (int k = 0; k < K; ++k) {
+          if (infoK[k] != 0) return infoK[k];
+          const int q = pt[g0 + k];
+          c.eigK[q].assign(wAll.begin() + (size_t)k * nd, wAll.begin() + (size_t)(k + 1) * nd);
+          // each complex level appears twice in the embedding
+          const int stride = nd / n;
+          ec[q].resize(n);
+          for (int j = 0; j < n; ++j) ec[q][j] = c.eigK[q][stride * j];
+        }
+        // X = L^-T (Q Z)
+        DH_TRY(ormtr_lower_many(s, c.kA.p, (long)nn, nd, c.kTau.p, nd, c.kZ.p, (long)nn, K,
+                                c.kDcWork.p, c.kDesc));
+        std::vector<GemmDesc<double>> prod(K);
+        for (int k = 0; k < K; ++k)
+          prod[k] = {nd, nd, nd, c.LinvK[pt[g0 + k]].p, (long)nd, c.kZ.p + k * nn, (long)nd,
+                     c.XK[pt[g0 + k]].p, (long)nd};
+        DH_TRY(c.kDesc.upload(prod.data(), K, s));
+        DH_TRY(gemm_batched<double>(s, true, false, c.kDesc.p, K, nd, nd, 1.0, 0.0));
+        DH_HIP(hipStreamSynchronize(s));
+        evt[2] += now() - tdc;
       }
-      for (int k = 0; k < K; ++k) ec[k] = c.eigK[k];
     }
     for (int k = 0; k < c.nk && !together && !ktail; ++k) {
       const int ndk = kpoint_dim(&c.kpts[3 * k], n);

@@ -240,6 +240,9 @@ int sytrd_lower_batched(hipStream_t s, double* a, long lda, long sA, int n, doub
 // per-launch timing of the tridiagonalisation's symmetric product: launches, seconds, bytes
 void symv_profiling(bool on);
 void symv_profile_stats(double* out);
+size_t ormtr_many_work(int n, int K);
+int ormtr_lower_many(hipStream_t s, const double* a, long sA, int n, const double* tau, long sV,
+                     double* z, long sZ, int K, double* work, DevBuf<GemmDesc<double>>& desc);
 int ormtr_lower(hipStream_t s, const double* a, long lda, int n, const double* tau, double* z,
                 long ldz, int ncols, double* work, size_t workSize);
 size_t ormtr_work_size(int n, int ncols);

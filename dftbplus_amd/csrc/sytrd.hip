@@ -852,7 +852,9 @@ size_t ormtr_work_size(int n, int ncols) { return (ormtr_work_bytes(n, ncols, 8)
 // at row c + shift and its other elements below it in column c of a
 template <typename T>
 __global__ void form_v_kernel(const T* a, long lda, int n, int j0, int pw, int shift, T* V,
-                              long ldv) {
+                              long ldv, long sA = 0, long sW = 0) {
+  a += blockIdx.z * sA;
+  V += blockIdx.z * sW;
   const int p = blockIdx.y;
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   const int r = j0 + shift + k;
@@ -873,7 +875,10 @@ __global__ void form_v_kernel(const T* a, long lda, int n, int j0, int pw, int s
 // takes 52 us.
 template <typename T>
 __global__ __launch_bounds__(256) void larft_kernel(const T* G, long ld, const T* tau, int j0,
-                                                    int nref, T* Tout) {
+                                                    int nref, T* Tout, long sV = 0, long sW = 0) {
+  G += blockIdx.y * sW;
+  tau += blockIdx.y * sV;
+  Tout += blockIdx.y * sW;
   constexpr int kLd = kOBH + 1;
   __shared__ T X[kOBH * kLd];
   __shared__ T tl[kOBH];
@@ -936,6 +941,50 @@ int ormtr_lower_t(hipStream_t s, const T* a, long lda, int n, const T* tau, T* z
                    kOB));
     DH_TRY(gemm<T>(s, false, false, m, ncols, pw, T(-1), ws.V, m, ws.W2, kOB, T(1), zr, ldz));
   }
+  return 0;
+}
+
+// Z_k <- Q_k Z_k (n x n each) for K problems, kOBH reflectors at a time: six launches a block for
+// all problems. desc: room for 4 descriptors per problem and block of reflectors.
+static long ormtr_many_stride(int n) { return 3L * kOBH * n + 2L * kOBH * kOBH; }
+size_t ormtr_many_work(int n, int K) { return (size_t)K * ormtr_many_stride(n); }
+
+int ormtr_lower_many(hipStream_t s, const double* a, long sA, int n, const double* tau, long sV,
+                     double* z, long sZ, int K, double* work, DevBuf<GemmDesc<double>>& desc) {
+  const int nref = n - 1;
+  if (nref <= 0 || K <= 0) return 0;
+  const long sW = ormtr_many_stride(n);
+  std::vector<GemmDesc<double>> h;
+  for (int j0 = (nref - 1) / kOBH * kOBH; j0 >= 0; j0 -= kOBH) {
+    const int pw = std::min(kOBH, nref - j0), m = n - j0 - 1;
+    for (int q = 0; q < 4; ++q)
+      for (int k = 0; k < K; ++k) {
+        double* V = work + k * sW;
+        double *W1 = V + (long)kOBH * n, *W2 = W1 + (long)kOBH * n, *G = W2 + (long)kOBH * n,
+               *T = G + kOBH * kOBH, *zr = z + k * sZ + j0 + 1;
+        if (q == 0) h.push_back({pw, pw, m, V, (long)m, V, (long)m, G, (long)kOBH});
+        if (q == 1) h.push_back({pw, n, m, V, (long)m, zr, (long)n, W1, (long)kOBH});
+        if (q == 2) h.push_back({pw, n, pw, T, (long)kOBH, W1, (long)kOBH, W2, (long)kOBH});
+        if (q == 3) h.push_back({m, n, pw, V, (long)m, W2, (long)kOBH, zr, (long)n});
+      }
+  }
+  DH_TRY(desc.upload(h.data(), h.size(), s));
+  const GemmDesc<double>* g = desc.p;
+  for (int j0 = (nref - 1) / kOBH * kOBH; j0 >= 0; j0 -= kOBH, g += 4 * (size_t)K) {
+    const int pw = std::min(kOBH, nref - j0), m = n - j0 - 1;
+    double *G = work + 3L * kOBH * n, *T = G + kOBH * kOBH;
+    hipLaunchKernelGGL(form_v_kernel<double>, dim3(cdiv(m, 256), pw, K), dim3(256), 0, s, a,
+                       (long)n, n, j0, pw, 1, work, (long)m, sA, sW);
+    DH_LAUNCH_CHECK();
+    DH_TRY(gemm_batched<double>(s, true, false, g, K, pw, pw, 1.0, 0.0));
+    hipLaunchKernelGGL(larft_kernel<double>, dim3(1, K), dim3(256), 0, s, G, (long)kOBH, tau, j0,
+                       pw, T, sV, sW);
+    DH_LAUNCH_CHECK();
+    DH_TRY(gemm_batched<double>(s, true, false, g + K, K, pw, n, 1.0, 0.0));
+    DH_TRY(gemm_batched<double>(s, false, false, g + 2 * K, K, pw, n, 1.0, 0.0));
+    DH_TRY(gemm_batched<double>(s, false, false, g + 3 * K, K, m, n, -1.0, 1.0));
+  }
+  DH_HIP(hipStreamSynchronize(s));   // the descriptors' host copy
   return 0;
 }
 

@@ -60,8 +60,8 @@ int dftbhip_dsytrd_noalloc(int n, double* a, int lda, double* d, double* e, doub
 /* Kernel tuning. param 0: tiles per workgroup of the tridiagonalisation's SYMV (2, 4, 8,
  * 16, or 0 = chosen from the trailing size per column, the default: the autotuned table of the
  * arithmetic type when there is one, else the tiles shared out evenly); param 1, value 0: drop the
- * autotuned tables; param 2: k-points that are all real and of one size are tridiagonalised
- * together, one launch per column kernel for all points (1, the default) or one by one (0);
+ * autotuned tables; param 2: the real k-points, and the complex ones, are solved together,
+ * one launch per kernel for all points (1, the default) or one by one (0);
  * param 3: the neighbour list, pairs and SK blocks of a geometry are built on the device (1,
  * the default) or on the host (0); param 4: the molecule batch's per-molecule Fermi levels,
  * energies, convergence tests and Broyden mixing run on host threads (0), as device kernels
