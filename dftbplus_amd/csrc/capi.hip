@@ -1491,6 +1491,7 @@ struct Context {
   // tridiagonals, d, e, tau, eigenvalues, workspaces and tables of a group of points
   DevBuf<double> kA, kZ, kD, kE, kTau, kW, kDcWork;
   DevBuf<GemmDesc<double>> kDesc;
+  DevBuf<int> kInfo;
   std::shared_ptr<StedcWs> kDc;
   DevBuf<char> kWs;
   std::vector<std::vector<double>> eigK, fillK;
@@ -1543,6 +1544,23 @@ struct Context {
 
 static double now() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
+// the k-points whose problem has dim rows (n: real, 2n: the embedding of a complex one)
+static std::vector<int> points_of_size(const std::vector<double>& kpts, int nk, int n, int dim) {
+  std::vector<int> pt;
+  for (int k = 0; k < nk; ++k)
+    if (kpoint_dim(&kpts[3 * k], n) == dim) pt.push_back(k);
+  return pt;
+}
+
+// points worked on together: the six matrices a point needs meanwhile stay within 32 GiB, in
+// groups of equal size
+static int kpoint_group(int count, int dim) {
+  const size_t bytes = 6 * sizeof(double) * (size_t)dim * dim;
+  const int most = (int)std::max<size_t>(1, (32ull << 30) / bytes);
+  const int groups = (count + most - 1) / most;
+  return (count + groups - 1) / groups;
 }
 
 static int ctx_geometry(Context& c, int nat, const double* coords, const int* species,
@@ -1721,7 +1739,40 @@ static int ctx_geometry(Context& c, int nat, const double* coords, const int* sp
     c.eigK.assign(c.nk, std::vector<double>());
     c.fillK.assign(c.nk, std::vector<double>());
     c.noccK.assign(c.nk, 0);
-    for (int k = 0; k < c.nk && info == 0; ++k) {
+    // points of one size are factored together, in groups that bound the memory
+    const bool together = g_kBatch && c.nk > 1;
+    std::vector<int> infoAll(c.nk, 0);
+    for (int dim = n; together && dim <= 2 * n; dim += n) {
+      const std::vector<int> pt = points_of_size(c.kpts, c.nk, n, dim);
+      if (pt.empty()) continue;
+      const size_t nn = (size_t)dim * dim;
+      const int G = kpoint_group((int)pt.size(), dim);
+      DH_TRY(c.eig.ensure(dim));
+      DH_TRY(c.kA.alloc(G * nn));
+      DH_TRY(c.kZ.alloc(G * nn));
+      DH_TRY(c.kDcWork.alloc(G * (nn + potrf_inv_work(dim))));
+      DH_TRY(c.kInfo.alloc(G));
+      for (size_t g0 = 0; g0 < pt.size(); g0 += G) {
+        const int K = std::min(G, (int)(pt.size() - g0));
+        for (int k = 0; k < K; ++k)
+          DH_TRY(launch_unpack_kpt(s, c.dblk.pr, c.dblk.norb.p, c.dblk.atomStart.p, c.blkT.p,
+                                   &c.kpts[3 * pt[g0 + k]], c.ov.p, c.kA.p + k * nn, dim, n));
+        std::vector<int> hInfo(K, 0);
+        DH_TRY(potrf_inverse_many(s, c.kA.p, c.kZ.p, c.kDcWork.p, dim, K, c.kDcWork.p + K * nn,
+                                  c.kDesc, c.kInfo.p, hInfo.data()));
+        for (int k = 0; k < K; ++k) {
+          const int q = pt[g0 + k];
+          infoAll[q] = hInfo[k];
+          DH_TRY(c.LinvK[q].alloc(nn));
+          DH_TRY(c.XK[q].alloc(nn));
+          DH_HIP(hipMemcpyAsync(c.LinvK[q].p, c.kDcWork.p + k * nn, nn * sizeof(double),
+                                hipMemcpyDeviceToDevice, s));
+        }
+      }
+    }
+    for (int k = 0; k < c.nk && info == 0; ++k) info = infoAll[k];
+    if (together && info == 0) c.eig.factored = true;
+    for (int k = 0; k < c.nk && info == 0 && !together; ++k) {
       const int ndk = kpoint_dim(&c.kpts[3 * k], n);
       DH_TRY(launch_unpack_kpt(s, c.dblk.pr, c.dblk.norb.p, c.dblk.atomStart.p, c.blkT.p,
                                &c.kpts[3 * k], c.ov.p, c.Sd.p, ndk, n));
@@ -2077,9 +2128,7 @@ static int ctx_scc_step(Context& c) {
     // points of one size (the real ones, and the embeddings of the complex ones) are solved together
     const bool together = !ktail && g_kBatch && c.nk > 1 && !c.eig.twoStage;
     for (int nd = n; together && nd <= 2 * n; nd += n) {
-      std::vector<int> pt;
-      for (int k = 0; k < c.nk; ++k)
-        if (kpoint_dim(&c.kpts[3 * k], n) == nd) pt.push_back(k);
+      const std::vector<int> pt = points_of_size(c.kpts, c.nk, n, nd);
       if (pt.empty()) continue;
       const int nPt = (int)pt.size();
       // the reductions per point, then one tridiagonalisation, divide and conquer and
@@ -2087,10 +2136,8 @@ static int ctx_scc_step(Context& c) {
       // of the chip idle and is bound by its launches. Groups bound the memory of the six
       // matrices a point needs meanwhile. A thread and a stream per point took 4.6 ms for the
       // divide and conquer and back-transformation of 8 points of 600 orbitals, this takes 1.5.
-      constexpr size_t kGroupBytes = 32ull << 30;
       const size_t nn = (size_t)nd * nd, wsStride = sytrd_work_bytes(nd, 8);
-      const int most = (int)std::max<size_t>(1, kGroupBytes / (6 * nn * sizeof(double)));
-      const int nGroups = (nPt + most - 1) / most, G = (nPt + nGroups - 1) / nGroups;
+      const int G = kpoint_group(nPt, nd);
       DH_TRY(c.eig.ensure(nd));
       DH_TRY(c.kA.alloc(G * nn));
       DH_TRY(c.kZ.alloc(G * nn));

@@ -240,6 +240,9 @@ int sytrd_lower_batched(hipStream_t s, double* a, long lda, long sA, int n, doub
 // per-launch timing of the tridiagonalisation's symmetric product: launches, seconds, bytes
 void symv_profiling(bool on);
 void symv_profile_stats(double* out);
+size_t potrf_inv_work(int n);
+int potrf_inverse_many(hipStream_t s, double* a, double* l, double* linv, int n, int K,
+                       double* work, DevBuf<GemmDesc<double>>& desc, int* dInfo, int* hInfo);
 size_t ormtr_many_work(int n, int K);
 int ormtr_lower_many(hipStream_t s, const double* a, long sA, int n, const double* tau, long sV,
                      double* z, long sZ, int K, double* work, DevBuf<GemmDesc<double>>& desc);

@@ -250,10 +250,14 @@ constexpr int kPotrfNB = 64;
 // columns: the block lives in registers (thread (ty, tx) of 16 x 16 holds rows ty + 16 p, columns
 // tx + 16 q), and a column takes one barrier: its unscaled entries go to LDS, and everyone
 // subtracts their products over the pivot. With the block in LDS and three barriers and a row of
-// divisions per column the kernel took 131 us; this form takes 42 us.
+// divisions per column the kernel took 131 us; this form takes 42 us. Problem blockIdx.x of many is
+// found at strides sA, sV.
 __global__ __launch_bounds__(256) void potrf_diag_kernel(double* a, long lda, int jb,
                                                          double* linv, long ldv, int offset,
-                                                         int* dInfo) {
+                                                         int* dInfo, long sA, long sV) {
+  a += blockIdx.x * sA;
+  if (linv) linv += blockIdx.x * sV;
+  dInfo += blockIdx.x;
   constexpr int kLd = kPotrfNB + 1;
   static_assert(kPotrfNB == 64, "potrf_diag: 4 x 4 elements per thread");
   __shared__ double X[kPotrfNB * kLd];
@@ -326,7 +330,7 @@ int potrf_lower_impl(hipStream_t s, double* a, long lda, int n, double* linv, lo
     const int jb = std::min(kPotrfNB, n - j);
     double* ljj = linv + j + (long)j * ldv;
     hipLaunchKernelGGL(potrf_diag_kernel, dim3(1), dim3(256), 0, s, a + j + (long)j * lda, lda, jb,
-                       ljj, ldv, j, dInfo);
+                       ljj, ldv, j, dInfo, 0L, 0L);
     DH_LAUNCH_CHECK();
     const int m = n - j - jb;
     if (m > 0) {
@@ -381,6 +385,80 @@ int trtri_from_diag(hipStream_t s, const double* l, long ldl, double* linv, long
     // descriptors must outlive the launches
     DH_HIP(hipStreamSynchronize(s));
   }
+  return 0;
+}
+
+// Inverse Cholesky factors of K matrices of size n (one after the other in a, overwritten) into
+// linv, the panels of the factors in l; work: potrf_inv_work(n) doubles per matrix. hInfo: K words.
+// A single matrix is bound by the chain of its small kernels (0.9 ms for 600 rows, whatever runs
+// beside it); here every launch takes all matrices.
+size_t potrf_inv_work(int n) { return (size_t)n * n / 2 + 64 * (size_t)n + 4096; }
+
+int potrf_inverse_many(hipStream_t s, double* a, double* l, double* linv, int n, int K,
+                       double* work, DevBuf<GemmDesc<double>>& desc, int* dInfo, int* hInfo) {
+  const long nn = (long)n * n, ld = n;
+  std::vector<GemmDesc<double>> h;
+  for (int j = 0; j + kPotrfNB < n; j += kPotrfNB) {
+    const int m = n - j - kPotrfNB;
+    const long r = j + kPotrfNB, jj = j + (long)j * ld, rj = r + (long)j * ld;
+    for (int q = 0; q < 2; ++q)
+      for (int k = 0; k < K; ++k) {
+        const long o = k * nn;
+        // L21 = A21 L11^-T, then A22 -= L21 L21^T
+        if (q == 0) h.push_back({m, kPotrfNB, kPotrfNB, a + o + rj, ld, linv + o + jj, ld,
+                                 l + o + rj, ld});
+        else h.push_back({m, m, kPotrfNB, l + o + rj, ld, l + o + rj, ld, a + o + r + r * ld, ld});
+      }
+  }
+  // pairs of diagonal blocks joined by doubling, as in trtri_from_diag
+  const int nleaf = (n + kPotrfNB - 1) / kPotrfNB;
+  struct Level {
+    int count, size;
+  };
+  std::vector<Level> levels;
+  for (int p = 1; p < nleaf; p *= 2) {
+    Level lv{0, 0};
+    for (int q = 0; q < 2; ++q)
+      for (int k = 0; k < K; ++k) {
+        const long o = k * nn;
+        double* t = work + k * potrf_inv_work(n);
+        for (int s0 = 0; s0 + p < nleaf; s0 += 2 * p) {
+          const int r1 = s0 * kPotrfNB, r2 = (s0 + p) * kPotrfNB, n1 = r2 - r1;
+          const int n2 = std::min((s0 + 2 * p) * kPotrfNB, n) - r2;
+          const long x11 = o + r1 + r1 * ld, x22 = o + r2 + r2 * ld, x21 = o + r2 + r1 * ld;
+          // T = L21 X11, X21 = -X22 T
+          if (q == 0) h.push_back({n2, n1, n1, l + x21, ld, linv + x11, ld, t, (long)n2});
+          else h.push_back({n2, n1, n2, linv + x22, ld, t, (long)n2, linv + x21, ld});
+          t += (size_t)n1 * n2;
+          if (q == 0) ++lv.count;
+          lv.size = std::max(lv.size, std::max(n1, n2));
+        }
+      }
+    levels.push_back(lv);
+  }
+  DH_TRY(desc.upload(h.data(), h.size(), s));
+  DH_TRY(fill<int>(s, dInfo, K, 0));
+  DH_TRY(fill<double>(s, linv, K * nn, 0.0));
+  const GemmDesc<double>* g = desc.p;
+  for (int j = 0; j < n; j += kPotrfNB) {
+    const int jb = std::min(kPotrfNB, n - j), m = n - j - jb;
+    const long jj = j + (long)j * ld;
+    hipLaunchKernelGGL(potrf_diag_kernel, dim3(K), dim3(256), 0, s, a + jj, ld, jb, linv + jj, ld,
+                       j, dInfo, nn, nn);
+    DH_LAUNCH_CHECK();
+    if (m <= 0) break;
+    DH_TRY(gemm_batched<double>(s, false, true, g, K, m, jb, 1.0, 0.0));
+    DH_TRY(gemm_batched<double>(s, false, true, g + K, K, m, m, -1.0, 1.0));
+    g += 2 * (size_t)K;
+  }
+  for (const Level& lv : levels) {
+    DH_TRY(gemm_batched<double>(s, false, false, g, lv.count, lv.size, lv.size, 1.0, 0.0));
+    g += lv.count;
+    DH_TRY(gemm_batched<double>(s, false, false, g, lv.count, lv.size, lv.size, -1.0, 0.0));
+    g += lv.count;
+  }
+  DH_HIP(hipMemcpyAsync(hInfo, dInfo, K * sizeof(int), hipMemcpyDeviceToHost, s));
+  DH_HIP(hipStreamSynchronize(s));   // also the descriptors' host copy
   return 0;
 }
 
