@@ -42,14 +42,26 @@ struct BatchDescs {
   GemmDesc<double>*hc, *chc, *back;
   int* solve;   // per molecule: solved in this call
 };
+constexpr int kFactorNB = 64;   // panel of the overlap factorisation (potrf_diag's block)
+struct FactorStep {
+  int panel, count, m, n;   // panel the products belong to (-1: joining of blocks), their extent
+  long first;               // first descriptor
+};
 struct BatchEigen {
   int first[kBatchClasses + 1] = {}, maxn[kBatchClasses] = {}, direct = 0;
   std::shared_ptr<StedcWs> dc;
   DevBuf<double> work, d, e, tau;
-  DevBuf<GemmDesc<double>> desc;
+  DevBuf<GemmDesc<double>> desc, factorDesc;
+  std::vector<FactorStep> steps;
   DevBuf<int> solve;
   int prepare(hipStream_t s, const BatchLayout& L, const std::vector<int>& order,
-              const std::vector<long>& orb0, const std::vector<long>& dOff);
+              const std::vector<long>& orb0, const std::vector<long>& dOff, double* matrices,
+              double* C);
+  int maxDirect() const {
+    int n = 0;
+    for (int c = 1; c < kBatchClasses; ++c) n = n > maxn[c] ? n : maxn[c];
+    return n;
+  }
 };
 // eigenvalues w (ascending per molecule, at orb0), eigenvectors C (packed), info per molecule
 // (0, or j+1 when the leading minor j+1 of S is not positive definite); work 3 x packed size,

@@ -448,23 +448,29 @@ __global__ __launch_bounds__(kSygvThreads) void batch_sygv_kernel(BatchLayout L,
 }
 
 // ------------------------------------------------------------------------------------------
-// Direct eigensolver for molecules of up to kWgBatchMax orbitals: Cw = L^-T once per geometry,
-// then per call A = Cw^T H Cw (batched MFMA GEMMs), tridiagonalisation with the matrix in the
-// registers of one workgroup (sytrd_resident.hip), divide and conquer of all molecules together
-// (stedc.hip), the reflectors applied to strips of eigenvectors, and C = Cw (Q Z). A parallel
+// Direct eigensolver for molecules of up to kWgBatchMax orbitals: L^-1 once per geometry (panels
+// of 64 columns, every launch for all molecules that reach its panel; one workgroup per molecule
+// in HBM took 2.1 ms for 190 orbitals), then per call A = L^-1 H L^-T (batched MFMA GEMMs),
+// tridiagonalisation with the matrix in the registers of one workgroup (sytrd_resident.hip),
+// divide and conquer of all molecules together (stedc.hip), the reflectors applied to strips of
+// eigenvectors, and C = L^-T (Q Z). A parallel
 // cyclic Jacobi with A and C in LDS ran here before, n dependent rounds per sweep and 7 to 10
 // sweeps. One SCC cycle of 32 molecules of 13 to 190 orbitals: 135 ms before, 16.7 ms now; of
 // 1000 molecules: 250 ms before, 51 ms now. Bound by the column chain of the reduction (0.38 ms
 // per iteration for 190 orbitals, 0.12 for 112), then by the solve's own latencies.
 // ------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(kSygvThreads) void batch_factor_kernel(BatchLayout L, const int* list,
-                                                                    const double* S, double* work,
-                                                                    int* info) {
-  const int m = list[blockIdx.x];
-  const int n = (int)(L.orb0[m + 1] - L.orb0[m]);
+// Start of the factorisation: B0 = S, the place of L^-1 zero, info 0
+__global__ void batch_factor_init_kernel(BatchLayout L, const int* list, const double* S,
+                                         double* work, int* info) {
+  const int m = list[blockIdx.y];
+  const long n = L.orb0[m + 1] - L.orb0[m], nn = n * n;
   double* B0 = work + 3 * L.dOff[m];
-  if (wg_factor(n, S + L.dOff[m], B0, B0 + 2 * (long)n * n, info + m) && threadIdx.x == 0)
-    info[m] = 0;
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < nn;
+       e += (long)gridDim.x * blockDim.x) {
+    B0[e] = S[L.dOff[m] + e];
+    B0[2 * nn + e] = 0.0;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) info[m] = 0;
 }
 
 // The products of a call, empty for molecules that are not active (or whose overlap failed)
@@ -479,10 +485,10 @@ __global__ void batch_desc_kernel(BatchLayout L, const int* list, int count, con
   const long nn = L.dOff[m + 1] - L.dOff[m], ld = L.orb0[m + 1] - L.orb0[m];
   double* B0 = work + 3 * L.dOff[m];
   double* B1 = B0 + nn;
-  const double* Cw = B1 + nn;
-  g.hc[t] = {n, n, n, H + L.dOff[m], ld, Cw, ld, B1, ld};
-  g.chc[t] = {n, n, n, Cw, ld, B1, ld, B0, ld};
-  g.back[t] = {n, n, n, Cw, ld, B1, ld, C + L.dOff[m], ld};
+  const double* Li = B1 + nn;
+  g.hc[t] = {n, n, n, H + L.dOff[m], ld, Li, ld, B1, ld};      // B1 = H L^-T
+  g.chc[t] = {n, n, n, Li, ld, B1, ld, B0, ld};                // B0 = L^-1 B1
+  g.back[t] = {n, n, n, Li, ld, B1, ld, C + L.dOff[m], ld};    // C = L^-T (Q Z)
   g.solve[m] = on;
 }
 
@@ -667,7 +673,8 @@ int launch_batch_pack(hipStream_t s, const PairsDev& pr, const int* norb, const 
 }
 
 int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<int>& order,
-                        const std::vector<long>& orb0, const std::vector<long>& dOff) {
+                        const std::vector<long>& orb0, const std::vector<long>& dOff,
+                        double* matrices, double* C) {
   int nDirect = 0;
   first[0] = 0;
   for (int c = 0; c < kBatchClasses; ++c) {
@@ -696,6 +703,54 @@ int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<i
   DH_TRY(e.alloc(norb));
   DH_TRY(tau.alloc(norb));
   direct = nDirect;
+  // the products of the factorisation; the list is sorted, so the molecules that reach a panel or
+  // a level are its first ones
+  std::vector<GemmDesc<double>> h;
+  steps.clear();
+  auto size = [&](int t) { return orb0[order[t] + 1] - orb0[order[t]]; };
+  const int big = nDirect > 0 ? (int)size(first[1]) : 0;
+  for (int j = 0; j + kFactorNB < big; j += kFactorNB)
+    for (int q = 0; q < 2; ++q) {
+      FactorStep st{j, 0, 0, 0, (long)h.size()};
+      for (int t = first[1]; t < L.nmol && size(t) > j + kFactorNB; ++t) {
+        const long n = size(t), nn = n * n, r = j + kFactorNB;
+        const int m = (int)(n - r);
+        double* A = matrices + 3 * dOff[order[t]];
+        // L21 = A21 L11^-T into B1, then A22 -= L21 L21^T
+        if (q == 0) h.push_back({m, kFactorNB, kFactorNB, A + r + j * n, n, A + 2 * nn + j + j * n, n,
+                                 A + nn + r + j * n, n});
+        else h.push_back({m, m, kFactorNB, A + nn + r + j * n, n, A + nn + r + j * n, n,
+                          A + r + r * n, n});
+        ++st.count;
+        st.m = std::max(st.m, m);
+        st.n = std::max(st.n, q == 0 ? kFactorNB : m);
+      }
+      steps.push_back(st);
+    }
+  // pairs of diagonal blocks joined: T = L21 X11 (in C's place), X21 = -X22 T
+  for (int p = kFactorNB; p < big; p *= 2)
+    for (int q = 0; q < 2; ++q) {
+      FactorStep st{-1, 0, 0, 0, (long)h.size()};
+      for (int t = first[1]; t < L.nmol && size(t) > p; ++t) {
+        const long n = size(t), nn = n * n;
+        double* A = matrices + 3 * dOff[order[t]];
+        double* T = C + dOff[order[t]];
+        for (int r1 = 0; r1 + p < n; r1 += 2 * p) {
+          const long r2 = r1 + p;
+          const int n2 = (int)(std::min(r2 + p, n) - r2);
+          double* X = A + 2 * nn;
+          if (q == 0) h.push_back({n2, p, p, A + nn + r2 + r1 * n, n, X + r1 + r1 * n, n, T, n2});
+          else h.push_back({n2, p, n2, X + r2 + r2 * n, n, T, n2, X + r2 + r1 * n, n});
+          T += (long)n2 * p;
+          ++st.count;
+          st.m = std::max(st.m, n2);
+          st.n = p;
+        }
+      }
+      steps.push_back(st);
+    }
+  DH_TRY(factorDesc.upload(h.data(), h.size(), s));
+  DH_HIP(hipStreamSynchronize(s));   // the descriptors' host copy
   return 0;
 }
 
@@ -714,9 +769,30 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
   GemmDesc<double>* g = E.desc.p;
   const BatchDescs ds{g, g + L.nmol, g + 2 * (size_t)L.nmol, E.solve.p};
   if (!warm) {
-    hipLaunchKernelGGL(batch_factor_kernel, dim3(nd), dim3(kSygvThreads), 0, s, L, list, S, work,
-                       info);
-    DH_LAUNCH_CHECK();
+    for (int p = 0; p < nd; p += 32768) {
+      hipLaunchKernelGGL(batch_factor_init_kernel, dim3(8, std::min(32768, nd - p)), dim3(256), 0, s,
+                         L, list + p, S, work, info);
+      DH_LAUNCH_CHECK();
+    }
+    int done = 0;   // panels whose diagonal block has been factored
+    auto diagonals = [&](int upTo) -> int {
+      for (; done <= upTo; done += kFactorNB)
+        DH_TRY(launch_potrf_diag_list(s, nd, list, L.dOff, L.orb0, work, done, info));
+      return 0;
+    };
+    bool second = false;
+    for (const FactorStep& st : E.steps) {
+      DH_TRY(diagonals(st.panel >= 0 ? st.panel : E.maxDirect() - 1));
+      const GemmDesc<double>* d = E.factorDesc.p + st.first;
+      if (st.panel >= 0)
+        DH_TRY(gemm_batched<double>(s, false, true, d, st.count, st.m, st.n, second ? -1.0 : 1.0,
+                                    second ? 1.0 : 0.0));
+      else
+        DH_TRY(gemm_batched<double>(s, false, false, d, st.count, st.m, st.n,
+                                    second ? -1.0 : 1.0, 0.0));
+      second = !second;
+    }
+    DH_TRY(diagonals(E.maxDirect() - 1));
   }
   hipLaunchKernelGGL(batch_desc_kernel, dim3(cdiv(nd, 256)), dim3(256), 0, s, L, list, nd, H, work,
                      C, info, active, ds);
@@ -733,8 +809,8 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
     hipStream_t sc = st[c];
     if (c > 1) DH_HIP(hipStreamWaitEvent(sc, done[0], 0));
     else sc = s;
-    DH_TRY(gemm_batched<double>(sc, false, false, ds.hc + o, cnt, mx, mx, 1.0, 0.0));
-    DH_TRY(gemm_batched<double>(sc, true, false, ds.chc + o, cnt, mx, mx, 1.0, 0.0));
+    DH_TRY(gemm_batched<double>(sc, false, true, ds.hc + o, cnt, mx, mx, 1.0, 0.0));
+    DH_TRY(gemm_batched<double>(sc, false, false, ds.chc + o, cnt, mx, mx, 1.0, 0.0));
     WgBatch bt;
     bt.list = list + o;
     bt.active = E.solve.p;
@@ -766,7 +842,7 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
 #undef DH_APPLY
       DH_LAUNCH_CHECK();
     }
-    return gemm_batched<double>(s, false, false, ds.back + o, cnt, mx, mx, 1.0, 0.0);
+    return gemm_batched<double>(s, true, false, ds.back + o, cnt, mx, mx, 1.0, 0.0);
   });
 }
 

@@ -2770,7 +2770,7 @@ static int batch_geometry(BatchContext& b, int nmol, const int* natMol, const do
   for (DevBuf<double>* x : {&b.Sd, &b.Hd, &b.Cv, &b.P}) DH_TRY(x->alloc(b.denseSize));
   DH_TRY(b.work.alloc(3 * b.denseSize));
   DH_TRY(b.gamma.alloc(b.gammaSize));
-  DH_TRY(b.be.prepare(s, b.L, order, b.orb0, b.dOff));
+  DH_TRY(b.be.prepare(s, b.L, order, b.orb0, b.dOff, b.work.p, b.Cv.p));
   DH_TRY(b.infoD.alloc(nmol));
   DH_TRY(b.noccD.alloc(nmol));
   DH_TRY(b.activeD.alloc(nmol));

@@ -240,6 +240,8 @@ int sytrd_lower_batched(hipStream_t s, double* a, long lda, long sA, int n, doub
 // per-launch timing of the tridiagonalisation's symmetric product: launches, seconds, bytes
 void symv_profiling(bool on);
 void symv_profile_stats(double* out);
+int launch_potrf_diag_list(hipStream_t s, int count, const int* list, const long* dOff,
+                           const long* orb0, double* work, int j, int* info);
 size_t potrf_inv_work(int n);
 int potrf_inverse_many(hipStream_t s, double* a, double* l, double* linv, int n, int K,
                        double* work, DevBuf<GemmDesc<double>>& desc, int* dInfo, int* hInfo);

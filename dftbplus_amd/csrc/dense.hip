@@ -252,12 +252,8 @@ constexpr int kPotrfNB = 64;
 // subtracts their products over the pivot. With the block in LDS and three barriers and a row of
 // divisions per column the kernel took 131 us; this form takes 42 us. Problem blockIdx.x of many is
 // found at strides sA, sV.
-__global__ __launch_bounds__(256) void potrf_diag_kernel(double* a, long lda, int jb,
-                                                         double* linv, long ldv, int offset,
-                                                         int* dInfo, long sA, long sV) {
-  a += blockIdx.x * sA;
-  if (linv) linv += blockIdx.x * sV;
-  dInfo += blockIdx.x;
+__device__ __forceinline__ void potrf_diag_block(double* a, long lda, int jb, double* linv,
+                                                 long ldv, int offset, int* dInfo) {
   constexpr int kLd = kPotrfNB + 1;
   static_assert(kPotrfNB == 64, "potrf_diag: 4 x 4 elements per thread");
   __shared__ double X[kPotrfNB * kLd];
@@ -321,6 +317,33 @@ __global__ __launch_bounds__(256) void potrf_diag_kernel(double* a, long lda, in
       const int i = e % jb, c = e / jb;
       linv[i + (long)c * ldv] = i >= c ? X[i * kLd + c] : 0.0;
     }
+}
+
+__global__ __launch_bounds__(256) void potrf_diag_kernel(double* a, long lda, int jb, double* linv,
+                                                         long ldv, int offset, int* dInfo, long sA,
+                                                         long sV) {
+  potrf_diag_block(a + blockIdx.x * sA, lda, jb, linv ? linv + blockIdx.x * sV : nullptr, ldv,
+                   offset, dInfo + blockIdx.x);
+}
+
+// Diagonal block j of the molecules in list: matrix at 3 dOff[m] of work, inverse two matrices on
+__global__ __launch_bounds__(256) void potrf_diag_list_kernel(const int* list, const long* dOff,
+                                                              const long* orb0, double* work,
+                                                              int j, int* info) {
+  const int m = list[blockIdx.x];
+  const long n = orb0[m + 1] - orb0[m];
+  if (j >= n) return;
+  double* a = work + 3 * dOff[m] + j + j * n;
+  potrf_diag_block(a, n, (int)min((long)kPotrfNB, n - j), a + 2 * n * n, n, j, info + m);
+}
+
+int launch_potrf_diag_list(hipStream_t s, int count, const int* list, const long* dOff,
+                           const long* orb0, double* work, int j, int* info) {
+  if (count <= 0) return 0;
+  hipLaunchKernelGGL(potrf_diag_list_kernel, dim3(count), dim3(256), 0, s, list, dOff, orb0, work,
+                     j, info);
+  DH_LAUNCH_CHECK();
+  return 0;
 }
 
 int potrf_lower_impl(hipStream_t s, double* a, long lda, int n, double* linv, long ldv,

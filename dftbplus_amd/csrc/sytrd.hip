@@ -142,7 +142,8 @@ struct SytrdWs {
 
 static int sytrd_slots(int n) {
   const int nRB = (n + kTB - 1) / kTB;
-  return nRB + nRB / kCHMin + 2;
+  // a column of tiles is worked out in at most half as many pieces, rounded up
+  return nRB + (nRB + kCHMin - 1) / kCHMin;
 }
 
 // byte layout of the workspace (each array 256-byte aligned)
