@@ -20,6 +20,7 @@
 #include <cstring>
 
 #include "common.h"
+#include "exchange_ring.h"
 #include "lanes.h"
 
 namespace dftbhip {
@@ -330,11 +331,12 @@ __global__ __launch_bounds__(64 * NW) void sytrd_wg_kernel(T* a, long lda, long 
 // written by the row's owner and polled by everyone (agent-scope 8-byte atomics, relaxed: each
 // word carries its own validity, kEmpty until it is written, so no fence and no counter is
 // needed). Three slots in turn. The thread that publishes row i sets the row's words of column
-// k - 1 back to kEmpty when its workgroup has gathered column k (then every workgroup has gathered
-// column k - 1), and waits for those stores before it publishes row i of column k + 1; a reader
-// polls row i of column k + 2, in that same slot, only after it has gathered row i of column
-// k + 1, so it can no longer meet the old words. A workgroup whose rows are
-// all reduced leaves. A wait is bounded; when one runs out the flag ends the others as well.
+// k - 1 back to kEmpty when its workgroup has gathered column k (then every workgroup has read
+// column k - 1, see ring_gathers), and waits for those stores before it publishes row i of column
+// k + 1; a reader polls row i of column k + 2, in that same slot, only after it has gathered row i
+// of column k + 1, so it can no longer meet the old words. A workgroup leaves when it has
+// published its last row: rows are not read after their column, so its own words may stay. A wait
+// is bounded; when one runs out the flag ends the others as well.
 // ---------------------------------------------------------------------------------------------
 constexpr u64 kEmpty = 0x7FF4D15EA5E0E5ADull;   // a signalling NaN that no operation returns
 
@@ -373,7 +375,7 @@ __global__ __launch_bounds__(NT) void sytrd_grid_kernel(T* a, long lda, long sA,
   tauOut += blockIdx.y * sV + c0;
   ring += blockIdx.y * sRing;
   const int m = n - c0;
-  const int lastRow = p + P * ((m - 1 - p) / P);
+  const int kGather = ring_gathers(ring_last_row(p, P, m), kEnd);
   double A[R][C], x[C], vp[C], wp[C];
   int own[C];   // slot of row j if this workgroup holds it
 #pragma unroll
@@ -470,85 +472,90 @@ __global__ __launch_bounds__(NT) void sytrd_grid_kernel(T* a, long lda, long sA,
     for (int u = 0; u < NG; ++u) {
       const int ps = min(4 * (wv + NW * u) + (lane >> 4), R - 1);
       const double y = part_total<NW>(sPart[lane & (NW - 1)][ps]);
-      if (prow[u] > k) {
+      if (ring_published(prow[u], k)) {
         put(ry + prow[u], word_of(y));
         put(ra + prow[u], word_of(sx[ps]));
       }
     }
-    // ---- gather y and the next column
-    u64 uy[C], ua[C];
-#pragma unroll
-    for (int q = 0; q < C; ++q) {
-      const int j = (int)t + NT * q;
-      uy[q] = j > k && j < m ? kEmpty : 0;   // 0.0 where there is nothing to gather
-      ua[q] = uy[q];
-    }
-    // Nothing can have arrived yet, and polls slow down the words on their way: at 1024 columns
-    // 4.6 us per column without this wait, 3.8 with 8 units of 64 clocks, 2.9 with 16 to 20, 3.2
-    // with 32.
-    __builtin_amdgcn_s_sleep(18);
-    for (long spins = 0;; ++spins) {
-      // the missing words, all loaded before the first is looked at: one trip to memory, not 2 C
+    const bool leaves = k == kGather;   // its last row is out
+    if (!leaves) {
+      // ---- gather y and the next column
+      u64 uy[C], ua[C];
 #pragma unroll
       for (int q = 0; q < C; ++q) {
-        if (uy[q] == kEmpty) uy[q] = get(ry + NT * q + t);
-        if (ua[q] == kEmpty) ua[q] = get(ra + NT * q + t);
+        const int j = (int)t + NT * q;
+        uy[q] = j > k && j < m ? kEmpty : 0;   // 0.0 where there is nothing to gather
+        ua[q] = uy[q];
       }
-      bool ok = true;
+      // Nothing can have arrived yet, and polls slow down the words on their way: at 1024
+      // columns 4.6 us per column without this wait, 3.8 with 8 units of 64 clocks, 2.9 with 16
+      // to 20, 3.2 with 32.
+      __builtin_amdgcn_s_sleep(18);
+      for (long spins = 0;; ++spins) {
+        // the missing words, all loaded before the first is looked at: one trip to memory, not 2 C
 #pragma unroll
-      for (int q = 0; q < C; ++q) ok = ok && uy[q] != kEmpty && ua[q] != kEmpty;
-      if (ok) break;
-      if ((spins & 1023) == 1023 || spins > spinLimit) {
-        if (spins > spinLimit)
-          __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-          sStop = 1;
-          break;
+        for (int q = 0; q < C; ++q) {
+          if (uy[q] == kEmpty) uy[q] = get(ry + NT * q + t);
+          if (ua[q] == kEmpty) ua[q] = get(ra + NT * q + t);
+        }
+        bool ok = true;
+#pragma unroll
+        for (int q = 0; q < C; ++q) ok = ok && uy[q] != kEmpty && ua[q] != kEmpty;
+        if (ok) break;
+        if ((spins & 1023) == 1023 || spins > spinLimit) {
+          if (spins > spinLimit)
+            __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          if (__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+            sStop = 1;
+            break;
+          }
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+      double y[C], an[C];
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        y[q] = __longlong_as_double((long long)uy[q]);
+        an[q] = __longlong_as_double((long long)ua[q]);
+      }
+      // ---- w and the next column
+      double dt = 0.0;
+#pragma unroll
+      for (int q = 0; q < C; ++q) {
+        const int j = (int)t + NT * q;
+        y[q] *= tau;
+        dt += y[q] * v[q];
+        if (j == k + 1) sB[2] = y[q];
+        if (own[q] >= 0) {
+          sv[own[q]] = v[q];
+          sw[own[q]] = y[q];
         }
       }
-      __builtin_amdgcn_s_sleep(1);
-    }
-    double y[C], an[C];
+      dt = wave_total(dt);
+      if (lane == 0) sD[wv] = dt;
+      lds_barrier();
+      if (sStop) return;
+      h = -0.5 * tau * part_total<NW>(sD[lane & (NW - 1)]);
+      const double wk = sB[2] + h;
 #pragma unroll
-    for (int q = 0; q < C; ++q) {
-      y[q] = __longlong_as_double((long long)uy[q]);
-      an[q] = __longlong_as_double((long long)ua[q]);
-    }
-    // ---- w and the next column
-    double dt = 0.0;
+      for (int q = 0; q < C; ++q) {
+        vp[q] = v[q];
+        wp[q] = y[q] + h * v[q];
+        x[q] = (int)t + NT * q > k ? an[q] - v[q] * wk - wp[q] : 0.0;
+      }
+      // this workgroup has gathered column k, so its words of column k - 1 are no longer needed
+      if (k > 0) {
+        u64* oy = ring + 2 * (slot == 0 ? kRingSlots - 1 : slot - 1) * mp;
 #pragma unroll
-    for (int q = 0; q < C; ++q) {
-      const int j = (int)t + NT * q;
-      y[q] *= tau;
-      dt += y[q] * v[q];
-      if (j == k + 1) sB[2] = y[q];
-      if (own[q] >= 0) {
-        sv[own[q]] = v[q];
-        sw[own[q]] = y[q];
+        for (int u = 0; u < NG; ++u)
+          if (ring_emptied(prow[u], k)) {
+            put(oy + prow[u], kEmpty);
+            put(oy + mp + prow[u], kEmpty);
+          }
       }
     }
-    dt = wave_total(dt);
-    if (lane == 0) sD[wv] = dt;
-    lds_barrier();
-    if (sStop) return;
-    h = -0.5 * tau * part_total<NW>(sD[lane & (NW - 1)]);
-    const double wk = sB[2] + h;
-#pragma unroll
-    for (int q = 0; q < C; ++q) {
-      vp[q] = v[q];
-      wp[q] = y[q] + h * v[q];
-      x[q] = (int)t + NT * q > k ? an[q] - v[q] * wk - wp[q] : 0.0;
-    }
-    // this workgroup has gathered column k, so its words of column k - 1 are no longer needed
-    if (k > 0) {
-      u64* oy = ring + 2 * (slot == 0 ? 2 : slot - 1) * mp;
-#pragma unroll
-      for (int u = 0; u < NG; ++u)
-        if (prow[u] >= k) {
-          put(oy + prow[u], kEmpty);
-          put(oy + mp + prow[u], kEmpty);
-        }
-    }
+    // ---- the column goes out, over what every workgroup has read into registers: it has
+    // published column k - 1 (or 0, which no workgroup leaves: it has four rows or more)
     if (p == (k + 1) % P) {
 #pragma unroll
       for (int q = 0; q < C; ++q) {
@@ -563,19 +570,8 @@ __global__ __launch_bounds__(NT) void sytrd_grid_kernel(T* a, long lda, long sA,
         tauOut[k] = (T)tau;
       }
     }
-    if (lastRow <= k + 1 && k + 1 < kEnd) return;
-    slot = slot == 2 ? 0 : slot + 1;
-  }
-  if (kEnd + 1 >= m) {
-    if (p == (m - 1) % P) {
-#pragma unroll
-      for (int q = 0; q < C; ++q)
-        if ((int)t + NT * q == m - 1) {
-          a[m - 1 + (long)(m - 1) * lda] = (T)x[q];
-          d[m - 1] = (T)x[q];
-        }
-    }
-    return;
+    if (leaves) return;
+    slot = slot == kRingSlots - 1 ? 0 : slot + 1;
   }
   // the trailing matrix goes back (lower triangle) for the one-workgroup kernel
 #pragma unroll
