@@ -37,20 +37,29 @@ __device__ __forceinline__ double pick(const double (&a)[N], int n, int k) {
 // Neville interpolation as polyInterU2 (interpolation.F90:182-239) on 8 uniform points
 // xa_i = (i0 + i) * dx, values y_i = tab[(i0 - 1 + i) * nint + col]. kMid: xx lies in the fourth
 // interval, as it does away from the ends of a table: the path through the tableau is then known
-// at compile time.
+// at compile time. Every rounding is written out (no contraction beyond the fma's here): past the
+// end of a table a second difference over 1e-5 divides by 1e-10, so that an ulp of a value is
+// 1e-11 in H0 and S there, whose last bits would otherwise change with the compiler's choice of
+// contractions, from kernel to kernel (and did: 8e-12, which a tail far from convergence made
+// 1e-4 of its charges).
 template <bool kDeriv, bool kMid>
 __device__ __forceinline__ double neville8(const double* tab, int nint, int col, int i0, double dx,
                                            double xx, int icl, double* dydx) {
-  double xa[8], cc[8], dd[8], cp[8], dp[8];
+#pragma clang fp contract(off)
+  double x[8], cc[8], dd[8], cp[8], dp[8], r2[8];   // x: xa_i - xx
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    xa[i] = (double)(i0 + i) * dx;
+    x[i] = fma((double)(i0 + i), dx, -xx);
     cc[i] = dd[i] = tab[(long)(i0 - 1 + i) * nint + col];
     cp[i] = dp[i] = 0.0;
   }
+  const double x0 = (double)i0 * dx;
   double delta[7];
 #pragma unroll
-  for (int i = 0; i < 7; ++i) delta[i] = 1.0 / (xa[i + 1] - xa[0]);
+  for (int i = 0; i < 7; ++i) {
+    const double h = i < 2 ? fma((double)(i0 + i + 1), dx, -x0) : (double)(i0 + i + 1) * dx - x0;
+    delta[i] = 1.0 / h;
+  }
   if (kMid) icl = 4;
   double yy = pick(cc, 8, icl - 1);
   double yp = 0.0;
@@ -59,15 +68,16 @@ __device__ __forceinline__ double neville8(const double* tab, int nint, int col,
   for (int mm = 1; mm < 8; ++mm) {
 #pragma unroll
     for (int ii = 0; ii < 8 - mm; ++ii) {
-      const double r2 = (dd[ii] - cc[ii + 1]) * delta[mm - 1];
+      const double diff = mm == 2 ? fma(r2[ii], x[ii + 1], -cc[ii + 1]) : dd[ii] - cc[ii + 1];
+      r2[ii] = diff * delta[mm - 1];
       if (kDeriv) {
         const double r2p = (dp[ii] - cp[ii + 1]) * delta[mm - 1];
         // derivative of c = (x_i - x) r2 and d = (x_{i+m} - x) r2
-        cp[ii] = -r2 + (xa[ii] - xx) * r2p;
-        dp[ii] = -r2 + (xa[ii + mm] - xx) * r2p;
+        cp[ii] = fma(x[ii], r2p, -r2[ii]);
+        dp[ii] = fma(x[ii + mm], r2p, -r2[ii]);
       }
-      cc[ii] = (xa[ii] - xx) * r2;
-      dd[ii] = (xa[ii + mm] - xx) * r2;
+      cc[ii] = x[ii] * r2[ii];
+      dd[ii] = x[ii + mm] * r2[ii];
     }
     const bool up = 2 * icl < 8 - mm;
     if (!up) icl -= 1;
@@ -80,8 +90,10 @@ __device__ __forceinline__ double neville8(const double* tab, int nint, int col,
 
 // the interval of xx among the points from i0 on, 1 .. 8
 __device__ __forceinline__ int neville_interval(int i0, double dx, double xx) {
-  const double x0 = (double)i0 * dx, x1 = (double)(i0 + 1) * dx;
-  const int icl = (int)ceil((xx - x0) * (1.0 / (x1 - x0)));
+#pragma clang fp contract(off)
+  const double x0 = (double)i0 * dx;
+  const int icl =
+      (int)ceil(fma(-(double)i0, dx, xx) * (1.0 / fma((double)(i0 + 1), dx, -x0)));
   return min(max(icl, 1), 8);
 }
 
@@ -89,7 +101,7 @@ __device__ __forceinline__ int neville_interval(int i0, double dx, double xx) {
 template <bool kDeriv>
 __device__ __forceinline__ double sk_integral(const double* tab, int nrows, int nint, int c,
                                               double dx, double r, double* d) {
-  const double rmax = nrows * dx + kDistFudge;
+  const double rmax = fma((double)nrows, dx, kDistFudge);
   const int ind = (int)floor(r / dx);
   if (kDeriv) *d = 0.0;
   if (r >= rmax) return 0.0;
@@ -101,12 +113,11 @@ __device__ __forceinline__ double sk_integral(const double* tab, int nrows, int 
                     : neville8<kDeriv, false>(tab, nint, c, ilast - 7, dx, r, icl, d);
   }
   const int i0 = nrows - 7;
-  const double x8 = nrows * dx;
   const double dr = r - rmax;
   double y[2];
 #pragma unroll 1
   for (int q = 0; q < 2; ++q) {
-    const double x = q == 0 ? x8 - kDeltaR : x8 + kDeltaR;
+    const double x = fma((double)nrows, dx, q == 0 ? -kDeltaR : kDeltaR);
     const double v =
         neville8<false, false>(tab, nint, c, i0, dx, x, neville_interval(i0, dx, x), nullptr);
     if (q == 0) y[0] = v;
