@@ -37,7 +37,8 @@ struct DevNeighbourList {
 
 // Builds the list for nat atoms at coords (host, 3 nat) with lattice lat (host, 9 doubles, or
 // null) and cutoff; blocks within skcut with norb orbitals per atom (host). Errors: atoms closer
-// than 0.01 bohr (kErrArg), more than 4096 neighbours of one atom (kErrArg).
+// than 0.01 bohr, coordinates or lattice vectors that are not finite, more than 4096 neighbours of
+// one atom (kErrArg each).
 int device_neighbours(hipStream_t s, int nat, const double* coords, const double* lat,
                       double cutoff, double skcut, const int* norb, DevNeighbourList& nl);
 

@@ -311,7 +311,7 @@ __device__ __forceinline__ void nl_visit(int a2, int nat, const NlGrid& g, const
       if (u >= pre[r]) q = start[r] + u - pre[r];
     const int pi = binItems[q];
     const double d2 = dist2_xyz(binX + 3 * (long)q, c2);
-    if (d2 > cut2) continue;
+    if (!(d2 <= cut2)) continue;   // nor has one that is no number
     const int t = pi / nat, a = pi - t * nat;
     if (a < a2) continue;
     if (d2 < kNlMinDist2) {
@@ -489,8 +489,19 @@ int device_neighbours(hipStream_t s, int nat, const double* coords, const double
                       double cutoff, double skcut, const int* norb, DevNeighbourList& nl) {
   DH_CHECK(nat >= 1 && coords && norb && cutoff > 0.0 && skcut <= cutoff,
            "neighbour list: bad arguments");
+  // a distance that is no number has no place in the sorted lists
+  for (int k = 0; k < 3 * nat; ++k)
+    if (!std::isfinite(coords[k])) {
+      set_error("neighbour list: coordinates of atom " + std::to_string(k / 3 + 1) +
+                " are not finite");
+      return kErrArg;
+    }
+  for (int k = 0; lat && k < 9; ++k)
+    DH_CHECK(std::isfinite(lat[k]), "neighbour list: lattice vectors are not finite");
   std::vector<double> tr;
   cell_translations(lat, cutoff, tr);
+  for (double x : tr)
+    DH_CHECK(std::isfinite(x), "neighbour list: lattice vectors out of range");
   const long ntr = (long)tr.size() / 3;
   const long P = ntr * nat;
   DH_CHECK(P < INT_MAX / 2, "neighbour list: too many candidate images");
