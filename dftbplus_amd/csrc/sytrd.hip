@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "symv_table.h"
 #include "tri_inverse.h"
 
 namespace dftbhip {
@@ -90,9 +91,9 @@ int set_symv_tiles(int tiles) {
 }
 
 // Tile choice by trailing size from the autotuner (symv_autotune), per arithmetic type
-// ([0] FP64, [1] FP32): rows (first trailing size, tiles) in ascending size; empty: shared out
-// evenly.
-static std::vector<std::pair<int, int>> g_tileTable[2];
+// ([0] FP64, [1] FP32): rows (first trailing size, tiles) in ascending size; empty, or 0 tiles:
+// shared out evenly.
+static TileTable g_tileTable[2];
 
 int clear_symv_tables() {
   g_tileTable[0].clear();
@@ -111,7 +112,7 @@ static int symv_tiles(int m, int K) {
     int v = t.front().second;
     for (const auto& r : t)
       if (mk >= r.first) v = r.second;
-    return v;
+    if (v > 0) return v;
   }
   const long nRB = (m + kTB - 1) / kTB, all = nRB * (nRB + 1) / 2 * K;
   return (int)std::max<long>(kCHMin, (all + kSymvSlots - 1) / kSymvSlots);
@@ -1003,14 +1004,12 @@ int sytrd_lower_f32(hipStream_t s, float* a, long lda, int n, float* d, float* e
 }
 // ---------------------------------------------------------------------------------------------
 // Autotuner of the SYMV tile count: the tridiagonalisation of a synthetic symmetric n x n matrix
-// is run once per tile option with every SYMV launch timed by HIP events; launches are grouped by
-// trailing size in buckets of kTuneBucket rows and each bucket takes the option of least summed
-// time, switching away from the option of the bucket below only for a gain of kTuneGain. The
-// result is installed as the tile table of the arithmetic type.
+// is run once per fixed tile count and once with the tiles shared out evenly, with every SYMV
+// launch timed by HIP events; launches are grouped by trailing size in buckets of kTuneBucket rows
+// and symv_choose picks from the summed times. Its table is installed for the arithmetic type.
+// 15769 rows, FP64, SYMV of one tridiagonalisation: even share 1.118 s, the fastest fixed count of
+// each bucket 1.140 s; 4000 rows: 27.4 and 25.3 ms.
 // ---------------------------------------------------------------------------------------------
-constexpr int kTuneBucket = 256;
-constexpr int kTuneOptions[4] = {2, 4, 8, 16};
-constexpr double kTuneGain = 0.02;
 
 // lower triangle of a symmetric matrix from a hash of (i, j): values in [-1, 1), diagonal
 // shifted by i / n
@@ -1030,8 +1029,7 @@ __global__ void synth_sym_kernel(T* a, long lda, int n) {
 }
 
 template <typename T>
-static int symv_autotune_t(hipStream_t s, int n, std::vector<std::pair<int, int>>& rows,
-                           std::vector<double>* detail) {
+static int symv_autotune_t(hipStream_t s, int n, TileTable& rows, std::vector<double>* detail) {
   DH_CHECK(n >= kTuneBucket && n <= 65535, "autotune: n must be in [256, 65535]");
   DevBuf<T> a, d, e, tau;
   DevBuf<char> work;
@@ -1042,15 +1040,18 @@ static int symv_autotune_t(hipStream_t s, int n, std::vector<std::pair<int, int>
   const size_t wb = sytrd_layout<T>(n, nullptr, nullptr);
   DH_TRY(work.alloc(wb));
   const int nb = (n + kTuneBucket - 1) / kTuneBucket;
-  std::vector<double> t(4 * (size_t)nb, 0.0);
+  std::vector<double> t((kTuneFixed + 1) * (size_t)nb, 0.0);
   std::vector<std::pair<int, float>> rec;
   SymvProfile& pf = g_symvProf;
   const bool on0 = pf.on;
   const double l0 = pf.launches, s0 = pf.seconds, b0 = pf.algBytes;
   const int tiles0 = g_symvTiles;
   int rc = 0;
-  for (int o = 0; o < 4 && rc == 0; ++o) {
-    g_symvTiles = kTuneOptions[o];
+  TileTable& table = g_tileTable[std::is_same<T, float>::value ? 1 : 0];
+  TileTable before;
+  before.swap(table);
+  for (int o = 0; o <= kTuneFixed && rc == 0; ++o) {
+    g_symvTiles = o < kTuneFixed ? kTuneOptions[o] : 0;
     ++g_tileGen;
     // untimed pass on a small matrix first: the option's kernels are loaded before timing
     for (int nn : {kTuneBucket, n}) {
@@ -1077,24 +1078,14 @@ static int symv_autotune_t(hipStream_t s, int n, std::vector<std::pair<int, int>
   pf.seconds = s0;
   pf.algBytes = b0;
   pf.sink = nullptr;
-  if (rc) return rc;
-  DH_HIP(hipStreamSynchronize(s));
-  // a bucket keeps the option of the bucket below unless another is kTuneGain faster there
-  // (buckets of small trailing sizes are launch bound and differ by noise only)
-  rows.clear();
-  int cur = -1;
-  for (int b = 0; b < nb; ++b) {
-    int best = 0;
-    for (int o = 1; o < 4; ++o)
-      if (t[(size_t)o * nb + b] < t[(size_t)best * nb + b]) best = o;
-    if (cur < 0 || t[(size_t)best * nb + b] < (1.0 - kTuneGain) * t[(size_t)cur * nb + b]) {
-      if (best != cur) rows.push_back({b * kTuneBucket, kTuneOptions[best]});
-      cur = best;
-    }
+  if (rc) {
+    table.swap(before);
+    return rc;
   }
-  rows.front().first = 0;
+  DH_HIP(hipStreamSynchronize(s));
+  symv_choose(t, nb, &rows, &table);
+  t.resize(kTuneFixed * (size_t)nb);
   if (detail) *detail = t;
-  g_tileTable[std::is_same<T, float>::value ? 1 : 0] = rows;
   ++g_tileGen;
   return 0;
 }

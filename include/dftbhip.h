@@ -102,11 +102,12 @@ int dftbhip_neighbour_list(int nAtom, const double* coords, const double* latVec
                            int* nAll, int* mNeighbour, double* coordsAll, int* img2CentCell,
                            int* iNeighbour, int* nNeighbour, double* neighDist2);
 /* Autotuner of the SYMV tile count (no counterpart in the reference): tridiagonalises a
- * synthetic symmetric n x n matrix (256 <= n <= 65535) once per option 2, 4, 8, 16 with every
- * SYMV launch timed, picks per 256-row bucket of trailing sizes the option of least time
- * (keeping the option of the bucket below unless another is at least 2 % faster) and
- * installs the result for precision 0 (FP64) or 1 (FP32). table: up to maxRows rows
- * (first trailing size, tiles), ascending; *nRows: rows in the installed table. detail
+ * synthetic symmetric n x n matrix (256 <= n <= 65535) once per option 2, 4, 8, 16 and once
+ * with the tiles shared out evenly (the default) with every SYMV launch timed, picks per 256-row
+ * bucket of trailing sizes the option of least time (keeping the option of the bucket below
+ * unless another is at least 2 % faster) and installs the result for precision 0 (FP64) or 1
+ * (FP32); buckets whose option is not 2 % faster than the even share keep that. table: up to
+ * maxRows rows (first trailing size, tiles), ascending; *nRows: rows of the options. detail
  * (optional, detailLen doubles): summed seconds, option-major: detail[o * nb + b] for option
  * o and bucket b, nb = ceil(n / 256). Allocates device memory for the test matrix. */
 int dftbhip_autotune(int n, int precision, int* table, int maxRows, int* nRows, double* detail,
