@@ -531,9 +531,10 @@ __global__ void secular_kernel(const MergeDev* md, DcArrays A) {
   const double noise = eps * (4.0 + 0.25 * sqrt((double)k));
   for (int it = 0; it < 80; ++it) {
     const double w = 1.0 + f.psi + f.phi;
-    if (fabs(w) <= noise * (1.0 + fabs(f.psi) + fabs(f.phi)) +
-                       2.0 * eps * fabs(tau) * (f.dpsi + f.dphi))
-      break;
+    const double tol = noise * (1.0 + fabs(f.psi) + fabs(f.phi)) +
+                       2.0 * eps * fabs(tau) * (f.dpsi + f.dphi);
+    // closer than about 1e-154 to a pole, where the halving may take tau, the slopes overflow
+    if (fabs(w) <= tol && tol < HUGE_VAL) break;
     if (w < 0.0) lo = tau;
     else hi = tau;
     // neighbours in the floating-point numbers: nothing lies between
