@@ -76,7 +76,7 @@ struct StedcWs {
   DevBuf<MergeDev> dmerge;
   DevBuf<ProblemDev> dproblem;
   DevBuf<GemmDesc<double>> ddesc;
-  DevBuf<double> darr;                    // double arrays of length `total`
+  DevBuf<double> darr;                    // double arrays of length `total`, then the scales
   DevBuf<int> iarr;                       // int arrays of length `total`, then the info words
   DevBuf<double> dd, de;                  // uploads of the host interface
   int* info = nullptr;
@@ -90,6 +90,7 @@ struct DcArrays {
   double *D, *z, *DL, *W, *tau, *lam, *zhat, *dval, *rc, *rs;
   int *ord, *idx, *cand, *flag, *type, *org, *row, *gcol, *dcol, *rp, *rn;
   int* info;   // per problem: not 0 when it failed; its merges and output are then skipped
+  double* scale;   // per problem: the power of two its elements are multiplied by
 };
 constexpr int kDcDoubles = 10, kDcInts = 11;
 
@@ -125,13 +126,14 @@ __global__ __launch_bounds__(64) void leaf_kernel(const double* dIn, const doubl
   const LeafDev L = leaves[blockIdx.x];
   const int m = L.m, t = threadIdx.x;
   if (A.info[L.prob] < 0) return;
+  const double sc = A.scale[L.prob];
   if (t < m) {
-    double v = dIn[L.s + t];
+    double v = sc * dIn[L.s + t];
     // the tears on both sides of the leaf
-    if (t == 0 && L.c0 > 0) v -= fabs(eIn[L.s - 1]);
-    if (t == m - 1 && L.c0 + m < L.n) v -= fabs(eIn[L.s + m - 1]);
+    if (t == 0 && L.c0 > 0) v -= fabs(sc * eIn[L.s - 1]);
+    if (t == m - 1 && L.c0 + m < L.n) v -= fabs(sc * eIn[L.s + m - 1]);
     d[t] = v;
-    e[t] = t < m - 1 ? eIn[L.s + t] : 0.0;
+    e[t] = t < m - 1 ? sc * eIn[L.s + t] : 0.0;
   }
   const int row = min(t, kLeaf - 1);       // lanes past the leaf repeat a row nobody reads
   if (t < kLeaf)
@@ -139,7 +141,7 @@ __global__ __launch_bounds__(64) void leaf_kernel(const double* dIn, const doubl
   __syncthreads();
   const double eps = 2.220446049250313e-16;
   // values that are no numbers would leave the lists of the merges incomplete
-  const bool finite = t >= m || (fabs(d[t]) < 1e300 && fabs(e[t]) < 1e300);
+  const bool finite = t >= m || (fabs(d[t]) < HUGE_VAL && fabs(e[t]) < HUGE_VAL);
   int fail = __ballot(!finite) != 0;
   for (int l = 0; l < m && !fail; ++l) {
     for (int iter = 0;; ++iter) {
@@ -268,7 +270,7 @@ __global__ __launch_bounds__(kDefT) void deflate_kernel(MergeDev* md, const doub
     }
     return;
   }
-  const double b = eIn[s + n1 - 1];
+  const double b = A.scale[m.prob] * eIn[s + n1 - 1];
   const double rho = 2.0 * fabs(b), sigma = b >= 0.0 ? 1.0 : -1.0;
   const double isq2 = 0.70710678118654752440;
   const double eps = 2.220446049250313e-16;
@@ -677,20 +679,42 @@ __global__ void collect_kernel(const ProblemDev* pr, const double* Qa, const dou
   const int c = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, lane = threadIdx.x & 63;
   if (c >= p.n || A.info[blockIdx.y] != 0) return;
   const int col = A.ord[p.s + c];
-  if (lane == 0) w[p.s + c] = A.D[col];
+  if (lane == 0) w[p.s + c] = A.D[col] / A.scale[blockIdx.y];   // a power of two
   const double* src = (p.parity ? Qb : Qa) + p.q + (long)(col - p.s) * p.n;
   double* dst = z + p.z + (long)c * p.ldz;
   for (int r = lane; r < p.n; r += 64) dst[r] = src[r];
 }
 
-// zeros, and the state of each problem: to be solved, or (-1) left as it is
-__global__ void stedc_zero_kernel(double* q, size_t n, const ProblemDev* pr, const int* active,
-                                  int* info, int ninfo) {
-  const size_t stride = (size_t)gridDim.x * blockDim.x;
-  size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (size_t k = i; k < (size_t)ninfo; k += stride)
-    info[k] = active && !active[pr[k].id] ? -1 : 0;
-  for (; i < n; i += stride) q[i] = 0.0;
+// Zeros, and for each problem its state, to be solved or (-1) left as it is, and its scale. The
+// deflation is to eps times the larger of the levels and z, so a matrix is scaled to a norm of at
+// least 1/2 (LAPACK: to 1), and so that its squares stay in range.
+constexpr int kZeroT = 256;
+__global__ __launch_bounds__(kZeroT) void stedc_zero_kernel(double* q, size_t n,
+                                                            const ProblemDev* pr,
+                                                            const int* active, const double* d,
+                                                            const double* e, int nprob,
+                                                            int* info, double* scale) {
+  __shared__ double part[kZeroT / 64];
+  for (int k = blockIdx.x; k < nprob; k += gridDim.x) {
+    const ProblemDev p = pr[k];
+    double v = 0.0;
+    for (int c = threadIdx.x; c < p.n; c += kZeroT) {
+      v = fmax(v, fabs(d[p.s + c]));
+      if (c + 1 < p.n) v = fmax(v, fabs(e[p.s + c]));
+    }
+    for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
+    __syncthreads();   // the last use of part
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 0; w < kZeroT / 64; ++w) v = fmax(v, part[w]);
+      const bool asIs = v == 0.0 || (v >= 0.5 && v < 1e100) || !(v < HUGE_VAL);
+      scale[k] = asIs ? 1.0 : ldexp(1.0, max(-1000, min(1000, -ilogb(v))));
+      info[k] = active && !active[p.id] ? -1 : 0;
+    }
+  }
+  const size_t stride = (size_t)gridDim.x * kZeroT;
+  for (size_t i = (size_t)blockIdx.x * kZeroT + threadIdx.x; i < n; i += stride) q[i] = 0.0;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -773,7 +797,7 @@ static int dc_tables(hipStream_t s, StedcWs& W, const std::vector<DcBlock>& bloc
   if (!W.merges.empty()) DH_TRY(W.dmerge.upload(W.merges.data(), W.merges.size(), s));
   DH_TRY(W.dproblem.upload(W.problems.data(), W.problems.size(), s));
   DH_TRY(W.ddesc.alloc(std::max<size_t>(2 * W.merges.size(), 1)));
-  DH_TRY(W.darr.alloc((size_t)kDcDoubles * W.total));
+  DH_TRY(W.darr.alloc((size_t)kDcDoubles * W.total + blocks.size()));
   DH_TRY(W.iarr.alloc((size_t)kDcInts * W.total + blocks.size()));
   W.info = W.iarr.p + (size_t)kDcInts * W.total;
   W.blocks = blocks;
@@ -793,6 +817,7 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
     for (int i = 0; i < kDcDoubles; ++i) *dp[i] = W.darr.p + (size_t)i * W.total;
     for (int i = 0; i < kDcInts; ++i) *ip[i] = W.iarr.p + (size_t)i * W.total;
     A.info = W.info;
+    A.scale = W.darr.p + (size_t)kDcDoubles * W.total;
   }
   const size_t sq = W.totalSq;
   double* Q[2] = {work, work + sq};
@@ -801,7 +826,8 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
   // zeros outside the blocks of the leaves; the second buffer's blocks are written whole, its
   // zeros outside them are read by the next height
   hipLaunchKernelGGL(stedc_zero_kernel, dim3((unsigned)std::min<size_t>(cdiv(2 * sq, 1024), 2048)),
-                     dim3(256), 0, s, work, 2 * sq, W.dproblem.p, active, W.info, (int)W.problems.size());
+                     dim3(kZeroT), 0, s, work, 2 * sq, W.dproblem.p, active, d, e,
+                     (int)W.problems.size(), A.info, A.scale);
   DH_LAUNCH_CHECK();
   hipLaunchKernelGGL(leaf_kernel, dim3((unsigned)W.leaves.size()), dim3(64), 0, s, d, e, W.dleaf.p,
                      Q[0], A);
@@ -833,6 +859,7 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
   for (size_t p = 0; p < W.problems.size(); p += kRows) {
     DcArrays Ap = A;
     Ap.info += p;
+    Ap.scale += p;
     hipLaunchKernelGGL(collect_kernel, dim3(cdiv((long)W.maxProblem * 64, 256),
                                             (unsigned)std::min<size_t>(kRows, W.problems.size() - p)),
                        dim3(256), 0, s, W.dproblem.p + p, Q[0], Q[1], w, z, Ap);
