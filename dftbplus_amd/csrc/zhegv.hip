@@ -252,17 +252,27 @@ __device__ inline double block_sum(double v, double* red) {
 // One cluster of m levels (pairs j0 .. j0+m-1) per workgroup: its 2m embedded eigenvectors
 // (columns 2 j0 ...) as complex vectors, Gram-Schmidt (twice) against the accepted ones in
 // eigenvalue order, accepted when the remaining norm exceeds 1/2 (the candidates have norm 1),
-// until m are accepted. The candidate is staged in work (2n doubles per cluster).
+// until m are accepted. The squared remaining norms of all 2 m sum to 2 (m - accepted), so in a
+// large cluster the last ones may be less: the candidates are gone through again with half the
+// norm, at the latest down to 1 / sqrt(m), and take their places by eigenvalue (taken: candidate
+// of each accepted vector, from j0 on). The candidate is staged in work (2n doubles per cluster).
 __global__ __launch_bounds__(256) void cluster_gs_kernel(const double* z, long ldz, int n,
                                                          const int* clusters, double* yr,
                                                          double* yi, long ldy, double* work,
-                                                         int* failed) {
+                                                         int* taken, int* failed) {
   __shared__ double red[4];
   const int j0 = clusters[2 * blockIdx.x], m = clusters[2 * blockIdx.x + 1];
   double* vr = work + (long)blockIdx.x * 2 * n;
   double* vi = vr + n;
+  taken += j0;
   int accepted = 0;
-  for (int t = 0; t < 2 * m && accepted < m; ++t) {
+  double least = 0.5;
+  for (int c = 0; accepted < m; ++c) {
+    const int t = c % (2 * m);
+    if (c > 0 && t == 0) {
+      if (least * least * m < 1.0) break;
+      least *= 0.5;
+    }
     const double* col = z + (long)(2 * j0 + t) * ldz;
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
       vr[i] = col[i];
@@ -290,12 +300,21 @@ __global__ __launch_bounds__(256) void cluster_gs_kernel(const double* z, long l
     double nr = 0.0;
     for (int i = threadIdx.x; i < n; i += blockDim.x) nr += vr[i] * vr[i] + vi[i] * vi[i];
     nr = sqrt(block_sum(nr, red));
-    if (nr > 0.5) {
-      double* orr = yr + (long)(j0 + accepted) * ldy;
-      double* oi = yi + (long)(j0 + accepted) * ldy;
+    if (nr > least) {
+      int at = accepted;   // its place: later candidates than t move up by one
+      while (at > 0 && taken[at - 1] > t) --at;
       for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        orr[i] = vr[i] / nr;
-        oi[i] = vi[i] / nr;
+        for (int a = accepted; a > at; --a) {
+          yr[i + (long)(j0 + a) * ldy] = yr[i + (long)(j0 + a - 1) * ldy];
+          yi[i + (long)(j0 + a) * ldy] = yi[i + (long)(j0 + a - 1) * ldy];
+        }
+        yr[i + (long)(j0 + at) * ldy] = vr[i] / nr;
+        yi[i + (long)(j0 + at) * ldy] = vi[i] / nr;
+      }
+      __syncthreads();   // everyone has found the place
+      if (threadIdx.x == 0) {
+        for (int a = accepted; a > at; --a) taken[a] = taken[a - 1];
+        taken[at] = t;
       }
       ++accepted;
     }
@@ -405,13 +424,14 @@ int ZhegvSolver::solve(hipStream_t s, const double* aDev, long lda, const double
   }
   nClusters = (int)cl.size() / 2;
   if (nClusters > 0) {
-    DH_TRY(clusterDev.alloc(cl.size()));
+    DH_TRY(clusterDev.alloc(cl.size() + n));
     DH_HIP(hipMemcpyAsync(clusterDev.p, cl.data(), cl.size() * sizeof(int),
                           hipMemcpyHostToDevice, s));
     DH_TRY(fill<int>(s, dinfo.p + 1, 1, 0));
     DH_CHECK((size_t)nClusters * 2 * n <= workSize, "hegvd: cluster workspace too small");
     hipLaunchKernelGGL(cluster_gs_kernel, dim3(nClusters), dim3(256), 0, s, Z2.p, (long)n2, n,
-                       clusterDev.p, Y.r, Y.i, ld, work.p, dinfo.p + 1);
+                       clusterDev.p, Y.r, Y.i, ld, work.p, clusterDev.p + cl.size(),
+                       dinfo.p + 1);
     DH_LAUNCH_CHECK();
     int failed = 0;
     DH_HIP(hipMemcpyAsync(&failed, dinfo.p + 1, sizeof(int), hipMemcpyDeviceToHost, s));
