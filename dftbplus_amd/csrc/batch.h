@@ -12,10 +12,13 @@ namespace dftbhip {
 constexpr int kBatchMaxOrb = 512;   // orbitals per molecule in a batch
 // size classes of the batched eigensolver, by orbital count (largest first): above kWgBatchMax
 // Jacobi with both matrices in HBM, up to it the direct solve, whose reduction has shapes for
-// 224, 192, 128, 64 and 32 orbitals
-constexpr int kBatchClasses = 6;
+// 224, 192, 128, 64 and 32 orbitals, and up to kBatchSmall Jacobi in LDS
+constexpr int kBatchSmall = 16;
+constexpr int kBatchJacobi = 6;   // the class of the smallest
+constexpr int kBatchClasses = 7;
 inline int batch_class(long n) {
-  return n > kWgBatchMax ? 0 : n > 192 ? 1 : n > 128 ? 2 : n > 64 ? 3 : n > 32 ? 4 : 5;
+  return n > kWgBatchMax ? 0 : n > 192 ? 1 : n > 128 ? 2 : n > 64 ? 3 : n > 32 ? 4
+         : n > kBatchSmall ? 5 : kBatchJacobi;
 }
 // info of a molecule whose eigensolver did not converge within its limit (distinct from the
 // leading minor of a non-positive-definite overlap)
@@ -50,7 +53,8 @@ struct FactorStep {
 struct BatchEigen {
   int first[kBatchClasses + 1] = {}, maxn[kBatchClasses] = {}, direct = 0;
   std::shared_ptr<StedcWs> dc;
-  DevBuf<double> work, d, e, tau;
+  DevBuf<double> work, vec;
+  double *d = nullptr, *e = nullptr, *tau = nullptr;   // in vec
   DevBuf<GemmDesc<double>> desc, factorDesc;
   std::vector<FactorStep> steps;
   DevBuf<int> solve;
@@ -59,7 +63,7 @@ struct BatchEigen {
               double* C);
   int maxDirect() const {
     int n = 0;
-    for (int c = 1; c < kBatchClasses; ++c) n = n > maxn[c] ? n : maxn[c];
+    for (int c = 1; c < kBatchJacobi; ++c) n = n > maxn[c] ? n : maxn[c];
     return n;
   }
 };
@@ -67,13 +71,13 @@ struct BatchEigen {
 // (0, or j+1 when the leading minor j+1 of S is not positive definite); work 3 x packed size,
 // kept between calls. Molecules with active[m] == 0 are skipped (active may be null: all).
 // warm: S is the one of the previous call on the same work array (a cold call factors S; the
-// Jacobi sweeps of large molecules then start from that call's eigenvectors).
-// st[0]: the stream of the call, st[1 .. kBatchClasses-1]: streams forked from it by the caller
+// Jacobi sweeps of the largest and smallest molecules then start from that call's eigenvectors).
+// s: the stream of the call; st[c]: that of class c, s itself or one forked from it by the caller
 // and joined afterwards; done[0 .. kBatchClasses-1]: events for the forks in between. Launches
 // only, so a call can be captured.
-int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L, const double* S,
-                      const double* H, double* work, double* w, double* C, int* info,
-                      const int* active, bool warm, hipEvent_t* done);
+int launch_batch_sygv(hipStream_t s, const hipStream_t* st, BatchEigen& E, const BatchLayout& L,
+                      const double* S, const double* H, double* work, double* w, double* C,
+                      int* info, const int* active, bool warm, hipEvent_t* done);
 // P = C diag(f) C^T over the first nocc columns; work as above (B1 is overwritten)
 int launch_batch_density(hipStream_t s, BatchEigen& E, const BatchLayout& L, const double* C,
                          const double* f, const int* nocc, double* P, const int* active,

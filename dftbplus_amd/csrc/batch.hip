@@ -448,7 +448,190 @@ __global__ __launch_bounds__(kSygvThreads) void batch_sygv_kernel(BatchLayout L,
 }
 
 // ------------------------------------------------------------------------------------------
-// Direct eigensolver for molecules of up to kWgBatchMax orbitals: L^-1 once per geometry (panels
+// The same for the smallest molecules with A (upper triangle packed by columns: (i, j), i <= j, at
+// i + j (j + 1) / 2) and C in LDS, the whole solve in one launch. The direct solve takes ten, so
+// up to kBatchSmall orbitals the sweeps are faster: per iteration of one molecule of 8 to 16
+// orbitals 191 against 215 us, of 1024 378 against 403 us; of 17 to 24 orbitals 206 against
+// 223 us for one but 572 against 525 us for 1024.
+// ------------------------------------------------------------------------------------------
+__device__ __forceinline__ int sym_idx(int i, int j) {
+  return i <= j ? i + j * (j + 1) / 2 : j + i * (i + 1) / 2;
+}
+
+__global__ __launch_bounds__(kSygvThreads) __attribute__((amdgpu_waves_per_eu(8)))
+void batch_sygv_small_kernel(BatchLayout L, const int* list, const double* S, const double* H,
+                             double* work, double* w, double* C, int* info, const int* active,
+                             int warm) {
+  constexpr int NT = kSygvThreads, kMaxN = kBatchSmall;
+  constexpr int kPacked = kMaxN * (kMaxN + 1) / 2;
+  constexpr int kStage = 2 * kGK * (kGT + 1);   // also the staging of the products
+  __shared__ double As[kPacked > kStage ? kPacked : kStage];
+  __shared__ double Cs[kMaxN * kMaxN];
+  __shared__ double rc[kMaxN / 2], rs[kMaxN / 2];
+  __shared__ int rp[kMaxN / 2], rq[kMaxN / 2];
+  __shared__ int perm[kMaxN];
+  __shared__ int nrot, need;
+  __shared__ unsigned long long dmaxBits;
+  const int m = list[blockIdx.x];
+  if (active && !active[m]) return;   // converged: eigenpairs stay from the last pass
+  const int tid = threadIdx.x;
+  const long base = L.dOff[m];
+  const int n = (int)(L.orb0[m + 1] - L.orb0[m]);
+  if (n > kMaxN) return;   // not of this class
+  const long nn = (long)n * n;
+  double* B0 = work + 3 * base;
+  double* B1 = B0 + nn;
+  double* Cw = B1 + nn;
+  if (!warm) {
+    if (!wg_factor(n, S + base, B0, Cw, info + m)) return;
+  }
+  double (*Xs)[kGT + 1] = reinterpret_cast<double (*)[kGT + 1]>(As);
+  double (*Ys)[kGT + 1] = reinterpret_cast<double (*)[kGT + 1]>(As + kGK * (kGT + 1));
+  wg_gemm<false, false>(n, n, H + base, Cw, nullptr, B1, Xs, Ys);
+  wg_gemm<true, false>(n, n, Cw, B1, nullptr, B0, Xs, Ys);
+  // A (symmetrized) into LDS
+  for (long e = tid; e < nn; e += NT) {
+    const int i = (int)(e % n), j = (int)(e / n);
+    if (i <= j) As[i + j * (j + 1) / 2] = 0.5 * (B0[i + (long)j * n] + B0[j + (long)i * n]);
+    Cs[e] = Cw[e];
+  }
+  __syncthreads();
+  auto lds_barrier = [&]() {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0); vmcnt, expcnt untouched (gfx9 encoding)
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  };
+  const int N2 = n + (n & 1);
+  const int np = N2 / 2;
+  const int nunit = np * (np + 1) / 2;
+  const int npair = n * (n - 1) / 2;
+  // rounding level of the matrix: 4 eps max |a_ii| (bits of non-negative doubles order as
+  // unsigned integers, so the maximum is an integer atomic)
+  if (tid == 0) dmaxBits = 0ull;
+  __syncthreads();
+  {
+    double dm = 0.0;
+    for (int i = tid; i < n; i += NT) dm = fmax(dm, fabs(As[sym_idx(i, i)]));
+    atomicMax(&dmaxBits, (unsigned long long)__double_as_longlong(dm));
+  }
+  __syncthreads();
+  const double rotFloor = 4.0 * 2.220446049250313e-16 * __longlong_as_double((long long)dmaxBits);
+  bool done = n <= 1;
+  for (int sweep = 0; sweep < kJacobiMaxSweeps && n > 1; ++sweep) {
+    // a sweep in which no pair passes the rotation test changes nothing: test all pairs first
+    if (tid == 0) {
+      nrot = 0;
+      need = 0;
+    }
+    lds_barrier();
+    for (int u = tid; u < npair; u += NT) {
+      int k1, k2;
+      unit_pairs(u, k1, k2);
+      const int p = k1, q = k2 + 1;
+      const double apq = As[sym_idx(p, q)];
+      const double app = As[sym_idx(p, p)], aqq = As[sym_idx(q, q)];
+      if (jacobi_rotates(apq, app, aqq, rotFloor)) need = 1;
+    }
+    lds_barrier();
+    if (need == 0) {
+      done = true;
+      break;
+    }
+    for (int r = 0; r < N2 - 1; ++r) {
+      for (int k = tid; k < np; k += NT) {
+        int p, q;
+        jacobi_pair(N2, r, k, p, q);
+        double c = 1.0, s = 0.0;
+        if (p < n && q < n) {
+          const double apq = As[sym_idx(p, q)];
+          const double app = As[sym_idx(p, p)], aqq = As[sym_idx(q, q)];
+          if (jacobi_rotates(apq, app, aqq, rotFloor)) {
+            const double th = (aqq - app) / (2.0 * apq);
+            const double t = copysign(1.0, th) / (fabs(th) + sqrt(th * th + 1.0));
+            c = 1.0 / sqrt(t * t + 1.0);
+            s = t * c;
+            atomicAdd(&nrot, 1);
+          }
+        }
+        rp[k] = p;
+        rq[k] = q;
+        rc[k] = c;
+        rs[k] = s;
+      }
+      lds_barrier();
+      // A <- J^T A J over the unordered 2 x 2 blocks (pairs k1 <= k2)
+      for (int u = tid; u < nunit; u += NT) {
+        int k1, k2;
+        unit_pairs(u, k1, k2);
+        const double s1 = rs[k1], s2 = rs[k2];
+        if (s1 == 0.0 && s2 == 0.0) continue;
+        const double c1 = rc[k1], c2 = rc[k2];
+        const int row[2] = {rp[k1], rq[k1]}, col[2] = {rp[k2], rq[k2]};
+        double x[4];
+        int o[4];
+        bool v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int ri = row[e & 1], ci = col[e >> 1];
+          v[e] = ri < n && ci < n;
+          o[e] = v[e] ? sym_idx(ri, ci) : 0;
+          x[e] = v[e] ? As[o[e]] : 0.0;
+        }
+        // e = 0 (p1, p2), 1 (q1, p2), 2 (p1, q2), 3 (q1, q2); columns first
+        const double y0 = c2 * x[0] - s2 * x[2];
+        const double y1 = c2 * x[1] - s2 * x[3];
+        const double y2 = s2 * x[0] + c2 * x[2];
+        const double y3 = s2 * x[1] + c2 * x[3];
+        const double z[4] = {c1 * y0 - s1 * y1, s1 * y0 + c1 * y1, c1 * y2 - s1 * y3,
+                             s1 * y2 + c1 * y3};
+        if (k1 == k2) {
+          // (p, p), (q, q) and the shared off-diagonal element
+          if (v[0]) As[o[0]] = z[0];
+          if (v[3]) As[o[3]] = z[3];
+          if (v[2]) As[o[2]] = z[2];
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (v[e]) As[o[e]] = z[e];
+        }
+      }
+      rotate_columns<8>(Cs, n, np, rp, rq, rc, rs);
+      lds_barrier();
+    }
+    const int nr = nrot;
+    lds_barrier();   // every thread has read nrot before the next sweep clears it
+    if (nr == 0) {
+      done = true;
+      break;
+    }
+  }
+  __syncthreads();   // every column of C written before other threads read it
+  double* wm = w + L.orb0[m];
+  for (int i = tid; i < n; i += NT) {
+    const double di = As[sym_idx(i, i)];
+    int rank = 0;
+    for (int j = 0; j < n; ++j) {
+      const double dj = As[sym_idx(j, j)];
+      rank += (dj < di || (dj == di && j < i)) ? 1 : 0;
+    }
+    perm[rank] = i;
+    wm[rank] = di;
+  }
+  __syncthreads();
+  double* Cm = C + base;
+  for (long e = tid; e < nn; e += NT) {
+    const int i = (int)(e % n), c = (int)(e / n);
+    Cm[e] = Cs[i + perm[c] * n];
+    Cw[e] = Cs[e];   // the next warm call starts from the rotated C
+  }
+  // a molecule whose last allowed sweep still rotated is reported (info > 0), not taken as
+  // converged
+  if (tid == 0) info[m] = done ? 0 : kBatchEigenNoConv;
+}
+
+// ------------------------------------------------------------------------------------------
+// Direct eigensolver for the other molecules of up to kWgBatchMax orbitals: L^-1 once per geometry (panels
 // of 64 columns, every launch for all molecules that reach its panel; one workgroup per molecule
 // in HBM took 2.1 ms for 190 orbitals), then per call A = L^-1 H L^-T (batched MFMA GEMMs),
 // tridiagonalisation with the matrix in the registers of one workgroup (sytrd_resident.hip),
@@ -675,18 +858,20 @@ int launch_batch_pack(hipStream_t s, const PairsDev& pr, const int* norb, const 
 int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<int>& order,
                         const std::vector<long>& orb0, const std::vector<long>& dOff,
                         double* matrices, double* C) {
-  int nDirect = 0;
   first[0] = 0;
   for (int c = 0; c < kBatchClasses; ++c) {
     first[c + 1] = first[c] + L.ncls[c];
     maxn[c] = L.ncls[c] > 0
                   ? (int)(orb0[order[first[c]] + 1] - orb0[order[first[c]]])   // largest first
                   : 0;
-    if (c > 0) nDirect += L.ncls[c];
   }
   DH_CHECK(first[kBatchClasses] == L.nmol, "batch_sygv: size classes do not cover the batch");
+  direct = first[kBatchJacobi] - first[1];
+  DH_TRY(desc.alloc(4 * (size_t)std::max(L.nmol, 1)));
+  if (direct == 0) return 0;
+  const int end = first[kBatchJacobi];
   std::vector<DcBlock> blocks;
-  for (int t = first[1]; t < L.nmol; ++t) {
+  for (int t = first[1]; t < end; ++t) {
     const int m = order[t];
     const int n = (int)(orb0[m + 1] - orb0[m]);
     // z goes to B1 of the molecule's work area
@@ -694,25 +879,24 @@ int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<i
   }
   if (!dc) dc.reset(stedc_ws_new(), stedc_ws_delete);
   size_t dcWork = 0;
-  if (!blocks.empty()) DH_TRY(stedc_many_prepare(s, blocks, dc.get(), &dcWork));
+  DH_TRY(stedc_many_prepare(s, blocks, dc.get(), &dcWork));
   DH_TRY(work.alloc(dcWork));
-  DH_TRY(desc.alloc(4 * (size_t)std::max(L.nmol, 1)));
-  DH_TRY(solve.alloc(std::max(L.nmol, 1)));
+  DH_TRY(solve.alloc(L.nmol));
   const size_t norb = orb0.back();
-  DH_TRY(d.alloc(norb));
-  DH_TRY(e.alloc(norb));
-  DH_TRY(tau.alloc(norb));
-  direct = nDirect;
+  DH_TRY(vec.alloc(3 * norb));
+  d = vec.p;
+  e = d + norb;
+  tau = e + norb;
   // the products of the factorisation; the list is sorted, so the molecules that reach a panel or
   // a level are its first ones
   std::vector<GemmDesc<double>> h;
   steps.clear();
   auto size = [&](int t) { return orb0[order[t] + 1] - orb0[order[t]]; };
-  const int big = nDirect > 0 ? (int)size(first[1]) : 0;
+  const int big = (int)size(first[1]);
   for (int j = 0; j + kFactorNB < big; j += kFactorNB)
     for (int q = 0; q < 2; ++q) {
       FactorStep st{j, 0, 0, 0, (long)h.size()};
-      for (int t = first[1]; t < L.nmol && size(t) > j + kFactorNB; ++t) {
+      for (int t = first[1]; t < end && size(t) > j + kFactorNB; ++t) {
         const long n = size(t), nn = n * n, r = j + kFactorNB;
         const int m = (int)(n - r);
         double* A = matrices + 3 * dOff[order[t]];
@@ -731,7 +915,7 @@ int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<i
   for (int p = kFactorNB; p < big; p *= 2)
     for (int q = 0; q < 2; ++q) {
       FactorStep st{-1, 0, 0, 0, (long)h.size()};
-      for (int t = first[1]; t < L.nmol && size(t) > p; ++t) {
+      for (int t = first[1]; t < end && size(t) > p; ++t) {
         const long n = size(t), nn = n * n;
         double* A = matrices + 3 * dOff[order[t]];
         double* T = C + dOff[order[t]];
@@ -749,18 +933,24 @@ int BatchEigen::prepare(hipStream_t s, const BatchLayout& L, const std::vector<i
       }
       steps.push_back(st);
     }
+  if (h.empty()) return 0;
   DH_TRY(factorDesc.upload(h.data(), h.size(), s));
   DH_HIP(hipStreamSynchronize(s));   // the descriptors' host copy
   return 0;
 }
 
-int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L, const double* S,
-                      const double* H, double* work, double* w, double* C, int* info,
-                      const int* active, bool warm, hipEvent_t* done) {
-  hipStream_t s = st[0];
+int launch_batch_sygv(hipStream_t s, const hipStream_t* st, BatchEigen& E, const BatchLayout& L,
+                      const double* S, const double* H, double* work, double* w, double* C,
+                      int* info, const int* active, bool warm, hipEvent_t* done) {
   if (L.ncls[0] > 0) {
-    hipLaunchKernelGGL(batch_sygv_kernel, dim3(L.ncls[0]), dim3(kSygvThreads), 0, st[1], L,
+    hipLaunchKernelGGL(batch_sygv_kernel, dim3(L.ncls[0]), dim3(kSygvThreads), 0, st[0], L,
                        L.order, S, H, work, w, C, info, active, warm ? 1 : 0);
+    DH_LAUNCH_CHECK();
+  }
+  if (L.ncls[kBatchJacobi] > 0) {
+    hipLaunchKernelGGL(batch_sygv_small_kernel, dim3(L.ncls[kBatchJacobi]), dim3(kSygvThreads), 0,
+                       st[kBatchJacobi], L, L.order + E.first[kBatchJacobi], S, H, work, w, C,
+                       info, active, warm ? 1 : 0);
     DH_LAUNCH_CHECK();
   }
   if (E.direct == 0) return 0;
@@ -798,7 +988,7 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
                      C, info, active, ds);
   DH_LAUNCH_CHECK();
   auto each = [&](auto&& f) -> int {
-    for (int c = 1; c < kBatchClasses; ++c)
+    for (int c = 1; c < kBatchJacobi; ++c)
       if (L.ncls[c] > 0) DH_TRY(f(c, E.first[c] - E.first[1], L.ncls[c], E.maxn[c]));
     return 0;
   };
@@ -807,8 +997,7 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
   DH_HIP(hipEventRecord(done[0], s));
   DH_TRY(each([&](int c, int o, int cnt, int mx) -> int {
     hipStream_t sc = st[c];
-    if (c > 1) DH_HIP(hipStreamWaitEvent(sc, done[0], 0));
-    else sc = s;
+    if (sc != s) DH_HIP(hipStreamWaitEvent(sc, done[0], 0));
     DH_TRY(gemm_batched<double>(sc, false, true, ds.hc + o, cnt, mx, mx, 1.0, 0.0));
     DH_TRY(gemm_batched<double>(sc, false, false, ds.chc + o, cnt, mx, mx, 1.0, 0.0));
     WgBatch bt;
@@ -817,14 +1006,14 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
     bt.aOff = L.dOff;
     bt.aMul = 3;
     bt.vOff = L.orb0;
-    DH_TRY(sytrd_wg_batch(sc, work, cnt, mx, bt, E.d.p, E.e.p, E.tau.p));
-    if (c > 1) {
+    DH_TRY(sytrd_wg_batch(sc, work, cnt, mx, bt, E.d, E.e, E.tau));
+    if (sc != s) {
       DH_HIP(hipEventRecord(done[c], sc));
       DH_HIP(hipStreamWaitEvent(s, done[c], 0));
     }
     return 0;
   }));
-  DH_TRY(stedc_many(s, E.d.p, E.e.p, w, work, E.work.p, E.solve.p, E.dc.get()));
+  DH_TRY(stedc_many(s, E.d, E.e, w, work, E.work.p, E.solve.p, E.dc.get()));
   hipLaunchKernelGGL(batch_info_kernel, dim3(cdiv(nd, 256)), dim3(256), 0, s, list, nd,
                      stedc_info(E.dc.get()), info);
   DH_LAUNCH_CHECK();
@@ -833,7 +1022,7 @@ int launch_batch_sygv(const hipStream_t* st, BatchEigen& E, const BatchLayout& L
       const dim3 grid(cdiv(mx, 32), std::min(32768, cnt - p));
 #define DH_APPLY(RQ_)                                                                           \
   hipLaunchKernelGGL((batch_apply_q_kernel<RQ_>), grid, dim3(256), 0, s, L, list + o + p, E.solve.p, \
-                     work, E.tau.p)
+                     work, E.tau)
       if (mx <= 32) DH_APPLY(4);
       else if (mx <= 64) DH_APPLY(8);
       else if (mx <= 128) DH_APPLY(16);

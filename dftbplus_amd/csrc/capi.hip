@@ -2621,11 +2621,43 @@ struct BatchContext {
   bool sccDone = false;
   // per-iteration transfers: eigenvalues and orbital charges and energies down, fillings up
   PinnedHost pEig, pFill, pQorb, pEorb;
-  // streams of the eigensolver's smaller size classes (default priority) and the events that
-  // fork them from s and join them back
-  static constexpr int kSx = kBatchClasses - 1;
-  hipStream_t sx[kSx] = {};
-  hipEvent_t fork = nullptr, join[kSx] = {}, stage[kBatchClasses] = {};
+  // Streams of the eigensolver's size classes (default priority) and the events that fork them
+  // from s and join them back. st: the stream of each class of the present batch; the largest one
+  // that is solved directly (or the only one) runs on s, the others on streams of their own, which
+  // are made when a batch first needs them (a small batch would wait for them longer than for its
+  // set-up).
+  hipStream_t sx[kBatchClasses] = {}, st[kBatchClasses] = {};
+  hipEvent_t fork = nullptr, join[kBatchClasses] = {}, stage[kBatchClasses] = {};
+  int class_streams() {
+    int main = 1;
+    while (main < kBatchClasses && L.ncls[main] == 0) ++main;
+    if (main == kBatchClasses) main = 0;
+    for (int c = 0; c < kBatchClasses; ++c) {
+      st[c] = s;
+      if (c == main || L.ncls[c] == 0) continue;
+      if (!fork) DH_HIP(hipEventCreate(&fork));
+      if (!join[c]) DH_HIP(hipEventCreate(&join[c]));
+      if (!sx[c]) DH_HIP(hipStreamCreate(&sx[c]));
+      st[c] = sx[c];
+    }
+    for (int c = 0; c < kBatchClasses; ++c)
+      if ((c == 0 || st[c] != s) && !stage[c]) DH_HIP(hipEventCreate(&stage[c]));
+    return 0;
+  }
+  int fork_classes() {
+    if (fork) DH_HIP(hipEventRecord(fork, s));
+    for (hipStream_t x : st)
+      if (x != s) DH_HIP(hipStreamWaitEvent(x, fork, 0));
+    return 0;
+  }
+  int join_classes() {
+    for (int c = 0; c < kBatchClasses; ++c) {
+      if (st[c] == s) continue;
+      DH_HIP(hipEventRecord(join[c], st[c]));
+      DH_HIP(hipStreamWaitEvent(s, join[c], 0));
+    }
+    return 0;
+  }
   BatchEigen be;
   // SCC iteration with the Fermi levels, energies, convergence and Broyden mixing on the device
   // (sccMode 1: launched one by one; 2: the warm iterations replay one captured HIP graph) or
@@ -2757,6 +2789,7 @@ static int batch_geometry(BatchContext& b, int nmol, const int* natMol, const do
     const long nm = b.orb0[m + 1] - b.orb0[m];
     ++b.L.ncls[batch_class(nm)];
   }
+  DH_TRY(b.class_streams());
   b.L.atom0 = b.atom0D.p;
   b.L.orb0 = b.orb0D.p;
   b.L.dOff = b.dOffD.p;
@@ -2898,16 +2931,10 @@ static int batch_scc_step(BatchContext& b) {
   for (int m = 0; m < nmol; ++m) active[m] = b.conv[m] ? 0 : 1;
   DH_HIP(hipMemcpyAsync(b.activeD.p, active.data(), nmol * sizeof(int), hipMemcpyHostToDevice, s));
   // the size classes of the eigensolver run side by side
-  DH_HIP(hipEventRecord(b.fork, s));
-  for (int q = 0; q < BatchContext::kSx; ++q) DH_HIP(hipStreamWaitEvent(b.sx[q], b.fork, 0));
-  hipStream_t st[kBatchClasses] = {s};
-  for (int q = 0; q < BatchContext::kSx; ++q) st[q + 1] = b.sx[q];
-  DH_TRY(launch_batch_sygv(st, b.be, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p, b.infoD.p,
-                           b.activeD.p, it > 1, b.stage));
-  for (int q = 0; q < BatchContext::kSx; ++q) {
-    DH_HIP(hipEventRecord(b.join[q], b.sx[q]));
-    DH_HIP(hipStreamWaitEvent(s, b.join[q], 0));
-  }
+  DH_TRY(b.fork_classes());
+  DH_TRY(launch_batch_sygv(s, b.st, b.be, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p,
+                           b.infoD.p, b.activeD.p, it > 1, b.stage));
+  DH_TRY(b.join_classes());
   b.eigv.resize(n);
   DH_HIP(hipMemcpyAsync(b.pEig.p, b.w.p, n * sizeof(double), hipMemcpyDeviceToHost, s));
   DH_HIP(hipMemcpyAsync(info.data(), b.infoD.p, nmol * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -3071,16 +3098,10 @@ static int batch_dev_enqueue(BatchContext& b, bool warm) {
                       b.vorb.p, b.hs.p));
   DH_TRY(launch_batch_unpack(s, b.dblk.pr, b.dblk.norb.p, b.dblk.atomStart.p, b.L, b.hs.p,
                              b.Hd.p, b.denseSize));
-  DH_HIP(hipEventRecord(b.fork, s));
-  for (int q = 0; q < BatchContext::kSx; ++q) DH_HIP(hipStreamWaitEvent(b.sx[q], b.fork, 0));
-  hipStream_t st[kBatchClasses] = {s};
-  for (int q = 0; q < BatchContext::kSx; ++q) st[q + 1] = b.sx[q];
-  DH_TRY(launch_batch_sygv(st, b.be, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p, b.infoD.p,
-                           b.activeD.p, warm, b.stage));
-  for (int q = 0; q < BatchContext::kSx; ++q) {
-    DH_HIP(hipEventRecord(b.join[q], b.sx[q]));
-    DH_HIP(hipStreamWaitEvent(s, b.join[q], 0));
-  }
+  DH_TRY(b.fork_classes());
+  DH_TRY(launch_batch_sygv(s, b.st, b.be, b.L, b.Sd.p, b.Hd.p, b.work.p, b.w.p, b.Cv.p,
+                           b.infoD.p, b.activeD.p, warm, b.stage));
+  DH_TRY(b.join_classes());
   DH_TRY(launch_bscc_info(s, d, b.infoD.p));
   DH_TRY(launch_bscc_fermi(s, d, b.w.p, b.f.p));
   DH_TRY(launch_batch_density(s, b.be, b.L, b.Cv.p, b.f.p, b.noccD.p, b.P.p, b.activeD.p,
@@ -3266,20 +3287,6 @@ extern "C" int dftbhip_batch_create(dftbhip_batch** bp, const dftbhip_params* p,
   auto* h = new dftbhip_batch();
   h->b.opt = *opt;
   h->b.s = dftbhip::g_rt.stream;
-  for (int q = 0; q < dftbhip::BatchContext::kSx; ++q) {
-    if (hipStreamCreate(&h->b.sx[q]) != hipSuccess || hipEventCreate(&h->b.join[q]) != hipSuccess) {
-      delete h;
-      dftbhip::set_error("batch_create: stream or event creation failed");
-      return dftbhip::kErrDevice;
-    }
-  }
-  bool events = hipEventCreate(&h->b.fork) == hipSuccess;
-  for (hipEvent_t& e : h->b.stage) events = events && hipEventCreate(&e) == hipSuccess;
-  if (!events) {
-    delete h;
-    dftbhip::set_error("batch_create: event creation failed");
-    return dftbhip::kErrDevice;
-  }
   const int rc = dftbhip::sk_setup(h->b.sk, p, h->b.s);
   if (rc != 0) {
     delete h;

@@ -72,12 +72,14 @@ struct StedcWs {
   std::vector<int> maxn;                  // largest block of height h
   int maxProblem = 0;
   long total = 0, totalSq = 0;
-  DevBuf<LeafDev> dleaf;
-  DevBuf<MergeDev> dmerge;
-  DevBuf<ProblemDev> dproblem;
-  DevBuf<GemmDesc<double>> ddesc;
-  DevBuf<double> darr;                    // double arrays of length `total`, then the scales
-  DevBuf<int> iarr;                       // int arrays of length `total`, then the info words
+  std::vector<char> staging;              // the tables as uploaded
+  DevBuf<char> tables, arrays;
+  const LeafDev* dleaf = nullptr;         // in tables
+  MergeDev* dmerge = nullptr;
+  const ProblemDev* dproblem = nullptr;
+  GemmDesc<double>* ddesc = nullptr;      // in arrays
+  double* darr = nullptr;                 // double arrays of length `total`, then the scales
+  int* iarr = nullptr;                    // int arrays of length `total`, then the info words
   DevBuf<double> dd, de;                  // uploads of the host interface
   int* info = nullptr;
 };
@@ -792,14 +794,30 @@ static int dc_tables(hipStream_t s, StedcWs& W, const std::vector<DcBlock>& bloc
     W.maxn.push_back(mx);
   }
   W.first.push_back((int)W.merges.size());
-  DH_TRY(W.dleaf.upload(W.leaves.data(), W.leaves.size(), s));
-  DH_TRY(W.dmerge.alloc(std::max<size_t>(W.merges.size(), 1)));
-  if (!W.merges.empty()) DH_TRY(W.dmerge.upload(W.merges.data(), W.merges.size(), s));
-  DH_TRY(W.dproblem.upload(W.problems.data(), W.problems.size(), s));
-  DH_TRY(W.ddesc.alloc(std::max<size_t>(2 * W.merges.size(), 1)));
-  DH_TRY(W.darr.alloc((size_t)kDcDoubles * W.total + blocks.size()));
-  DH_TRY(W.iarr.alloc((size_t)kDcInts * W.total + blocks.size()));
-  W.info = W.iarr.p + (size_t)kDcInts * W.total;
+  // one buffer each for the tables and the arrays: a new batch or size makes all of them anew
+  auto up = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+  const size_t bl = up(W.leaves.size() * sizeof(LeafDev)),
+               bm = up(W.merges.size() * sizeof(MergeDev)),
+               bp = up(W.problems.size() * sizeof(ProblemDev));
+  W.staging.resize(bl + bm + bp);
+  std::copy_n(reinterpret_cast<const char*>(W.leaves.data()), W.leaves.size() * sizeof(LeafDev),
+              W.staging.begin());
+  std::copy_n(reinterpret_cast<const char*>(W.merges.data()), W.merges.size() * sizeof(MergeDev),
+              W.staging.begin() + bl);
+  std::copy_n(reinterpret_cast<const char*>(W.problems.data()),
+              W.problems.size() * sizeof(ProblemDev), W.staging.begin() + bl + bm);
+  DH_TRY(W.tables.upload(W.staging.data(), W.staging.size(), s));
+  W.dleaf = reinterpret_cast<const LeafDev*>(W.tables.p);
+  W.dmerge = reinterpret_cast<MergeDev*>(W.tables.p + bl);
+  W.dproblem = reinterpret_cast<const ProblemDev*>(W.tables.p + bl + bm);
+  const size_t bd = up(2 * W.merges.size() * sizeof(GemmDesc<double>)),
+               ba = up(((size_t)kDcDoubles * W.total + blocks.size()) * sizeof(double)),
+               bi = ((size_t)kDcInts * W.total + blocks.size()) * sizeof(int);
+  DH_TRY(W.arrays.alloc(bd + ba + bi));
+  W.ddesc = reinterpret_cast<GemmDesc<double>*>(W.arrays.p);
+  W.darr = reinterpret_cast<double*>(W.arrays.p + bd);
+  W.iarr = reinterpret_cast<int*>(W.arrays.p + bd + ba);
+  W.info = W.iarr + (size_t)kDcInts * W.total;
   W.blocks = blocks;
   return 0;
 }
@@ -814,10 +832,10 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
                                &A.rc, &A.rs};
     int** ip[kDcInts] = {&A.ord, &A.idx, &A.cand, &A.flag, &A.type, &A.org, &A.row, &A.gcol,
                          &A.dcol, &A.rp, &A.rn};
-    for (int i = 0; i < kDcDoubles; ++i) *dp[i] = W.darr.p + (size_t)i * W.total;
-    for (int i = 0; i < kDcInts; ++i) *ip[i] = W.iarr.p + (size_t)i * W.total;
+    for (int i = 0; i < kDcDoubles; ++i) *dp[i] = W.darr + (size_t)i * W.total;
+    for (int i = 0; i < kDcInts; ++i) *ip[i] = W.iarr + (size_t)i * W.total;
     A.info = W.info;
-    A.scale = W.darr.p + (size_t)kDcDoubles * W.total;
+    A.scale = W.darr + (size_t)kDcDoubles * W.total;
   }
   const size_t sq = W.totalSq;
   double* Q[2] = {work, work + sq};
@@ -826,10 +844,10 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
   // zeros outside the blocks of the leaves; the second buffer's blocks are written whole, its
   // zeros outside them are read by the next height
   hipLaunchKernelGGL(stedc_zero_kernel, dim3((unsigned)std::min<size_t>(cdiv(2 * sq, 1024), 2048)),
-                     dim3(kZeroT), 0, s, work, 2 * sq, W.dproblem.p, active, d, e,
+                     dim3(kZeroT), 0, s, work, 2 * sq, W.dproblem, active, d, e,
                      (int)W.problems.size(), A.info, A.scale);
   DH_LAUNCH_CHECK();
-  hipLaunchKernelGGL(leaf_kernel, dim3((unsigned)W.leaves.size()), dim3(64), 0, s, d, e, W.dleaf.p,
+  hipLaunchKernelGGL(leaf_kernel, dim3((unsigned)W.leaves.size()), dim3(64), 0, s, d, e, W.dleaf,
                      Q[0], A);
   DH_LAUNCH_CHECK();
   for (size_t h = 1; h + 1 < W.first.size(); ++h) {
@@ -838,8 +856,8 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
     double* Qn = Q[h & 1];
     for (int f = W.first[h]; f < W.first[h + 1]; f += kRows) {
       const int nm = std::min(kRows, W.first[h + 1] - f);
-      MergeDev* md = W.dmerge.p + f;
-      GemmDesc<double>* gd = W.ddesc.p + 2 * (size_t)f;
+      MergeDev* md = W.dmerge + f;
+      GemmDesc<double>* gd = W.ddesc + 2 * (size_t)f;
       hipLaunchKernelGGL(deflate_kernel, dim3(nm), dim3(kDefT), 0, s, md, e, Qo, Qn, Qg, U, gd, A);
       DH_LAUNCH_CHECK();
       hipLaunchKernelGGL(rotate_kernel, dim3(cdiv(mx, 64), nm), dim3(64), 0, s, md, Qo, A);
@@ -862,7 +880,7 @@ static int dc_launch(hipStream_t s, StedcWs& W, const double* d, const double* e
     Ap.scale += p;
     hipLaunchKernelGGL(collect_kernel, dim3(cdiv((long)W.maxProblem * 64, 256),
                                             (unsigned)std::min<size_t>(kRows, W.problems.size() - p)),
-                       dim3(256), 0, s, W.dproblem.p + p, Q[0], Q[1], w, z, Ap);
+                       dim3(256), 0, s, W.dproblem + p, Q[0], Q[1], w, z, Ap);
     DH_LAUNCH_CHECK();
   }
   return 0;
