@@ -1,4 +1,4 @@
-"""Molecule batch (one block-diagonal system, batched Jacobi eigensolver) against a loop of
+"""Molecule batch (one block-diagonal system, solved by size classes) against a loop of
 single-molecule calculations of the plain path and against the CPU oracle."""
 import numpy as np
 import pytest
@@ -68,9 +68,9 @@ def _chain(norb, rng):
 
 
 def test_batch_size_classes_one_iteration():
-    """Molecules at the edges of the eigensolver's size classes (LDS A and C up to 64 and 112
-    orbitals, LDS A up to 190, HBM above), single atoms and odd sizes included, after one SCC
-    iteration: the batch equals the single-molecule runs of the plain path."""
+    """Molecules at and beside edges of the eigensolver's size classes (Jacobi in LDS up to 16
+    orbitals, direct with shapes for 32, 64, 128, 192 and 224), single atoms and odd sizes included,
+    after one SCC iteration: the batch equals the single-molecule runs of the plain path."""
     import dataclasses
     from dftbplus_amd import api, synth
     _, params, opts = synth.workload("molecules1")
@@ -94,10 +94,9 @@ def test_batch_size_classes_one_iteration():
 
 def test_batch_level_at_zero_converges():
     """A molecule with an eigenvalue at 0 Ha (every on-site energy shifted by the constant a
-    secant search on the oracle finds) converges like any other: the Jacobi rotation test has a
-    rounding-level floor, so a pair touching a diagonal entry near 0 does not rotate on noise
-    until the sweep limit (which would now be reported as an error). The batch equals the
-    oracle for that molecule and a neighbour."""
+    secant search on the oracle finds) converges like any other, here in the direct solver's classes
+    (those of the Jacobi kernels, whose rotation test has a rounding-level floor for it: the same
+    test in test_gpu_batch_small). The batch equals the oracle for that molecule and a neighbour."""
     import copy
     from dftbplus_amd import api, synth
     from oracle import dftb_ref as R
