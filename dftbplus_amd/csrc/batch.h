@@ -12,13 +12,19 @@ namespace dftbhip {
 constexpr int kBatchMaxOrb = 512;   // orbitals per molecule in a batch
 // size classes of the batched eigensolver, by orbital count (largest first): above kWgBatchMax
 // Jacobi with both matrices in HBM, up to it the direct solve, whose reduction has shapes for
-// 224, 192, 128, 64 and 32 orbitals, and up to kBatchSmall Jacobi in LDS
+// 224, 192, 128, 64 and 32 orbitals. Molecules of up to kBatchSmall orbitals are swept by Jacobi
+// in LDS if the batch has none that is solved directly: the sweeps save the direct solve's
+// launches, which cost nothing where a larger molecule needs them, and would be one more branch
+// beside the classes' reductions (32 molecules of 13 to 190 orbitals: 15.5 ms with the sweeps,
+// 13.9 without).
 constexpr int kBatchSmall = 16;
 constexpr int kBatchJacobi = 6;   // the class of the smallest
 constexpr int kBatchClasses = 7;
-inline int batch_class(long n) {
+inline bool batch_direct(long n) { return n > kBatchSmall && n <= kWgBatchMax; }
+// anyDirect: batch_direct holds for some molecule of the batch
+inline int batch_class(long n, bool anyDirect) {
   return n > kWgBatchMax ? 0 : n > 192 ? 1 : n > 128 ? 2 : n > 64 ? 3 : n > 32 ? 4
-         : n > kBatchSmall ? 5 : kBatchJacobi;
+         : n > kBatchSmall || anyDirect ? 5 : kBatchJacobi;
 }
 // info of a molecule whose eigensolver did not converge within its limit (distinct from the
 // leading minor of a non-positive-definite overlap)

@@ -2785,10 +2785,10 @@ static int batch_geometry(BatchContext& b, int nmol, const int* natMol, const do
   b.L.nmol = nmol;
   b.L.order = b.orderD.p;
   for (int& c : b.L.ncls) c = 0;
-  for (int m : order) {
-    const long nm = b.orb0[m + 1] - b.orb0[m];
-    ++b.L.ncls[batch_class(nm)];
-  }
+  auto norbMol = [&](int m) { return b.orb0[m + 1] - b.orb0[m]; };
+  const bool anyDirect = std::any_of(order.begin(), order.end(),
+                                     [&](int m) { return batch_direct(norbMol(m)); });
+  for (int m : order) ++b.L.ncls[batch_class(norbMol(m), anyDirect)];
   DH_TRY(b.class_streams());
   b.L.atom0 = b.atom0D.p;
   b.L.orb0 = b.orb0D.p;
