@@ -116,11 +116,6 @@ __global__ void expand_kernel(int nat, const long* iAtomStart, const double* va,
   for (long o = iAtomStart[a]; o < iAtomStart[a + 1]; ++o) vo[o] = va[a];
 }
 
-__global__ void scale_kernel(int n, const double* a, const double* b, double* c) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) c[i] = a[i] * b[i];
-}
-
 // ------------------------------------------------------------------------------------------
 // Slater-Koster parameters on the device
 // ------------------------------------------------------------------------------------------

@@ -224,8 +224,6 @@ int add_f32(hipStream_t s, const double* a, long lda, const float* b, long ldb, 
             long ldd, int m, int n);
 int symmetrize_lower(hipStream_t s, double* a, long lda, int n);
 int symmetrize_lower(hipStream_t s, float* a, long lda, int n);
-int zero_strict_upper(hipStream_t s, double* a, long lda, int n);
-
 
 // ------------------------------------------------------------------------------------------
 // Symmetric eigensolver pieces (sytrd.hip, stedc.hip)

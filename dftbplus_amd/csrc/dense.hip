@@ -122,12 +122,6 @@ __global__ void symmetrize_lower_kernel(T* a, long lda, int n) {
   }
 }
 
-__global__ void zero_upper_kernel(double* a, long lda, int n) {
-  const int j = blockIdx.y;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < j && i < n; i += gridDim.x * blockDim.x)
-    a[i + (long)j * lda] = 0.0;
-}
-
 template <typename T>
 static int symmetrize_lower_t(hipStream_t s, T* a, long lda, int n) {
   if (n <= 1) return 0;
@@ -235,13 +229,6 @@ int f16_convert(hipStream_t s, const double* x, const double* y, const double* l
 
 template int transpose2d<double, double>(hipStream_t, const double*, long, double*, long, int, int);
 template int transpose2d<float, double>(hipStream_t, const float*, long, double*, long, int, int);
-
-int zero_strict_upper(hipStream_t s, double* a, long lda, int n) {
-  if (n <= 1) return 0;
-  hipLaunchKernelGGL(zero_upper_kernel, dim3(cdiv(n, 256), n), dim3(256), 0, s, a, lda, n);
-  DH_LAUNCH_CHECK();
-  return 0;
-}
 
 constexpr int kPotrfNB = 64;
 

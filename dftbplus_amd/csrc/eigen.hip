@@ -59,23 +59,6 @@ int EigenSolver::reduce(hipStream_t s, const double* Li, const double* H, long l
   return 0;
 }
 
-int EigenSolver::tridiag_eigen(hipStream_t s, const double* dDev, const double* eDev,
-                               std::vector<double>& wHost, int* info) {
-  *info = 0;
-  DH_TRY(stedc_device(s, n, dDev, eDev, w.p, Zd.p, n, work.p, workSize, dc_ws()));
-  wHost.resize(n);
-  return stedc_fetch(s, n, w.p, wHost.data(), dc_ws(), info);
-}
-
-int EigenSolver::vectors_from(hipStream_t s, const double* Li, const double* A,
-                              const double* tauDev, int nvec, double* X, long ldx) {
-  if (nvec <= 0) return 0;
-  DH_TRY(ormtr_lower(s, A, n, n, tauDev, Zd.p, n, nvec, work.p, workSize));
-  DH_TRY(gemm<double>(s, true, false, n, nvec, n, 1.0, Li, n, Zd.p, n, 0.0, X, ldx, false,
-                      kKAUpper));
-  return 0;
-}
-
 int EigenSolver::solve(hipStream_t s, const double* H, long ldh, std::vector<double>& wHost,
                        int* info, double* times) {
   DH_CHECK(factored, "eigensolver: overlap not factorised");
@@ -92,7 +75,9 @@ int EigenSolver::solve(hipStream_t s, const double* H, long ldh, std::vector<dou
     DH_TRY(sytrd_lower(s, C.p, n, n, d.p, e.p, tau.p, work.p, workSize));
   }
   DH_HIP(hipEventRecord(ev[2], s));
-  DH_TRY(tridiag_eigen(s, d.p, e.p, wHost, info));
+  DH_TRY(stedc_device(s, n, d.p, e.p, w.p, Zd.p, n, work.p, workSize, dc_ws()));
+  wHost.resize(n);
+  DH_TRY(stedc_fetch(s, n, w.p, wHost.data(), dc_ws(), info));
   if (*info != 0) return 0;
   DH_HIP(hipEventRecord(ev[3], s));
   DH_HIP(hipEventSynchronize(ev[3]));
@@ -110,14 +95,14 @@ int EigenSolver::solve(hipStream_t s, const double* H, long ldh, std::vector<dou
 
 int EigenSolver::vectors(hipStream_t s, int nvec, double* X, long ldx) {
   if (nvec <= 0) return 0;
-  if (twoStage) {
+  if (twoStage)
     DH_TRY(ormtr_2stage(s, C.p, n, n, Zd.p, n, nvec, band.p, bandBytes, work.p,
                         workSize * sizeof(double)));
-    DH_TRY(gemm<double>(s, true, false, n, nvec, n, 1.0, Linv.p, n, Zd.p, n, 0.0, X, ldx, false,
-                        kKAUpper));
-    return 0;
-  }
-  return vectors_from(s, Linv.p, C.p, tau.p, nvec, X, ldx);
+  else
+    DH_TRY(ormtr_lower(s, C.p, n, n, tau.p, Zd.p, n, nvec, work.p, workSize));
+  DH_TRY(gemm<double>(s, true, false, n, nvec, n, 1.0, Linv.p, n, Zd.p, n, 0.0, X, ldx, false,
+                      kKAUpper));
+  return 0;
 }
 
 // Ogita-Aishima correction E (n x nv) from G = X^T S X and M = X^T H X (both full):

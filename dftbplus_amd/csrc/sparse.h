@@ -57,9 +57,6 @@ struct RepDev {
 int launch_build_h0s(hipStream_t s, const SkDev& sk, const PairsDev& pr, const double* coords,
                      double* h0, double* ov);
 template <typename T>
-int launch_unpack(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
-                  const double* x, T* dense, long ld, int n);
-template <typename T>
 int launch_pack(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
                 const T* dense, long ld, double* x);
 // k-point matrices (blkT: fractional cell translation of the image of each block, kf:
@@ -76,9 +73,6 @@ int launch_pack_kpt(hipStream_t s, const PairsDev& pr, const int* norb, const lo
                     int n, double* x);
 int launch_shift(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
                  const double* h0, const double* ov, const double* vorb, double* h);
-int launch_mulliken(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
-                    const double* ov, const double* h0, const double* rho, double* qorb,
-                    double* eorb, int nOrb);
 int launch_pair_forces(hipStream_t s, const SkDev& sk, const PairsDev& pr, const int* norb,
                        const long* iAtomStart, const double* coords, const double* rho,
                        const double* erho, const double* vorb, int mode, double delta,

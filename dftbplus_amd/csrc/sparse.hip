@@ -222,8 +222,8 @@ __device__ __forceinline__ double sk_lane(const SkDev& sk, const SkPair& pr, con
 
 constexpr int kBlkLanes = 16;
 
-// H0 and S blocks. Bound by the arithmetic of one interpolation per lane: 85 us for the blocks of
-// 1000 molecules, 95 us for 2744 atoms (760 and 903 us with a thread per block, its arrays in
+// H0 and S blocks. Bound by the arithmetic of one interpolation per lane: 102 us for the blocks
+// of 1000 molecules, 114 us for 2744 atoms (760 and 903 us with a thread per block, its arrays in
 // scratch memory).
 __global__ __launch_bounds__(256) void build_h0s_kernel(SkDev sk, PairsDev pr, const double* coords, double* h0,
                                  double* s) {
@@ -259,23 +259,6 @@ __global__ __launch_bounds__(256) void build_h0s_kernel(SkDev sk, PairsDev pr, c
 // The per-iteration sparse kernels below give each SK block kBlkLanes lanes too, lane e holding
 // element e (lanes past n1 n2 idle): the blocks of a wave are consecutive in the sparse arrays,
 // so their loads and stores are contiguous.
-
-// Dense fill of both triangles; blocks of periodic images of the same pair are summed.
-template <typename T>
-__global__ void unpack_kernel(PairsDev pr, const int* norbAtom, const long* iAtomStart,
-                              const double* x, T* dense, long ld) {
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  const int k = (int)(t / kBlkLanes), e = (int)(t % kBlkLanes);
-  if (k >= pr.nblk) return;
-  const int a1 = pr.at1[k], a2 = pr.at2[k];
-  const int n1 = norbAtom[a1], n2 = norbAtom[a2];
-  if (e >= n1 * n2) return;
-  const int r = e % n2, c = e / n2;
-  const long o1 = iAtomStart[a1], o2 = iAtomStart[a2];
-  const T v = (T)x[pr.start[k] + e];
-  atomicAdd(&dense[(o2 + r) + (o1 + c) * ld], v);
-  if (a1 != a2) atomicAdd(&dense[(o1 + c) + (o2 + r) * ld], v);
-}
 
 template <typename T>
 __global__ void pack_kernel(PairsDev pr, const int* norbAtom, const long* iAtomStart,
@@ -396,68 +379,13 @@ __global__ void shift_kernel(PairsDev pr, const int* norbAtom, const long* iAtom
   h[i] = h0[i] + 0.5 * s[i] * (vorb[o2 + r] + vorb[o1 + c]);
 }
 
-// q_mu += sum_nu S rho (column sums to atom 1, row sums to atom 2 for off-site blocks);
-// the same contraction with H0 gives the non-SCC energy per orbital. A block's column and row
-// sums are gathered by shuffles inside its lane group (every lane takes part), then one lane
-// per column (r = 0) and per row (c = 0) adds them.
-__global__ void mulliken_kernel(PairsDev pr, const int* norbAtom, const long* iAtomStart,
-                                const double* s, const double* h0, const double* rho,
-                                double* qorb, double* eorb) {
-  const long t = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  const int k = (int)(t / kBlkLanes), e = (int)(t % kBlkLanes);
-  const int lane = threadIdx.x & 63;
-  int a1 = 0, a2 = 0, n1 = 1, n2 = 1;
-  double pq = 0.0, pe = 0.0;
-  const bool blk = k < pr.nblk;
-  if (blk) {
-    a1 = pr.at1[k];
-    a2 = pr.at2[k];
-    n1 = norbAtom[a1];
-    n2 = norbAtom[a2];
-    if (e < n1 * n2) {
-      const long i = pr.start[k] + e;
-      pq = s[i] * rho[i];
-      pe = h0 ? h0[i] * rho[i] : 0.0;
-    }
-  }
-  const bool valid = blk && e < n1 * n2;
-  const int r = e % n2, c = e / n2;
-  double cq = 0.0, ce = 0.0, rq = 0.0, re = 0.0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    // column c: lanes e + j (r = 0 lanes), row r: lanes e + j n2 (c = 0 lanes)
-    const double vq = __shfl(pq, min(lane + j, 63), 64);
-    const double ve = __shfl(pe, min(lane + j, 63), 64);
-    const double wq = __shfl(pq, min(lane + j * n2, 63), 64);
-    const double we = __shfl(pe, min(lane + j * n2, 63), 64);
-    if (j < n2) {
-      cq += vq;
-      ce += ve;
-    }
-    if (j < n1) {
-      rq += wq;
-      re += we;
-    }
-  }
-  if (!valid) return;
-  const long o1 = iAtomStart[a1], o2 = iAtomStart[a2];
-  if (r == 0) {
-    atomicAdd(&qorb[o1 + c], cq);
-    if (eorb) atomicAdd(&eorb[o1 + c], ce);
-  }
-  if (c == 0 && a1 != a2) {
-    atomicAdd(&qorb[o2 + r], rq);
-    if (eorb) atomicAdd(&eorb[o2 + r], re);
-  }
-}
-
 // Pair forces: gradient contribution of every off-site block. mode 0: central finite
 // differences with step delta on the bond vector (the reference default); mode 1: analytic
 // derivative of the interpolated and rotated blocks (the adjoint of the assembly).
 // Lanes as above: six interpolations per lane in mode 0, one in mode 1, the element's
 // contribution summed over the block's lanes. A thread per pair (60 interpolations one after the
 // other, blocks in scratch memory) took 3.9 ms for 1000 molecules and 4.6 ms for 2744 atoms; now
-// 0.43 and 0.48 ms.
+// 0.45 and 0.50 ms.
 template <int kMode>
 __global__ __launch_bounds__(256) void pair_force_kernel(SkDev sk, PairsDev pr, const int* norbAtom,
                                   const long* iAtomStart, const double* coords, const double* rho,
@@ -755,18 +683,6 @@ int launch_build_h0s(hipStream_t s, const SkDev& sk, const PairsDev& pr, const d
 }
 
 template <typename T>
-int launch_unpack(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
-                  const double* x, T* dense, long ld, int n) {
-  DH_TRY(fill2d<T>(s, dense, ld, n, n, T(0)));
-  if (pr.nblk == 0) return 0;
-  hipLaunchKernelGGL((unpack_kernel<T>), dim3(cdiv((long)pr.nblk * kBlkLanes, 256)),
-                     dim3(256), 0, s, pr, norb,
-                     iAtomStart, x, dense, ld);
-  DH_LAUNCH_CHECK();
-  return 0;
-}
-
-template <typename T>
 int launch_pack(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
                 const T* dense, long ld, double* x) {
   if (pr.nblk == 0) return 0;
@@ -821,19 +737,6 @@ int launch_shift(hipStream_t s, const PairsDev& pr, const int* norb, const long*
   hipLaunchKernelGGL(shift_kernel, dim3(cdiv((long)pr.nblk * kBlkLanes, 256)),
                      dim3(256), 0, s, pr, norb,
                      iAtomStart, h0, ov, vorb, h);
-  DH_LAUNCH_CHECK();
-  return 0;
-}
-
-int launch_mulliken(hipStream_t s, const PairsDev& pr, const int* norb, const long* iAtomStart,
-                    const double* ov, const double* h0, const double* rho, double* qorb,
-                    double* eorb, int nOrb) {
-  DH_TRY(fill<double>(s, qorb, nOrb, 0.0));
-  if (eorb) DH_TRY(fill<double>(s, eorb, nOrb, 0.0));
-  if (pr.nblk == 0) return 0;
-  hipLaunchKernelGGL(mulliken_kernel, dim3(cdiv((long)pr.nblk * kBlkLanes, 256)),
-                     dim3(256), 0, s, pr, norb,
-                     iAtomStart, ov, h0, rho, qorb, eorb);
   DH_LAUNCH_CHECK();
   return 0;
 }
@@ -1231,10 +1134,6 @@ int launch_mulliken_rows(hipStream_t s, const RowBlocksDev& rb, const int* norb,
   return 0;
 }
 
-template int launch_unpack<double>(hipStream_t, const PairsDev&, const int*, const long*,
-                                   const double*, double*, long, int);
-template int launch_unpack<float>(hipStream_t, const PairsDev&, const int*, const long*,
-                                  const double*, float*, long, int);
 template int launch_pack<double>(hipStream_t, const PairsDev&, const int*, const long*,
                                  const double*, long, double*);
 template int launch_pack<float>(hipStream_t, const PairsDev&, const int*, const long*,
