@@ -4,9 +4,10 @@
 // consecutively and the neighbour list holds only intra-molecule pairs, so the sparse kernels
 // (H0/S assembly, shift, pack, Mulliken, pair forces, repulsive) run unchanged over the union.
 // What is per molecule lives here: the dense matrices (packed one after the other, n_m x n_m
-// column-major), the generalized eigensolver (Cholesky and L^-T once per geometry, then per call
-// a direct solve, or for molecules above kWgBatchMax orbitals parallel cyclic Jacobi by one
-// workgroup), the density matrices and the cluster gamma matrix with its products and gradient.
+// column-major), the generalized eigensolver (Cholesky and the inverse factor once per geometry,
+// then per call a direct solve, or parallel cyclic Jacobi by one workgroup: in HBM for molecules
+// above kWgBatchMax orbitals, in LDS for those of up to kBatchSmall in a batch without larger
+// direct ones), the density matrices and the cluster gamma matrix with its products and gradient.
 // The eigensolver and density kernels visit the molecules largest first (BatchLayout::order).
 #include "batch.h"
 #include "gamma_dev.h"
@@ -631,16 +632,17 @@ void batch_sygv_small_kernel(BatchLayout L, const int* list, const double* S, co
 }
 
 // ------------------------------------------------------------------------------------------
-// Direct eigensolver for the other molecules of up to kWgBatchMax orbitals: L^-1 once per geometry (panels
-// of 64 columns, every launch for all molecules that reach its panel; one workgroup per molecule
-// in HBM took 2.1 ms for 190 orbitals), then per call A = L^-1 H L^-T (batched MFMA GEMMs),
-// tridiagonalisation with the matrix in the registers of one workgroup (sytrd_resident.hip),
-// divide and conquer of all molecules together (stedc.hip), the reflectors applied to strips of
-// eigenvectors, and C = L^-T (Q Z). A parallel
-// cyclic Jacobi with A and C in LDS ran here before, n dependent rounds per sweep and 7 to 10
-// sweeps. One SCC cycle of 32 molecules of 13 to 190 orbitals: 135 ms before, 16.7 ms now; of
-// 1000 molecules: 250 ms before, 51 ms now. Bound by the column chain of the reduction (0.38 ms
-// per iteration for 190 orbitals, 0.12 for 112), then by the solve's own latencies.
+// Direct eigensolver for the other molecules of up to kWgBatchMax orbitals: L^-1 once per
+// geometry (panels of 64 columns, every launch for all molecules that reach its panel; one
+// workgroup per molecule in HBM took 2.1 ms for 190 orbitals), then per call A = L^-1 H L^-T
+// (batched MFMA GEMMs), tridiagonalisation with the matrix in the registers of one workgroup
+// (sytrd_resident.hip), divide and conquer of all molecules together (stedc.hip), the reflectors
+// applied to strips of eigenvectors, and C = L^-T (Q Z). A parallel cyclic Jacobi with A and C in
+// LDS ran here before, n dependent rounds per sweep and 7 to 10 sweeps. From
+// set-up to forces, 32 molecules of 13 to 190 orbitals, eight iterations: 138 ms before, 14.6 ms
+// now; 1000 molecules, five iterations: 249 ms before, 43.6 ms now. Bound by the column chain of
+// the reduction (0.38 ms per iteration for 190 orbitals, 0.12 for 112), then by the solve's own
+// latencies.
 // ------------------------------------------------------------------------------------------
 // Start of the factorisation: B0 = S, the place of L^-1 zero, info 0
 __global__ void batch_factor_init_kernel(BatchLayout L, const int* list, const double* S,
