@@ -1,5 +1,6 @@
-"""The batch's smallest molecules (up to 16 orbitals, swept in LDS), alone and beside the other size
-classes, and the rounding floor of both Jacobi kernels."""
+"""The batch's smallest molecules: up to 16 orbitals, swept in LDS (alone or beside molecules above the
+direct classes) or solved directly beside larger ones, and the rounding floor of both Jacobi
+kernels."""
 import copy
 import dataclasses
 
